@@ -129,3 +129,26 @@ def test_quantize_levels_batched_vs_oracle(hk, tmp_path, nlevel, bf, d, n):
     want = Oracle().hkm_quantize(levels, bf, v)
     assert np.array_equal(got, want)
     assert got.min() >= 0 and got.max() < bf ** nlevel
+
+
+@pytest.mark.parametrize("nlevel,bf,d,n", [(1, 7, 20, 300), (2, 2, 16, 4097), (3, 90, 4, 9001),
+                                           (3, 91, 4, 9001)])
+def test_quantize_ordering_paths_vs_oracle(hk, tmp_path, nlevel, bf, d, n):
+    """The points' ordering by node on each side of its limits: the root's
+    level alone, a partial last segment, and last levels of 8,100 (LDS table)
+    and 8,281 nodes (an atomic per point).  Integer trees and points: the
+    oracle's leaves; a NaN point leaves the descent with -1."""
+    from oracle_bind import Oracle
+    rng = np.random.default_rng(nlevel * 1000 + bf)
+    levels = [np.rint(rng.uniform(0, 200, (bf ** (l + 1), d))).astype(np.float32)
+              for l in range(nlevel)]
+    v = np.rint(rng.uniform(0, 200, (n, d))).astype(np.float32)
+    path = tmp_path / "int.hkm"
+    _tree_file(path, levels, bf)
+    t = hk.hkm_read(path)
+    print("hkm_quantize nlevel=%d bf=%d d=%d n=%d" % (nlevel, bf, d, n), flush=True)
+    want = Oracle().hkm_quantize(levels, bf, v)
+    assert np.array_equal(t.quantize(v), want)
+    v[n // 2] = np.nan
+    want[n // 2] = -1
+    assert np.array_equal(t.quantize(v), want)

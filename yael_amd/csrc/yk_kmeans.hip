@@ -620,71 +620,127 @@ extern "C" int yk_kpp_update(const float *v, long n, int d, const double *vn, lo
 }
 
 // hkm tree descent (hkm_quantize, hkm.c:131-150), a level at a time: the
-// points are ordered by their current node (a counting sort on the device:
-// histogram, exclusive scan, scatter of point indices), every node is one
-// instance of the batched FP32 assign (yk_batch_assign_idx: k = 1 over the
-// node's bf children with the FP32 form's arithmetic, nn.c:383-446, points
-// read through the index table), and each point's node becomes
+// points are ordered by their current node (histogram, exclusive scan,
+// scatter of point indices; the root's level takes them as they are), every
+// node is one instance of the batched FP32 assign (yk_batch_assign_idx: k = 1
+// over the node's bf children with the FP32 form's arithmetic, nn.c:383-446,
+// points read through the index table), and each point's node becomes
 // node * bf + child.  A point with no child below 1e30 gets -1 and leaves
-// the descent (the reference would index outside the level).
+// the descent (the reference would index outside the level).  The order of a
+// node's points is free: each point's child depends on that point alone.
+//
+// Ordering: workgroup w owns a contiguous segment of the points and counts
+// it in an LDS table of the nodes; one global atomic per (workgroup, node
+// present) adds the counts, or takes the workgroup's places in the node's
+// list, where LDS atomics hand them out.  (A global atomic per point queues
+// at a level of few nodes: 1e6 points through two levels of 32 children,
+// d = 128: 28.1 of the descent's 28.8 ms; the whole descent now 0.575 ms.)  Levels of more than
+// YK_HQ_LDS_NODES nodes (a 32 KB table) keep the atomic per point: their
+// addresses are many.
+#define YK_HQ_LDS_NODES 8192
+#define YK_HQ_SEG 4096  // points per workgroup: 16 per thread
 
-__global__ void yk_hq_hist_kernel(const int *__restrict__ node, long n, int *__restrict__ cnt) {
-  const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (i < n && node[i] >= 0) atomicAdd(&cnt[node[i]], 1);
+template <bool SCATTER>
+__global__ __launch_bounds__(256) void yk_hq_place_kernel(const int *__restrict__ node, long n,
+                                                          int nn, int *__restrict__ cnt,
+                                                          int *__restrict__ perm) {
+  extern __shared__ int tab[];  // nn
+  constexpr int NJ = YK_HQ_SEG / 256;
+  for (int p = threadIdx.x; p < nn; p += 256) tab[p] = 0;
+  __syncthreads();
+  const long p0 = blockIdx.x * (long)YK_HQ_SEG + threadIdx.x;
+  int a[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; j++) a[j] = p0 + 256 * j < n ? node[p0 + 256 * j] : -1;
+  int rank[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; j++) rank[j] = a[j] >= 0 ? atomicAdd(&tab[a[j]], 1) : 0;
+  __syncthreads();
+  // cnt: the nodes' counts (histogram), or their next free places (scatter)
+  for (int p = threadIdx.x; p < nn; p += 256) {
+    const int c = tab[p];
+    if (c) {
+      const int base = atomicAdd(&cnt[p], c);
+      if (SCATTER) tab[p] = base;
+    }
+  }
+  if (!SCATTER) return;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NJ; j++)
+    if (a[j] >= 0) perm[tab[a[j]] + rank[j]] = (int)(p0 + 256 * j);
+}
+
+// the same with a global atomic per point (levels of many nodes)
+template <bool SCATTER>
+__global__ __launch_bounds__(256) void yk_hq_place_many_kernel(const int *__restrict__ node,
+                                                               long n, int *__restrict__ cnt,
+                                                               int *__restrict__ perm) {
+  const long i = blockIdx.x * 256L + threadIdx.x;
+  if (i >= n || node[i] < 0) return;
+  const int at = atomicAdd(&cnt[node[i]], 1);
+  if (SCATTER) perm[at] = (int)i;
 }
 
 // one workgroup: off[p] (points before node p, p <= nn), cursor = off, and
-// the work items: itoff[p] = items before node p (ceil(count / 128) each)
+// the work items: itoff[p] = items before node p (ceil(count / 128) each).
+// Thread t sums a contiguous run of nodes; the threads' totals are scanned
+// by shuffles inside the waves, then over the 16 wave totals.
 __global__ __launch_bounds__(1024) void yk_hq_scan_kernel(const int *__restrict__ cnt, long nn,
                                                           long *__restrict__ off,
-                                                          long *__restrict__ cursor,
+                                                          int *__restrict__ cursor,
                                                           long *__restrict__ itoff) {
-  __shared__ long sp[1024], si[1024];
-  const int t = threadIdx.x;
-  const long per = (nn + 1023) / 1024, lo = t * per, hi = min(nn, lo + per);
-  long a = 0, b = 0;
+  __shared__ int wp[16], wi[16];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const long per = (nn + 1023) / 1024, lo = min(nn, t * per), hi = min(nn, lo + per);
+  int a = 0, b = 0;  // at most n points and n + nn items: below 2^31
   for (long p = lo; p < hi; p++) {
     a += cnt[p];
-    b += (cnt[p] + 127) / 128;
+    b += (cnt[p] + 127) >> 7;
   }
-  sp[t] = a;
-  si[t] = b;
-  __syncthreads();
-  if (t == 0) {  // exclusive prefix over the 1024 partials
-    long ra = 0, rb = 0;
-    for (int u = 0; u < 1024; u++) {
-      const long xa = sp[u], xb = si[u];
-      sp[u] = ra;
-      si[u] = rb;
-      ra += xa;
-      rb += xb;
+  int ia = a, ib = b;  // inclusive scans
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int ua = __shfl_up(ia, o), ub = __shfl_up(ib, o);
+    if (lane >= o) {
+      ia += ua;
+      ib += ub;
     }
-    off[nn] = ra;
-    itoff[nn] = rb;
+  }
+  if (lane == 63) {
+    wp[wave] = ia;
+    wi[wave] = ib;
   }
   __syncthreads();
-  a = sp[t];
-  b = si[t];
+  for (int w = 0; w < wave; w++) {
+    ia += wp[w];
+    ib += wi[w];
+  }
+  if (t == 1023) {
+    off[nn] = ia;
+    itoff[nn] = ib;
+  }
+  a = ia - a;
+  b = ib - b;
   for (long p = lo; p < hi; p++) {
     off[p] = a;
     cursor[p] = a;
     itoff[p] = b;
     a += cnt[p];
-    b += (cnt[p] + 127) / 128;
+    b += (cnt[p] + 127) >> 7;
   }
 }
 
-__global__ void yk_hq_scatter_kernel(const int *__restrict__ node, long n, long *cursor,
-                                     int *__restrict__ perm) {
-  const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (i < n && node[i] >= 0) perm[atomicAdd((unsigned long long *)&cursor[node[i]], 1ull)] = (int)i;
-}
-
-// work item j -> (node, tile): the node by binary search over itoff
+// work item j -> (node, tile): the node by binary search over itoff; items
+// past the level's last one get node -1 (the assign skips them)
 __global__ void yk_hq_items_kernel(const long *__restrict__ itoff, long nn, long nitems,
                                    int *__restrict__ item_inst, int *__restrict__ item_tile) {
   const long j = blockIdx.x * (long)blockDim.x + threadIdx.x;
   if (j >= nitems) return;
+  if (j >= itoff[nn]) {
+    item_inst[j] = -1;
+    return;
+  }
   long lo = 0, hi = nn;  // itoff[lo] <= j < itoff[hi]
   while (hi - lo > 1) {
     const long mid = (lo + hi) >> 1;
@@ -695,6 +751,19 @@ __global__ void yk_hq_items_kernel(const long *__restrict__ itoff, long nn, long
   }
   item_inst[j] = (int)lo;
   item_tile[j] = (int)(j - itoff[lo]);
+}
+
+// the root's level: one node of all the points, in their own order
+__global__ void yk_hq_root_kernel(long n, long nitems, long *__restrict__ off,
+                                  int *__restrict__ item_inst, int *__restrict__ item_tile) {
+  const long j = blockIdx.x * (long)blockDim.x + threadIdx.x;
+  if (j == 0) {
+    off[0] = 0;
+    off[1] = n;
+  }
+  if (j >= nitems) return;
+  item_inst[j] = 0;
+  item_tile[j] = (int)j;
 }
 
 // the level's centroids with each node's bf children padded to kpad rows
@@ -713,10 +782,12 @@ __global__ void yk_hq_pad_kernel(const float *__restrict__ cl, const float *__re
   if (c4 == 0) dstn[row] = cnl[src];
 }
 
+// the points still descending (off[nn] of them): node = node * bf + child
 __global__ void yk_hq_update_kernel(const int *__restrict__ perm, const int *__restrict__ child,
-                                    long m, int bf, int *__restrict__ node) {
+                                    const long *__restrict__ off, long nn, int bf,
+                                    int *__restrict__ node) {
   const long j = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (j >= m) return;
+  if (j >= off[nn]) return;
   const int i = perm[j], c = child[j];
   node[i] = c < 0 ? -1 : node[i] * bf + c;
 }
@@ -726,70 +797,117 @@ __global__ void yk_hq_fill_kernel(int *p, long n, int v) {
   if (i < n) p[i] = v;
 }
 
+// The descent's workspace, kept for the next call up to YK_HQ_KEEP bytes (a
+// hipMalloc and hipFree per call wait for the device); a larger one is freed
+// with its call.  Used under the library lock.
+#define YK_HQ_KEEP ((size_t)256 << 20)
+static void *g_hq_mem = nullptr;
+static size_t g_hq_bytes = 0;
+
+static int yk_hq_descend(const float *v, const double *vn, long n, int d, int nlevel, int bf,
+                         const float *cent, const float *cn, int *idx, long nn_max, char *q) {
+  const int ld = yk_ld(d), kpad = (bf + 31) & ~31;
+  hipStream_t st = yk_stream();
+  auto carve = [&](size_t b) {
+    char *r = q;
+    q += (b + 255) & ~(size_t)255;
+    return (void *)r;
+  };
+  const size_t n_i = sizeof(int) * (size_t)n, nn_l = sizeof(long) * (size_t)(nn_max + 1);
+  const size_t items_max = (size_t)(n / 128 + nn_max + 1);
+  int *perm = (int *)carve(n_i), *child = (int *)carve(n_i);
+  float *dis = (float *)carve(n_i);
+  int *cnt = (int *)carve(sizeof(int) * (size_t)nn_max);
+  int *cursor = (int *)carve(sizeof(int) * (size_t)nn_max);
+  long *off = (long *)carve(nn_l), *itoff = (long *)carve(nn_l);
+  int *item_inst = (int *)carve(sizeof(int) * items_max);
+  int *item_tile = (int *)carve(sizeof(int) * items_max);
+  float *pc = (float *)carve(sizeof(float) * (size_t)nn_max * kpad * ld);
+  float *pcn = (float *)carve(sizeof(float) * (size_t)nn_max * kpad);
+  const unsigned gb = (unsigned)((n + 255) / 256);
+  const unsigned gs = (unsigned)((n + YK_HQ_SEG - 1) / YK_HQ_SEG);
+  long lvl = 0, nn = 1;  // first centroid row of the level, its parent nodes
+  for (int l = 0; l < nlevel; l++) {
+    // an upper bound of the level's work items: nothing is read back, the
+    // items past the last one are skipped
+    const long nitems = l == 0 ? (n + 127) / 128 : n / 128 + nn;
+    const unsigned gi = (unsigned)((nitems + 255) / 256);
+    if (l == 0) {
+      hipLaunchKernelGGL(yk_hq_root_kernel, dim3(gi), dim3(256), 0, st, n, nitems, off, item_inst,
+                         item_tile);
+    } else {
+      const bool lds = nn <= YK_HQ_LDS_NODES;
+      const size_t tab = sizeof(int) * (size_t)nn;
+      hipLaunchKernelGGL(yk_hq_fill_kernel, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, st,
+                         cnt, nn, 0);
+      if (lds)
+        hipLaunchKernelGGL(yk_hq_place_kernel<false>, dim3(gs), dim3(256), tab, st, idx, n,
+                           (int)nn, cnt, (int *)nullptr);
+      else
+        hipLaunchKernelGGL(yk_hq_place_many_kernel<false>, dim3(gb), dim3(256), 0, st, idx, n, cnt,
+                           (int *)nullptr);
+      hipLaunchKernelGGL(yk_hq_scan_kernel, dim3(1), dim3(1024), 0, st, cnt, nn, off, cursor,
+                         itoff);
+      if (lds)
+        hipLaunchKernelGGL(yk_hq_place_kernel<true>, dim3(gs), dim3(256), tab, st, idx, n, (int)nn,
+                           cursor, perm);
+      else
+        hipLaunchKernelGGL(yk_hq_place_many_kernel<true>, dim3(gb), dim3(256), 0, st, idx, n,
+                           cursor, perm);
+      hipLaunchKernelGGL(yk_hq_items_kernel, dim3(gi), dim3(256), 0, st, itoff, nn, nitems,
+                         item_inst, item_tile);
+    }
+    const long prow = nn * kpad * (ld / 4);
+    hipLaunchKernelGGL(yk_hq_pad_kernel, dim3((unsigned)((prow + 255) / 256)), dim3(256), 0, st,
+                       cent + lvl * ld, cn + lvl, nn, bf, kpad, ld, pc, pcn);
+    YK_HIP(hipGetLastError());
+    // the root's children are the points' nodes themselves
+    YK_TRY(yk_batch_assign_idx(nitems, item_inst, item_tile, off, d, bf, kpad, v, vn,
+                               l == 0 ? nullptr : perm, pc, pcn, nullptr, l == 0 ? idx : child,
+                               dis));
+    if (l > 0) {
+      hipLaunchKernelGGL(yk_hq_update_kernel, dim3(gb), dim3(256), 0, st, perm, child, off, nn, bf,
+                         idx);
+      YK_HIP(hipGetLastError());
+    }
+    lvl += nn * bf;
+    nn *= bf;
+  }
+  return YK_OK;
+}
+
 extern "C" int yk_hkm_quantize(const float *v, const double *vn, long n, int d, int nlevel, int bf,
                                const float *cent, const float *cn, int *idx) {
   YK_TRY(yk_init());
   if (n <= 0) return YK_OK;
   if (nlevel < 1 || bf < 1) return yk_set_error(YK_EINVAL, "yk_hkm_quantize: bad tree");
   if (n > 0x7fffffffL) return yk_set_error(YK_EINVAL, "yk_hkm_quantize: n exceeds int32");
+  YkGuard guard;  // the workspace
   const int ld = yk_ld(d), kpad = (bf + 31) & ~31;
-  hipStream_t st = yk_stream();
   // the widest level's parent nodes: bf^(nlevel-1)
   long nn_max = 1;
   for (int l = 1; l < nlevel; l++) nn_max *= bf;
-  void *mem = nullptr;
   const size_t n_i = sizeof(int) * (size_t)n, nn_l = sizeof(long) * (size_t)(nn_max + 1);
   const size_t items_max = (size_t)(n / 128 + nn_max + 1);
-  const size_t bytes = 4 * n_i + 3 * nn_l + sizeof(int) * (size_t)nn_max +
+  const size_t bytes = 3 * n_i + 2 * nn_l + 2 * sizeof(int) * (size_t)nn_max +
                        2 * sizeof(int) * items_max +
                        sizeof(float) * (size_t)nn_max * kpad * (ld + 1) + 16 * 256;
-  YK_TRY(yk_malloc(&mem, bytes));
-  char *q = (char *)mem;
-  auto carve = [&](size_t b) {
-    char *r = q;
-    q += (b + 255) & ~(size_t)255;
-    return (void *)r;
-  };
-  int *perm = (int *)carve(n_i), *child = (int *)carve(n_i);
-  float *dis = (float *)carve(n_i);
-  int *cnt = (int *)carve(sizeof(int) * (size_t)nn_max);
-  long *off = (long *)carve(nn_l), *cursor = (long *)carve(nn_l), *itoff = (long *)carve(nn_l);
-  int *item_inst = (int *)carve(sizeof(int) * items_max);
-  int *item_tile = (int *)carve(sizeof(int) * items_max);
-  float *pc = (float *)carve(sizeof(float) * (size_t)nn_max * kpad * ld);
-  float *pcn = (float *)carve(sizeof(float) * (size_t)nn_max * kpad);
-  int rc = YK_OK;
-  const unsigned gb = (unsigned)((n + 255) / 256);
-  hipLaunchKernelGGL(yk_hq_fill_kernel, dim3(gb), dim3(256), 0, st, idx, n, 0);  // node 0
-  long lvl = 0, nn = 1;  // first centroid row of the level, its parent nodes
-  for (int l = 0; l < nlevel && rc == YK_OK; l++) {
-    hipLaunchKernelGGL(yk_hq_fill_kernel, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, st,
-                       cnt, nn, 0);
-    hipLaunchKernelGGL(yk_hq_hist_kernel, dim3(gb), dim3(256), 0, st, idx, n, cnt);
-    hipLaunchKernelGGL(yk_hq_scan_kernel, dim3(1), dim3(1024), 0, st, cnt, nn, off, cursor,
-                       itoff);
-    hipLaunchKernelGGL(yk_hq_scatter_kernel, dim3(gb), dim3(256), 0, st, idx, n, cursor, perm);
-    long tot[2] = {0, 0};  // points still descending, work items
-    rc = yk_memcpy_d2h(&tot[0], off + nn, sizeof(long));
-    if (rc == YK_OK) rc = yk_memcpy_d2h(&tot[1], itoff + nn, sizeof(long));
-    if (rc != YK_OK || tot[0] == 0) break;
-    hipLaunchKernelGGL(yk_hq_items_kernel, dim3((unsigned)((tot[1] + 255) / 256)), dim3(256), 0,
-                       st, itoff, nn, tot[1], item_inst, item_tile);
-    const long prow = nn * kpad * (ld / 4);
-    hipLaunchKernelGGL(yk_hq_pad_kernel, dim3((unsigned)((prow + 255) / 256)), dim3(256), 0, st,
-                       cent + lvl * ld, cn + lvl, nn, bf, kpad, ld, pc, pcn);
-    YK_HIP(hipGetLastError());
-    rc = yk_batch_assign_idx(tot[1], item_inst, item_tile, off, d, bf, kpad, v, vn, perm, pc,
-                             pcn, nullptr, child, dis);
-    if (rc != YK_OK) break;
-    hipLaunchKernelGGL(yk_hq_update_kernel, dim3((unsigned)((tot[0] + 255) / 256)), dim3(256), 0,
-                       st, perm, child, tot[0], bf, idx);
-    YK_HIP(hipGetLastError());
-    lvl += nn * bf;
-    nn *= bf;
+  void *mem = nullptr;
+  if (bytes > YK_HQ_KEEP) {
+    YK_TRY(yk_malloc(&mem, bytes));
+  } else {
+    if (bytes > g_hq_bytes) {
+      if (g_hq_mem) YK_TRY(yk_free(g_hq_mem));
+      g_hq_mem = nullptr;
+      g_hq_bytes = 0;
+      YK_TRY(yk_malloc(&g_hq_mem, bytes));
+      g_hq_bytes = bytes;
+    }
+    mem = g_hq_mem;
   }
+  const int rc = yk_hq_descend(v, vn, n, d, nlevel, bf, cent, cn, idx, nn_max, (char *)mem);
   const int rs = yk_sync();
-  yk_free(mem);
+  if (mem != g_hq_mem) yk_free(mem);
   return rc != YK_OK ? rc : rs;
 }
 

@@ -198,7 +198,8 @@ __global__ __launch_bounds__(256) void yk_scan_f32(ScanArgs a0) {
   int tile, split;
   if (a0.item_inst) {
     const int inst = a0.item_inst[item];
-    if (a0.done && a0.done[inst]) continue;
+    // -1: an item past a level's last one (the tree descent's launch bound)
+    if (inst < 0 || (a0.done && a0.done[inst])) continue;
     tile = a0.item_tile[item];
     split = 0;
     const long off = a0.inst_off[inst];

@@ -474,3 +474,56 @@ def test_knn_large_k_weights_nan_and_k_equals_nb(ya, oracle):
         assert np.array_equal(np.sort(gd[:, :nfin], 1).view(np.int32),
                               np.sort(od[:, :nfin], 1).view(np.int32))
         parity.check_knn(2, q, b, k, gi, gd, oi, od, w=w, exact=True, label="nan k%d" % k)
+
+
+@pytest.mark.parametrize("nq,nb,d,k", [
+    (64, 700, 128, 1), (65, 701, 128, 1), (129, 33, 16, 1), (300, 5000, 8, 1), (700, 2049, 250, 1),
+    (1, 3000, 128, 2), (32, 999, 40, 16), (33, 1000, 56, 10), (64, 64, 128, 16),
+    (65, 17, 16, 16), (128, 1500, 24, 3), (129, 9000, 128, 10), (257, 20000, 64, 16),
+    (300, 4000, 112, 5), (100, 3001, 130, 7), (260, 2500, 256, 12), (70, 1200, 257, 4),
+    (300, 9001, 200, 60), (130, 6000, 129, 17)])
+@pytest.mark.parametrize("typ,weighted", [(2, False), (16, False), (2, True)])
+def test_scan_variants_bitexact(ya, oracle, nq, nb, d, k, typ, weighted):
+    """Each side of the scans' limits: 32 and 64 queries (streaming), 128
+    (one or two query tiles per wave), d = 16 .. 128, 256 and beyond (chunk
+    counts; blocks per stage), partial last blocks, k = 1, 2 .. 16 (proven
+    starting bound, no readback) and above, L2, dot product, weights.  Integer
+    data (weights are powers of two): the oracle's lists bit for bit."""
+    rng = np.random.default_rng(nq * 7 + nb + d * 3 + k + typ)
+    hi = 9 if d > 128 else 200
+    b = rng.integers(0, hi, (nb, d)).astype(np.float32)
+    q = rng.integers(0, hi, (nq, d)).astype(np.float32)
+    w = 2.0 ** rng.integers(-2, 3, nb).astype(np.float32) if weighted else None
+    print("scan", nq, nb, d, k, typ, weighted, flush=True)
+    gi, gd = ya.knn(q, b, k, distance_type=typ, weights=w)
+    oi, od = oracle.knn_full(typ, b, q, k, w)
+    parity.check_knn(typ, q, b, k, gi, gd, oi, od, w=w, exact=True,
+                     label="scan%d_%d_%d_%d" % (nq, nb, d, k))
+
+
+@pytest.mark.parametrize("nq", [5, 100, 300])
+@pytest.mark.parametrize("k", [2, 16])
+def test_small_k_overflow_and_nan(ya, oracle, nq, k):
+    """k <= 16 where thousands of rows lie within the starting bound (a base
+    of 6,000 equal rows and a few nearer ones outside the sampled blocks): the
+    candidate lists overflow and the register top-16 scan answers; NaN rows
+    and a NaN query never enter.  Exact ties go to the lowest index."""
+    rng = np.random.default_rng(k + nq)
+    nb, d = 40000, 24
+    b = rng.integers(100, 200, (nb, d)).astype(np.float32)
+    b[1000:7000] = 3.0
+    b[[33, 70, 12345]] = 2.0
+    b[5::97] = np.nan
+    q = np.zeros((nq, d), np.float32)
+    q[1::2] = rng.integers(0, 200, (nq // 2, d))
+    q[-1] = np.nan
+    print("overflow", nq, k, flush=True)
+    gi, gd = ya.knn(q, b, k)
+    oi, od = oracle.knn_full(2, b, q, k)
+    assert np.array_equal(gd.view(np.int32)[:-1], od.view(np.int32)[:-1])
+    # every finite query: the lists by (value, index)
+    for i in range(nq - 1):
+        dist = ((b.astype(np.float64) - q[i].astype(np.float64)) ** 2).sum(1)
+        want = np.lexsort((np.arange(nb), np.where(np.isnan(dist), np.inf, dist)))[:k]
+        assert np.array_equal(gi[i], want), i
+    assert (gi[-1] == -1).all()

@@ -465,7 +465,7 @@ extern "C" int yk_prof_get(int which, double *total_ms, long *count) {
 // ---------------------------------------------------------------------------
 // persistent-grid sizing
 
-#define YK_OCC_CACHE 64
+#define YK_OCC_CACHE 256
 static const void *g_occ_fn[YK_OCC_CACHE];
 static int g_occ_block[YK_OCC_CACHE], g_occ_val[YK_OCC_CACHE], g_occ_n = 0;
 static int g_cu_count = 0;

@@ -15,8 +15,9 @@
 //
 // Scan kernel (gfx950, wave64, v_mfma_f32_32x32x2_f32):
 //   * a workgroup of W waves; each wave owns 32*NB queries (the MFMA
-//     columns, held in registers when d <= 128) and streams its workgroup's
-//     base range in blocks of 32 rows (the MFMA rows) from global memory;
+//     columns, held in registers when d <= 128, in the LDS-staged kernel
+//     d <= 256) and takes its workgroup's base range in blocks of 32 rows (the
+//     MFMA rows), streamed from global memory or staged through LDS;
 //   * per 16-wide k-chunk a lane loads 8 contiguous floats (two dwordx4) of
 //     its row: A and B use the same k permutation, each 64-byte row segment
 //     is read once per block;
@@ -24,18 +25,19 @@
 //     the epilogue is lane-local:
 //       MODE 0  running (value, index) minimum           -> k = 1
 //       MODE 1  each lane's own minimum over its rows     -> the threshold
-//               sketch for k > 16
-//       MODE 2  register top-R of keys (R <= 16)          -> 2 <= k <= 16
+//               sketch for k > 1
+//       MODE 2  register top-R of keys (R <= 16)          -> what the filtered
+//               pass leaves over for k <= 16
 //       MODE 3  append every key <= the query's threshold T_q to a per-query
 //               candidate list (staged in LDS, one global
-//               atomic per YK_CSTAGE keys)                -> k > 16
+//               atomic per YK_CSTAGE keys)                -> k > 1
 //   * a persistent grid (resident workgroups only) walks the work items;
 //     each XCD owns a contiguous run of items so workgroups that share a
 //     base range share that XCD's L2;
 //   * the base is split over work items when the query tiles alone cannot
 //     fill 256 CUs; split results are merged by small sort kernels.
 //
-// k > 16 is exact in two passes: (A) MODE 1 over a 1-in-stride sample of
+// k > 1 is exact in two passes: (A) MODE 1 over a 1-in-stride sample of
 // base blocks with >= k splits gives, per query, >= 2k minima of disjoint
 // row subsets -- distinct real keys -- whose k-th smallest T_q bounds the
 // true k-th smallest key from above.  (B) MODE 3 over the whole base
@@ -48,9 +50,12 @@
 #include <pthread.h>
 #include <stdio.h>
 
+#include <type_traits>
+
 #include "../../include/yael_mi355x.h"
 #include "yk.h"
 #include "yk_dev.h"
+#include "yk_wsel.h"
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 // word 3 of a raw (untyped, stride 0) buffer descriptor on gfx9-family GPUs
@@ -92,6 +97,9 @@ struct ScanArgs {
   const int *done;  // instances already finished (skipped)
   const int *qidx;  // optional: point j of the concatenation is row qidx[j] of q / qn
   int *tick;        // per XCD, zero at launch: item tickets (nullptr: static order)
+  const int *flag;  // MODE 2 as the fallback of the filtered search: 0 = nothing left to do
+  int units;        // yk_scan_f32_lds, MODE 0: > 0 even shares of tiles x units blocks
+  int inter;        // MODE 1: split s takes sampled blocks s, s + nsplit, ...
 };
 
 // The hardware hands consecutive block ids to the 8 XCDs in turn; give each
@@ -113,22 +121,67 @@ __device__ __forceinline__ void yk_reg_insert(uint64_t (&t)[R], uint64_t x) {
   t[0] = x < t[0] ? x : t[0];
 }
 
+// A lane's 16 row norms, in registers or (the LDS-staged kernel) read from
+// LDS where they are used: value i's norm is float 8 (i >> 2) + (i & 3) of
+// the lane half's block norms.
+struct YkNormRegs {
+  float n[16];
+  __device__ __forceinline__ float operator[](int i) const { return n[i]; }
+};
+struct YkNormLds {
+  const float *p;
+  __device__ __forceinline__ float operator[](int i) const { return p[8 * (i >> 2) + (i & 3)]; }
+  __device__ __forceinline__ float pick(int is) const { return p[8 * (is >> 2) + (is & 3)]; }
+};
+
+// The approximations of a lane's 16 values, m_i = bn - 2 acc (type 16: acc);
+// fl(qn + m_i) differs from the exact expression by far less than slack =
+// 2^-19 (|q|^2 + max|b|^2) (|2 q.b| <= |q|^2 + |b|^2).  Returns their minimum;
+// x -> fl(qn + x) is monotone, so the query norm is added once, to it.
+template <bool DOT, class Norms>
+__device__ __forceinline__ float yk_approx16(const f32x16 &acc, const Norms &nn, float (&m)[16]) {
+  float mm = INFINITY;
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    m[i] = DOT ? acc[i] : __builtin_fmaf(-2.0f, acc[i], nn[i]);
+    mm = fminf(mm, m[i]);
+  }
+  return mm;
+}
+
+// Of the lane's values with m_i <= th: how many, and the last one's i and
+// acc.  One candidate per lane is the common case of the filtered pass: the
+// wave then evaluates, tests and appends one exact value, not sixteen.
+__device__ __forceinline__ int yk_pick16(const f32x16 &acc, const float (&m)[16], float th,
+                                         int &is, float &as) {
+  int cnt = 0;
+  is = 0;
+  as = acc[0];
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    const bool c = m[i] <= th;
+    cnt += c ? 1 : 0;
+    is = c ? i : is;
+    as = c ? acc[i] : as;
+  }
+  return cnt;
+}
+
 // One full block's epilogue for k = 1 and the sketch (each lane keeps the best
-// of its own rows), unweighted.  The lane's 16 values are tested first on
-// the float approximation qn + (bn - 2 acc), which differs from the exact
-// expression by far less than slack = 2^-19 (|q|^2 + max|b|^2)
-// (|2 q.b| <= |q|^2 + |b|^2); x -> fl(qn + x) is monotone, so the query
-// norm is added once, to the minimum of bn - 2 acc.  A block that may hold
-// a better value takes the exact FP64-normed expression for all 16 values,
-// branch-free, in ascending row order with a strict '<' (the smallest index
-// wins a tie).  The test is skipped (test = false) for a range's first
-// blocks: a wave runs the exact pass when any of its 64 lanes may improve,
-// which at block j of a range happens with probability about
-// 1 - (1 - 1/(j+1))^64, so early blocks would pay for both.
-template <bool DOT>
-__device__ __forceinline__ void yk_best1_block(const f32x16 &acc, const float (&nn)[16],
-                                               double qnd, long bb, int h, bool test, float &bv,
-                                               int &bi) {
+// of its own rows), unweighted.  With `test` the float approximations decide
+// first whether any of the lane's values can improve its best; a range's
+// first blocks go without: a wave runs the exact pass when any of its 64
+// lanes may improve, which at block j of a range happens with probability
+// about 1 - (1 - 1/(j+1))^64, so early blocks would pay for both.  The exact
+// pass takes the exact FP64-normed expression for all 16 values, branch-free,
+// in ascending row order with a strict '<' (the smallest index wins a tie).
+// (Picking out the lanes' one candidate by the approximations first, to
+// evaluate one exact value per lane, measured slower: 26.8 against 18.2 ms
+// for the 8 sub-spaces of 1e6 points, d = 16, k = 256, 10 iterations -- the
+// selects cost as much as the FP64 operations they replace.)
+template <bool DOT, class Norms>
+__device__ __forceinline__ void yk_best1_block(const f32x16 &acc, const Norms &nn, double qnd,
+                                               long bb, int h, bool test, float &bv, int &bi) {
   // Empty asm statements on the operands keep each pass inside its branch
   // (the compiler would otherwise hoist parts it shares with the general
   // path, executing them for every block).
@@ -148,18 +201,36 @@ __device__ __forceinline__ void yk_best1_block(const f32x16 &acc, const float (&
   }
   double qd = qnd;
   asm volatile("" : "+v"(qd));
-  // value i sits at row bb + 4 h + 8 (i >> 2) + (i & 3)
-  int bo = -1;
+  // value i sits at row bb + 4 h + 8 (i >> 2) + (i & 3); values 0-7 and 8-15
+  // as two chains, the first also holding the earlier blocks' best.  (The
+  // fused form rounds as bn+qn - 2 acc does: 2 acc is exact, and where it
+  // would overflow the norms' sum has too.)
+  float b0 = bv, b1 = bv;
+  int o0 = -1, o1 = -1;
 #pragma unroll
-  for (int i = 0; i < 16; i++) {
-    float ax = acc[i], nx = nn[i];
-    asm volatile("" : "+v"(ax), "+v"(nx));
-    const float v = DOT ? ax : (float)(qd + (double)nx) - 2.0f * ax;
-    const bool take = v < bv;
-    bv = take ? v : bv;
-    bo = take ? 8 * (i >> 2) + (i & 3) : bo;
+  for (int i = 0; i < 8; i++) {
+    const float v0 = DOT ? acc[i] : __builtin_fmaf(-2.0f, acc[i], (float)(qd + (double)nn[i]));
+    const float v1 =
+        DOT ? acc[i + 8] : __builtin_fmaf(-2.0f, acc[i + 8], (float)(qd + (double)nn[i + 8]));
+    const bool t0 = v0 < b0, t1 = v1 < b1;
+    b0 = t0 ? v0 : b0;
+    o0 = t0 ? 8 * (i >> 2) + (i & 3) : o0;
+    b1 = t1 ? v1 : b1;
+    o1 = t1 ? 16 + 8 * (i >> 2) + (i & 3) : o1;
   }
+  const bool t = b1 < b0;
+  bv = t ? b1 : b0;
+  const int bo = t ? o1 : o0;
   if (bo >= 0) bi = (int)bb + 4 * h + bo;
+}
+
+// the largest of a lane's 16 row norms
+template <class Norms>
+__device__ __forceinline__ float yk_max16(const Norms &nn) {
+  float nmax = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; i++) nmax = fmaxf(nmax, nn[i]);
+  return nmax;
 }
 
 // NCH > 0: queries register-resident, exactly NCH 16-wide chunks (ld = 16
@@ -174,6 +245,7 @@ __global__ __launch_bounds__(256) void yk_scan_f32(ScanArgs a0) {
   // XCD x owns the contiguous run of work items [x*per_xcd, (x+1)*per_xcd)
   // (split-major, so concurrently running workgroups of one XCD share a base
   // range in its L2), and its workgroups stride through that run.
+  if (MODE == 2 && a0.flag && *a0.flag == 0) return;
   const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3, wpx = gridDim.x >> 3;
   const int ibeg = xcd * a0.per_xcd, iend = min(a0.total, ibeg + a0.per_xcd);
   // MODE 3: candidate keys are staged in LDS, YK_CSTAGE per (query tile,
@@ -220,8 +292,13 @@ __global__ __launch_bounds__(256) void yk_scan_f32(ScanArgs a0) {
     split = item / a0.tiles_x;
   }
   const long qbase = ((long)tile * nwave + wave) * (32 * NB);
-  const long bbeg = (long)split * a.brange;
-  const long bend = min(a.nb, bbeg + a.brange);
+  // (interleaved sketch splits: neighbouring sampled blocks fall into
+  // different splits, so rows near each other in the base do not all end up
+  // in one subset's minimum)
+  const bool inter = MODE == 1 && a.inter;
+  const long bbeg = (long)split * (inter ? a.bstep : a.brange);
+  const long bend = inter ? a.nb : min(a.nb, bbeg + a.brange);
+  if (inter) a.bstep *= a.nsplit;
   const int nch = a.ld >> 4;
   const int ld = a.ld;
   const bool dot = (a.type == YK_DOT);
@@ -259,11 +336,11 @@ __global__ __launch_bounds__(256) void yk_scan_f32(ScanArgs a0) {
     ncs[j] = 0;
 #pragma unroll
     for (int s = 0; s < (MODE == 2 ? R : 1); s++) top[j][s] = YK_KEY_NONE;
-    T[j] = MODE == 3 ? a.thr[qrow[j]] : 0;
+    T[j] = MODE == 3 || (MODE == 2 && a.thr) ? a.thr[qrow[j]] : 0;
     Tv[j] = (T[j] == 0) ? -INFINITY
                         : (T[j] == YK_KEY_NONE ? INFINITY : yk_fkey_inv((uint32_t)(T[j] >> 32)));
   }
-  if (MODE == 3) {
+  if (MODE == 3 || (MODE == 2 && a.thr)) {
     bool act = false;
 #pragma unroll
     for (int j = 0; j < NB; j++) act |= qok[j] && T[j] != 0;
@@ -385,7 +462,9 @@ __global__ __launch_bounds__(256) void yk_scan_f32(ScanArgs a0) {
     }
 
     // epilogue: lane holds query column r and base rows 8g + 4h + e
-    float nn[16], ww[16];
+    YkNormRegs nrm;
+    float (&nn)[16] = nrm.n;
+    float ww[16];
 #pragma unroll
     for (int g = 0; g < 4; g++) {
       const long b4 = bb + 8 * g + 4 * h;
@@ -404,9 +483,9 @@ __global__ __launch_bounds__(256) void yk_scan_f32(ScanArgs a0) {
         if (!wts && bb + 32 <= bend) {
           const bool test = bb - bbeg >= 48L * a.bstep;
           if (dot)
-            yk_best1_block<true>(acc[j], nn, qnd[j], bb, h, test, bv[j], bi[j]);
+            yk_best1_block<true>(acc[j], nrm, qnd[j], bb, h, test, bv[j], bi[j]);
           else
-            yk_best1_block<false>(acc[j], nn, qnd[j], bb, h, test, bv[j], bi[j]);
+            yk_best1_block<false>(acc[j], nrm, qnd[j], bb, h, test, bv[j], bi[j]);
           continue;
         }
       }
@@ -511,6 +590,418 @@ __global__ __launch_bounds__(256) void yk_scan_f32(ScanArgs a0) {
 }
 
 // ---------------------------------------------------------------------------
+// LDS-staged scan: k = 1, the sketch and the filtered pass for more than 64
+// queries and d <= 256.
+//
+// The streaming kernel above loads every base fragment once per wave, 16
+// bytes from each of 32 rows per instruction: the vector L1 takes those rows
+// one line at a time and bounded it at 55-60% of the FP32 MFMA rate (d = 128;
+// n = 1e5 points to 1,024 centroids 0.290 ms, 90 TFLOP/s).  Here the
+// workgroup's four waves share each block: a 32-row block is one contiguous
+// piece of memory, loaded 1 KB per wave instruction straight into the other
+// of two LDS buffers while a stage is multiplied (no registers hold it: 16
+// of them made the two-tile kernel spill).  The four 16-byte units of a
+// row's chunk are stored in the order unit ^ (row & 3), which spreads the
+// rows' reads over four times the banks and leaves the chunk a constant
+// offset of the read's address.  One barrier per stage.  Two query tiles per wave (NB = 2, d <= 128:
+// 128 registers of queries) use each fragment read from LDS twice; short
+// vectors stage G blocks at once so that a stage is at least 64 MFMAs per
+// tile.  Same MFMA operands, same order, same epilogue arithmetic as the
+// streaming kernel: the same bits.  n = 1e5 points to 1,024 centroids: 0.290
+// -> 0.235 ms (112 TFLOP/s; n = 1e6: 123).  What is left of the FP32 rate
+// (153 TFLOP/s for a large library product): timing builds without the
+// epilogue 135, without the loads too 141 TFLOP/s at n = 1e6, and at n = 1e5
+// ~0.03 ms of start (every workgroup's 128 KB of queries at once).
+template <int NCH>
+struct YkLdsShape {
+  static constexpr int U = 4 * NCH;  // float4 units of a row
+  static constexpr int G = NCH == 1 ? 8 : NCH == 2 ? 4 : NCH <= 4 ? 2 : 1;  // blocks per stage
+  static constexpr int KL = G * 32 * U / 64;  // 1 KB wave loads of a stage
+  static constexpr int NL = (KL + 3) / 4;     // of them per wave
+  // MODE 3: keys staged per (lane, query tile); fewer where two workgroups
+  // would not fit a CU's LDS otherwise
+  static constexpr int CST = NCH > 8 ? 4 : 8;
+};
+
+// the first of the W even shares of T units that covers unit u; shares are
+// [w T / W, (w + 1) T / W)
+__device__ __forceinline__ long yk_share_of(long u, long T, long W) {
+  long w = u * W / T;
+  while ((w + 1) * T / W <= u) w++;
+  while (w * T / W > u) w--;
+  return w;
+}
+
+// 16 bytes per lane from rs at voff straight to LDS at dst + 16 lane (dst
+// uniform over the wave; complete when vmcnt says so)
+__device__ __forceinline__ void yk_load_lds16(__amdgpu_buffer_rsrc_t rs, float4 *dst, int voff) {
+#ifdef __HIP_DEVICE_COMPILE__  // (the host pass does not know the 16-byte form)
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void *)dst, 16,
+                                           voff, 0, 0, 0);
+#endif
+}
+
+template <int NB, int NCH, int MODE, bool WT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void
+yk_scan_f32_lds(ScanArgs a0) {
+  using S = YkLdsShape<NCH>;
+  constexpr int U = S::U, G = S::G, KL = S::KL, NL = S::NL, CST = S::CST;
+  constexpr int ld = 16 * NCH, TQ = 128 * NB;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 31, h = lane >> 5;
+  // (the tiles first: the LDS offset of a direct load is 16 bits wide)
+  struct Shared {
+    float4 tile[2][G * 32 * U];
+    float norm[2][G * 32];
+    float wt[2][WT ? G * 32 : 1];
+    uint64_t cstage[MODE == 3 ? 4 * NB * 64 * CST : 1];
+    int item;
+  };
+  __shared__ Shared sm;
+  uint64_t *const cs = sm.cstage + (MODE == 3 ? wave * NB * 64 * CST : 0);
+  const bool dot = a0.type == YK_DOT;
+
+  // Work: split items with per-XCD tickets, as above; or, MODE 0 over a base
+  // that stays in the L2 (a0.units blocks), an even share of the tiles x
+  // units (tile, block) pairs per workgroup: a share that covers a tile only
+  // in part leaves its minima in part[(share, head or tail), query] for
+  // yk_merge_share_kernel.
+  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3, wpx = gridDim.x >> 3;
+  const int ibeg = xcd * a0.per_xcd, iend = min(a0.total, ibeg + a0.per_xcd);
+  const long T_units = (long)a0.tiles_x * a0.units;
+  long cur = a0.units ? blockIdx.x * T_units / gridDim.x : 0;
+  const long cend = a0.units ? (blockIdx.x + 1L) * T_units / gridDim.x : 0;
+  auto next_item = [&](int it) {
+    if (!a0.tick) return it + wpx;
+    __syncthreads();
+    if (tid == 0) sm.item = ibeg + wpx + atomicAdd(&a0.tick[xcd], 1);
+    __syncthreads();
+    return sm.item;
+  };
+  for (int item = ibeg + local; a0.units ? cur < cend : item < iend;
+       item = a0.units ? 0 : next_item(item)) {
+    ScanArgs a = a0;
+    int tile, split = 0, slot = -1;
+    long bbeg, bend, bstep = a0.bstep;
+    if (a0.units) {
+      tile = (int)(cur / a0.units);
+      const long b0 = cur - (long)tile * a0.units;
+      const long b1 = min((long)a0.units, b0 + (cend - cur));
+      cur += b1 - b0;
+      slot = b0 > 0 ? 0 : (b1 < a0.units ? 1 : -1);
+      bbeg = 32 * b0;
+      bend = min(a.nb, 32 * b1);
+    } else if (MODE == 0 && NB == 1 && a0.item_inst) {
+      const int inst = a0.item_inst[item];
+      if (inst < 0 || (a0.done && a0.done[inst])) continue;
+      tile = a0.item_tile[item];
+      const long off = a0.inst_off[inst];
+      if (a0.qidx) {
+        a.qidx = a0.qidx + off;
+      } else {
+        a.q = a0.q + off * ld;
+        a.qn = a0.qn + off;
+      }
+      a.nq = a0.inst_off[inst + 1] - off;
+      a.b = a0.b + (long)inst * a0.kpad * ld;
+      a.bn = a0.bn + (long)inst * a0.kpad;
+      a.nb = a0.kc;
+      a.out_i = a0.out_i + off;
+      a.out_d = a0.out_d + off;
+      bbeg = 0;
+      bend = a.nb;
+    } else {
+      tile = item % a0.tiles_x;
+      split = item / a0.tiles_x;
+      if (MODE == 1 && a0.inter) {
+        bbeg = (long)split * a0.bstep;
+        bend = a.nb;
+        bstep = a0.bstep * a0.nsplit;
+      } else {
+        bbeg = (long)split * a0.brange;
+        bend = min(a.nb, bbeg + a0.brange);
+      }
+    }
+    const long qbase = ((long)tile * 4 + wave) * (32 * NB);
+    const bool live = qbase < a.nq;  // the wave's queries exist (uniform)
+
+    int qrow[NB];
+    long qsrc[NB];
+    bool qok[NB];
+    double qnd[NB];
+    float bv[NB], Tv[NB];
+    int bi[NB], ncs[NB];
+    bool act = false;
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+      const long qi = qbase + j * 32 + r;
+      qok[j] = qi < a.nq;
+      qrow[j] = (int)(qok[j] ? qi : a.nq - 1);
+      qsrc[j] = MODE == 0 && NB == 1 && a.qidx ? (long)a.qidx[qrow[j]] : qrow[j];
+      qnd[j] = dot ? 0.0 : a.qn[qsrc[j]];
+      bv[j] = 1e30f;
+      bi[j] = -1;
+      ncs[j] = 0;
+      // MODE 3: the bound's value (its row is looked up where a value equals
+      // it); 0: the query is already final
+      const uint64_t T = MODE == 3 ? a.thr[qrow[j]] : 0;
+      Tv[j] = T == 0 || !qok[j] ? -INFINITY
+                                : (T == YK_KEY_NONE ? INFINITY : yk_fkey_inv((uint32_t)(T >> 32)));
+      act |= qok[j] && T != 0;
+    }
+    if (MODE == 3 && !__syncthreads_or(act)) continue;  // every query of the tile is final
+    float4 qreg[NB][2 * NCH];
+    if (live) {
+#pragma unroll
+      for (int j = 0; j < NB; j++)
+#pragma unroll
+        for (int c = 0; c < NCH; c++) {
+          const float *p = a.q + qsrc[j] * ld + c * 16 + h * 8;
+          qreg[j][2 * c] = *(const float4 *)p;
+          qreg[j][2 * c + 1] = *(const float4 *)(p + 4);
+        }
+    }
+    auto flush = [&](int j, int n) {
+      const int base = atomicAdd(&a.cnt[qrow[j]], n);
+      const uint64_t *src = cs + (j * 64 + lane) * CST;
+      for (int s_ = 0; s_ < n; s_++)
+        if (base + s_ < YK_CAND_CAP) a.cand[(long)qrow[j] * YK_CAND_CAP + base + s_] = src[s_];
+    };
+
+    // wave load i of a stage: lane l stores unit 64 (4 i + wave) + l of the
+    // stage's LDS image, (row, place) = (unit / U, unit % U)
+    int voff[NL];
+#pragma unroll
+    for (int i = 0; i < NL; i++) {
+      const int unit = 64 * (4 * i + wave) + lane, g = unit / (32 * U);
+      const int row = unit / U % 32, u = unit % U ^ (row & 3);
+      voff[i] = (int)((g * bstep * ld + row * ld + u * 4) * 4);
+    }
+    const int nst = (int)(((bend - bbeg + bstep - 1) / bstep + G - 1) / G);
+    const long nb32 = (a.nb + 31) & ~31L;
+    float ld_n = 0.f, ld_w = 0.f;
+    auto load = [&](int st, int buf) {
+      const long row = bbeg + (long)st * G * bstep;  // the stage's first row, below bend
+      // (rows past the base read as zeros; their values are masked)
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+          (void *)(a.b + row * ld), 0, (int)min((a.nb - row) * ld * 4, 0x7fffffffL),
+          YK_BUF_DWORD3);
+#pragma unroll
+      for (int i = 0; i < NL; i++)
+        if (KL % 4 == 0 || 4 * i + wave < KL)
+          yk_load_lds16(rs, sm.tile[buf] + 64 * (4 * i + wave), voff[i]);
+      if (tid < 32 * G) {
+        const long nr = row + (tid >> 5) * bstep + (tid & 31);
+        if (!dot) ld_n = nr < nb32 ? a.bn[nr] : 0.f;
+        if (WT) ld_w = nr < nb32 ? a.w[nr] : 0.f;
+      }
+    };
+    // the stage's norms, and the wait for its direct loads
+    auto store = [&](int buf) {
+      if (tid < 32 * G) {
+        sm.norm[buf][tid] = ld_n;
+        if (WT) sm.wt[buf][tid] = ld_w;
+      }
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    };
+
+    auto block = [&](const float4 *tp, const float *np, const float *wp, long bb, bool test) {
+      f32x16 acc[NB];
+#pragma unroll
+      for (int j = 0; j < NB; j++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[j][e] = 0.f;
+      // row r's units 2 h and 2 h + 1 of chunk c sit at 4 c + (unit ^ (r & 3))
+      const float4 *tp0 = tp + ((2 * h) ^ (r & 3)), *tp1 = tp + ((2 * h + 1) ^ (r & 3));
+      float4 av[2][2];
+      av[0][0] = tp0[0];
+      av[0][1] = tp1[0];
+#pragma unroll
+      for (int c = 0; c < NCH; c++) {
+        if (c + 1 < NCH) {
+          av[(c + 1) & 1][0] = tp0[4 * c + 4];
+          av[(c + 1) & 1][1] = tp1[4 * c + 4];
+        }
+        const float4 x0 = av[c & 1][0], x1 = av[c & 1][1];
+        const float xs[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+        for (int t = 0; t < 8; t++)
+#pragma unroll
+          for (int j = 0; j < NB; j++) {
+            const float4 y = qreg[j][2 * c + (t >> 2)];
+            const float ys = (t & 3) == 0 ? y.x : (t & 3) == 1 ? y.y : (t & 3) == 2 ? y.z : y.w;
+            acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(xs[t], ys, acc[j], 0, 0, 0);
+          }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      const YkNormLds nn = {np};
+#pragma unroll
+      for (int j = 0; j < NB; j++) {
+        if constexpr (MODE != 3) {
+          if (!WT && bb + 32 <= bend) {
+            if (dot)
+              yk_best1_block<true>(acc[j], nn, qnd[j], bb, h, test, bv[j], bi[j]);
+            else
+              yk_best1_block<false>(acc[j], nn, qnd[j], bb, h, test, bv[j], bi[j]);
+            continue;
+          }
+        }
+        // Only a lane with a value that may enter goes on; one such value
+        // is taken by itself, several by the loop over all 16.  Weighted
+        // values are w times the approximations, so within |w| slack of the
+        // exact ones (and 1e-36 covers products that round in the denormal
+        // range).  Negated comparisons: a NaN goes on to the exact test.
+        const float lim = MODE == 3 ? Tv[j] : bv[j];
+        const float qf = (float)qnd[j];
+        const float slack = dot ? 0.f : 0x1p-19f * (qf + yk_max16(nn));
+        const long b0 = bb + 4 * h;
+        auto enter = [&](float v, int i) {  // the exact value i of the lane
+          const long bidx = b0 + 8 * (i >> 2) + (i & 3);
+          if (MODE != 3) {
+            if (bidx < bend && v < bv[j]) {  // strict '<' in ascending index order
+              bv[j] = v;
+              bi[j] = (int)bidx;
+            }
+          } else if (bidx < bend && v <= Tv[j] && Tv[j] > -INFINITY) {  // (drops NaN)
+            const uint64_t key = yk_key(v, (int)bidx);
+            if (v < Tv[j] || key <= a.thr[qrow[j]]) {
+              const int n = ncs[j];
+              cs[(j * 64 + lane) * CST + n] = key;
+              if (n + 1 == CST) {
+                flush(j, CST);
+                ncs[j] = 0;
+              } else {
+                ncs[j] = n + 1;
+              }
+            }
+          }
+        };
+        auto exact = [&](float ac, float nm) {
+          return dot ? ac : (float)(qnd[j] + (double)nm) - 2.0f * ac;
+        };
+        if constexpr (!WT) {
+          float m[16];
+          const float mm = dot ? yk_approx16<true>(acc[j], nn, m) : yk_approx16<false>(acc[j], nn, m);
+          if (qf + mm - slack > lim || mm == INFINITY) {
+            if (lim < INFINITY) continue;
+          }
+          // m_i <= th for every value that may enter: qf + m_i - slack <=
+          // lim, with twice the slack for the roundings of this line
+          int is;
+          float as;
+          const int cnt = yk_pick16(acc[j], m, dot ? lim : lim - qf + 2.0f * slack, is, as);
+          if (cnt == 1) {
+            enter(exact(as, nn.pick(is)), is);
+          } else if (cnt > 1 || !(lim < INFINITY)) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) enter(exact(acc[j][i], nn[i]), i);
+          }
+        } else {
+          // (the value's weighted approximation less its error, against the
+          // bound: a lane's one such value by itself, several by the loop)
+          const float limw = lim + 1e-36f;
+          const YkNormLds ww = {wp};
+          int cnt = 0, is = 0;
+          float as = acc[j][0];
+#pragma unroll
+          for (int i = 0; i < 16; i++) {
+            const float ap = dot ? acc[j][i] : qf + __builtin_fmaf(-2.0f, acc[j][i], nn[i]);
+            const bool c = !(ap * ww[i] - slack * fabsf(ww[i]) > limw);
+            cnt += c ? 1 : 0;
+            is = c ? i : is;
+            as = c ? acc[j][i] : as;
+          }
+          if (cnt == 1) {
+            enter(exact(as, nn.pick(is)) * ww.pick(is), is);
+          } else if (cnt > 1) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) enter(exact(acc[j][i], nn[i]) * ww[i], i);
+          }
+        }
+      }
+    };
+
+    load(0, 0);
+    store(0);
+    __syncthreads();
+    for (int st = 0; st < nst; st++) {
+      const int buf = st & 1;
+      if (st + 1 < nst) load(st + 1, buf ^ 1);
+      if (live) {
+#pragma unroll 1
+        for (int g = 0; g < G; g++) {
+          const long bb = bbeg + ((long)st * G + g) * bstep;
+          if (bb >= bend) break;
+          block(sm.tile[buf] + (g * 32 + r) * U, sm.norm[buf] + g * 32 + 4 * h,
+                sm.wt[buf] + (WT ? g * 32 + 4 * h : 0), bb, st * G + g >= 48);
+        }
+      }
+      if (st + 1 < nst) store(buf ^ 1);
+      __syncthreads();
+    }
+
+    if (MODE == 0) {
+#pragma unroll
+      for (int j = 0; j < NB; j++) {
+        const float ov = __shfl_xor(bv[j], 32);
+        const int oi = __shfl_xor(bi[j], 32);
+        if (ov < bv[j] || (ov == bv[j] && oi < bi[j])) {
+          bv[j] = ov;
+          bi[j] = oi;
+        }
+        const long qi = qbase + j * 32 + r;
+        if (h == 0 && qok[j]) {
+          const uint64_t key = bi[j] < 0 ? YK_KEY_NONE : yk_key(bv[j], bi[j]);
+          if (slot >= 0) {
+            a.part[(blockIdx.x * 2L + slot) * TQ + wave * 32 * NB + j * 32 + r] = key;
+          } else if (a.nsplit > 1) {
+            a.part[qi * a.nsplit + split] = key;
+          } else {
+            a.out_d[qi] = bv[j];
+            a.out_i[qi] = bi[j];
+          }
+        }
+      }
+    } else if (MODE == 1) {
+#pragma unroll
+      for (int j = 0; j < NB; j++) {
+        const long qi = qbase + j * 32 + r;
+        if (qok[j])
+          a.part[(qi * a.nsplit + split) * 2 + h] = bi[j] < 0 ? YK_KEY_NONE : yk_key(bv[j], bi[j]);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < NB; j++)
+        if (ncs[j] > 0) flush(j, ncs[j]);
+    }
+  }  // work
+}
+
+// k = 1 over even shares (yk_scan_f32_lds with units): the queries of tiles
+// cut by a share's end, from the shares' minima (at most W + 1 of the tiles
+// are cut; the others were written by the scan)
+__global__ __launch_bounds__(256) void yk_merge_share_kernel(const uint64_t *__restrict__ part,
+                                                             long nq, int tq, long units, long T,
+                                                             long W, int *out_i, float *out_d) {
+  const long q = blockIdx.x * 256L + threadIdx.x;
+  if (q >= nq) return;
+  const long tile = q / tq, lo = tile * units, hi = lo + units;
+  long w = yk_share_of(lo, T, W);
+  if ((w + 1) * T / W >= hi) return;  // one share covers the tile
+  uint64_t best = YK_KEY_NONE;
+  for (; w < W; w++) {
+    const long s = w * T / W;
+    if (s >= hi) break;
+    if ((w + 1) * T / W == s) continue;  // an empty share
+    const uint64_t v = part[(w * 2 + (s > lo ? 0 : 1)) * tq + q % tq];
+    best = v < best ? v : best;
+  }
+  out_i[q] = best == YK_KEY_NONE ? -1 : (int)(uint32_t)best;
+  out_d[q] = best == YK_KEY_NONE ? 1e30f : yk_fkey_inv((uint32_t)(best >> 32));
+}
+
+// ---------------------------------------------------------------------------
 // small per-query sorts
 
 __device__ __forceinline__ void yk_store_key(uint64_t key, int *oi, float *od) {
@@ -518,22 +1009,23 @@ __device__ __forceinline__ void yk_store_key(uint64_t key, int *oi, float *od) {
   *od = key == YK_KEY_NONE ? __uint_as_float(0xffffffffu) : yk_fkey_inv((uint32_t)(key >> 32));
 }
 
-// k = 1 merge of per-split minima (nothing below 1e30 -> (-1, 1e30))
-__global__ void yk_merge1_kernel(const uint64_t *__restrict__ part, long nq, int nsplit,
-                                 int *out_i, float *out_d) {
-  long q = blockIdx.x * (long)blockDim.x + threadIdx.x;
+// k = 1 merge of per-split minima (nothing below 1e30 -> (-1, 1e30)): one
+// wave per query, its lanes striding the splits (a thread per query walked
+// them one by one)
+__global__ __launch_bounds__(256) void yk_merge1_kernel(const uint64_t *__restrict__ part, long nq,
+                                                        int nsplit, int *out_i, float *out_d) {
+  const long q = blockIdx.x * 4L + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
   if (q >= nq) return;
   uint64_t best = YK_KEY_NONE;
-  for (int s = 0; s < nsplit; s++) {
-    uint64_t v = part[q * nsplit + s];
+  for (int s = lane; s < nsplit; s += 64) {
+    const uint64_t v = part[q * nsplit + s];
     best = v < best ? v : best;
   }
-  if (best == YK_KEY_NONE) {
-    out_i[q] = -1;
-    out_d[q] = 1e30f;
-  } else {
-    out_i[q] = (int)(uint32_t)best;
-    out_d[q] = yk_fkey_inv((uint32_t)(best >> 32));
+  best = yk_wave_min64(best);
+  if (lane == 0) {
+    out_i[q] = best == YK_KEY_NONE ? -1 : (int)(uint32_t)best;
+    out_d[q] = best == YK_KEY_NONE ? 1e30f : yk_fkey_inv((uint32_t)(best >> 32));
   }
 }
 
@@ -556,43 +1048,114 @@ __device__ void yk_block_bitonic(uint64_t *s, int p2) {
   }
 }
 
-// Sort the n keys of each query (src + q*n); then either write the k
-// smallest (out_i/out_d) or, when thr != NULL, the k-th smallest as the
-// query's threshold (YK_KEY_NONE when fewer than k real keys: admit all).
+// The k smallest of each query's n keys (src + q*n), sorted: the end of the
+// register top-R scan, for the queries the filtered pass left (*flag != 0,
+// thr[q] != 0).
 __global__ __launch_bounds__(256) void yk_sortsel_kernel(const uint64_t *__restrict__ src,
                                                          int n, int k, int p2, int *out_i,
-                                                         float *out_d, uint64_t *thr) {
+                                                         float *out_d,
+                                                         const uint64_t *__restrict__ thr,
+                                                         const int *__restrict__ flag) {
   extern __shared__ uint64_t s[];
+  if (*flag == 0) return;
   const long q = blockIdx.x;
+  if (thr[q] == 0) return;
   const uint64_t *p = src + q * (long)n;
   for (int i = threadIdx.x; i < p2; i += blockDim.x) s[i] = i < n ? p[i] : YK_KEY_NONE;
   __syncthreads();
   yk_block_bitonic(s, p2);
-  if (thr) {
-    if (threadIdx.x == 0) thr[q] = k <= p2 ? s[k - 1] : YK_KEY_NONE;
-    return;
-  }
   for (int i = threadIdx.x; i < k; i += blockDim.x)
     yk_store_key(i < p2 ? s[i] : YK_KEY_NONE, out_i + q * k + i, out_d + q * k + i);
 }
 
-// After a MODE 3 pass: queries whose list fitted get their k smallest and
-// become inactive (thr = 0); overflowing queries get the k-th smallest
-// captured key as a tighter threshold, their count is reset, *flag is set.
-// A query with fewer than k keys under a bound (the estimated starting
-// bound, or with NaN distances, which no bound admits, any bound) gets no
-// bound, its count reset and the flag: its next pass admits every value
-// (and overflows, the overflow's bound then being a proven one); a query
-// with fewer than k keys and no bound has no more to find.
-__global__ __launch_bounds__(256) void yk_select_kernel(const uint64_t *__restrict__ cand,
+// The filtered pass's starting bounds, one wave per query: the m-th smallest
+// of the query's n <= 4096 sketch minima (YK_KEY_NONE, admit all, when fewer
+// than need of them are real keys); the query's candidate count and the
+// flag start at zero.
+__global__ __launch_bounds__(256) void yk_thr_kernel(const uint64_t *__restrict__ src, long nq,
+                                                     int n, int m, int need,
+                                                     uint64_t *__restrict__ thr,
+                                                     int *__restrict__ cnt, int *flag) {
+  const long q = blockIdx.x * 4L + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (q == 0 && lane == 0) *flag = 0;
+  if (q >= nq) return;
+  const uint64_t *p = src + q * (long)n;
+  uint64_t t = YK_KEY_NONE;
+  auto kth = [&](auto e) {
+    constexpr int E = decltype(e)::value;
+    uint64_t v[E];
+    yk_wave_load<E>(p, n, lane, v);
+    int nreal = 0;
+#pragma unroll
+    for (int i = 0; i < E; i++) nreal += __popcll(__builtin_amdgcn_ballot_w64(v[i] != YK_KEY_NONE));
+    if (nreal >= need) t = yk_wave_kth<E>(v, m, false);
+  };
+  if (n >= need) {
+    if (n <= 256)
+      kth(std::integral_constant<int, 4>());
+    else if (n <= 512)
+      kth(std::integral_constant<int, 8>());
+    else if (n <= 1024)
+      kth(std::integral_constant<int, 16>());
+    else if (n <= 2048)
+      kth(std::integral_constant<int, 32>());
+    else
+      kth(std::integral_constant<int, 64>());
+  }
+  if (lane == 0) {
+    thr[q] = t;
+    cnt[q] = 0;
+  }
+}
+
+template <int E, int E2>
+__device__ __forceinline__ void yk_cand_topk(const uint64_t *p, int m, int n, int k, int lane,
+                                             uint64_t *lds, int *oi, float *od, uint64_t *thr,
+                                             int *cnt, int *flag) {
+  uint64_t v[E];
+  yk_wave_load<E>(p, m, lane, v);
+  if (n > YK_CAND_CAP) {
+    const uint64_t x = yk_wave_kth<E>(v, k, false);
+    if (lane == 0) {
+      *thr = x;
+      *cnt = 0;
+      atomicOr(flag, 1);
+    }
+    return;
+  }
+  uint64_t w[E2];
+  yk_wave_topk_reg<E, E2>(v, k, lane, lds, w);
+#pragma unroll
+  for (int i = 0; i < E2; i++) {
+    const int e = lane * E2 + i;
+    if (e < k) yk_store_key(w[i], oi + e, od + e);
+  }
+  if (lane == 0) *thr = 0;
+}
+
+// After a MODE 3 pass, one wave per query (k <= 64 E2): queries whose list
+// fitted get their k smallest and become inactive (thr = 0); overflowing
+// queries get the k-th smallest captured key as a tighter threshold, their
+// count is reset, *flag is set.  A query with fewer than k keys under a bound
+// (the estimated starting bound, or with NaN distances, which no bound
+// admits, any bound) gets no bound, its count reset and the flag: its next
+// pass admits every value (and overflows, the overflow's bound then being a
+// proven one); a query with fewer than k keys and no bound has no more to
+// find.  (The keys are held in registers and the k-th found by ballot
+// counts, as in the precision form: 1e4 lists of ~700 keys, k = 100, 0.049
+// -> 0.012 ms against a workgroup's bitonic sort per query.)
+template <int E2>
+__global__ __launch_bounds__(256) void yk_select_kernel(const uint64_t *__restrict__ cand, long nq,
                                                         int *cnt, uint64_t *thr, int k,
                                                         int *out_i, float *out_d, int *flag) {
-  __shared__ uint64_t s[YK_CAND_CAP];
-  const long q = blockIdx.x;
-  if (thr[q] == 0) return;
+  __shared__ uint64_t lds[4][64 * E2];
+  const long q = blockIdx.x * 4L + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (q >= nq || thr[q] == 0) return;
   const int n = cnt[q];
   if (n < k && thr[q] != YK_KEY_NONE) {
-    if (threadIdx.x == 0) {
+    if (lane == 0) {
       thr[q] = YK_KEY_NONE;
       cnt[q] = 0;
       atomicOr(flag, 1);
@@ -600,24 +1163,19 @@ __global__ __launch_bounds__(256) void yk_select_kernel(const uint64_t *__restri
     return;
   }
   const int m = n < YK_CAND_CAP ? n : YK_CAND_CAP;
-  int p2 = 1;
-  while (p2 < m) p2 <<= 1;
   const uint64_t *p = cand + q * (long)YK_CAND_CAP;
-  for (int i = threadIdx.x; i < p2; i += blockDim.x) s[i] = i < m ? p[i] : YK_KEY_NONE;
-  __syncthreads();
-  yk_block_bitonic(s, p2);
-  if (n > YK_CAND_CAP) {
-    if (threadIdx.x == 0) {
-      thr[q] = s[k - 1];
-      cnt[q] = 0;
-      atomicOr(flag, 1);
-    }
-    return;
-  }
-  for (int i = threadIdx.x; i < k; i += blockDim.x)
-    yk_store_key(i < p2 ? s[i] : YK_KEY_NONE, out_i + q * k + i, out_d + q * k + i);
-  __syncthreads();
-  if (threadIdx.x == 0) thr[q] = 0;
+  int *oi = out_i + q * k;
+  float *od = out_d + q * k;
+  if (m <= 256)
+    yk_cand_topk<4, E2>(p, m, n, k, lane, lds[wave], oi, od, thr + q, cnt + q, flag);
+  else if (m <= 512)
+    yk_cand_topk<8, E2>(p, m, n, k, lane, lds[wave], oi, od, thr + q, cnt + q, flag);
+  else if (m <= 1024)
+    yk_cand_topk<16, E2>(p, m, n, k, lane, lds[wave], oi, od, thr + q, cnt + q, flag);
+  else if (m <= 2048)
+    yk_cand_topk<32, E2>(p, m, n, k, lane, lds[wave], oi, od, thr + q, cnt + q, flag);
+  else
+    yk_cand_topk<64, E2>(p, m, n, k, lane, lds[wave], oi, od, thr + q, cnt + q, flag);
 }
 
 __global__ void yk_zero_cnt_kernel(int *cnt, long n) {
@@ -628,13 +1186,24 @@ __global__ void yk_zero_cnt_kernel(int *cnt, long n) {
 // ---------------------------------------------------------------------------
 // planning and launch
 
+// Which scan a search takes.  Up to 64 queries a pass over the base is bound
+// by its bytes, and a wave streams rows straight to registers (YK_STREAM; one
+// or two waves per workgroup, so that every wave has queries of its own);
+// beyond that the workgroup shares the base through LDS (YK_LDS1: 32 queries
+// per wave, YK_LDS2: 64).  d > 256 streams both operands.
+enum { YK_STREAM = 0, YK_LDS1 = 1, YK_LDS2 = 2 };
+#define YK_STREAM_NQ 64
+
 struct YkPlan {
-  int nblk;    // query blocks of 32 per wave (NB)
+  int kind;
   int waves;   // waves per workgroup
   int tiles;   // query tiles
   int nsplit;  // base splits
   long brange;
   long bstep;
+  int inter;   // sketch: interleaved splits
+  int slots;   // workgroups resident at once
+  int units;   // k = 1: even shares of tiles x units blocks over `slots` workgroups
 };
 
 // Launch-plan knobs the autotuner chooses among (every choice gives the
@@ -645,43 +1214,157 @@ static const long yk_item_targets[3] = {4096, 2048, 8192};
 static const int yk_stride_scale[4][2] = {{1, 1}, {1, 2}, {2, 1}, {16, 3}};  // num., denom.
 #define YK_NCFG 12
 
-// Split the base so that tiles * nsplit reaches the item target (~8 per
-// resident workgroup by default), with at least min_rows rows per split and
-// at most max_split splits.
-static YkPlan yk_plan(long nq, long nb, long sample, long min_splits, long max_split,
-                      int cfg = 0) {
-  YkPlan p;
-  p.nblk = 1;
-  p.waves = 4;
-  const long qt = 32L * p.nblk * p.waves;
-  p.tiles = (int)((nq + qt - 1) / qt);
+typedef void (*YkScanKernel)(ScanArgs);
+
+// the streaming kernel with exactly ld/16 register-resident chunks (ld <=
+// 128), else the one streaming both operands
+template <int MODE, int R>
+static YkScanKernel yk_stream_pick(int ld, bool weighted) {
+  if (weighted && ld <= 32) return yk_scan_f32<1, 0, MODE, R>;  // no weights in NCH <= 2
+  switch (ld >> 4) {
+    case 1: return yk_scan_f32<1, 1, MODE, R>;
+    case 2: return yk_scan_f32<1, 2, MODE, R>;
+    case 3: return yk_scan_f32<1, 3, MODE, R>;
+    case 4: return yk_scan_f32<1, 4, MODE, R>;
+    case 5: return yk_scan_f32<1, 5, MODE, R>;
+    case 6: return yk_scan_f32<1, 6, MODE, R>;
+    case 7: return yk_scan_f32<1, 7, MODE, R>;
+    case 8: return yk_scan_f32<1, 8, MODE, R>;
+    default: return yk_scan_f32<1, 0, MODE, R>;
+  }
+}
+
+template <int MODE, bool WT>
+static YkScanKernel yk_lds_pick(int kind, int ld) {
+  if (kind == YK_LDS2) {
+    switch (ld >> 4) {
+      case 1: return yk_scan_f32_lds<2, 1, MODE, WT>;
+      case 2: return yk_scan_f32_lds<2, 2, MODE, WT>;
+      case 3: return yk_scan_f32_lds<2, 3, MODE, WT>;
+      case 4: return yk_scan_f32_lds<2, 4, MODE, WT>;
+      case 5: return yk_scan_f32_lds<2, 5, MODE, WT>;
+      case 6: return yk_scan_f32_lds<2, 6, MODE, WT>;
+      case 7: return yk_scan_f32_lds<2, 7, MODE, WT>;
+      default: return yk_scan_f32_lds<2, 8, MODE, WT>;
+    }
+  }
+  switch (ld >> 4) {
+    case 1: return yk_scan_f32_lds<1, 1, MODE, WT>;
+    case 2: return yk_scan_f32_lds<1, 2, MODE, WT>;
+    case 3: return yk_scan_f32_lds<1, 3, MODE, WT>;
+    case 4: return yk_scan_f32_lds<1, 4, MODE, WT>;
+    case 5: return yk_scan_f32_lds<1, 5, MODE, WT>;
+    case 6: return yk_scan_f32_lds<1, 6, MODE, WT>;
+    case 7: return yk_scan_f32_lds<1, 7, MODE, WT>;
+    case 8: return yk_scan_f32_lds<1, 8, MODE, WT>;
+    case 9: return yk_scan_f32_lds<1, 9, MODE, WT>;
+    case 10: return yk_scan_f32_lds<1, 10, MODE, WT>;
+    case 11: return yk_scan_f32_lds<1, 11, MODE, WT>;
+    case 12: return yk_scan_f32_lds<1, 12, MODE, WT>;
+    case 13: return yk_scan_f32_lds<1, 13, MODE, WT>;
+    case 14: return yk_scan_f32_lds<1, 14, MODE, WT>;
+    case 15: return yk_scan_f32_lds<1, 15, MODE, WT>;
+    default: return yk_scan_f32_lds<1, 16, MODE, WT>;
+  }
+}
+
+static YkScanKernel yk_scan_pick(int mode, int kind, int ld, bool weighted) {
+  if (kind != YK_STREAM && weighted)
+    return mode == 0   ? yk_lds_pick<0, true>(kind, ld)
+           : mode == 1 ? yk_lds_pick<1, true>(kind, ld)
+                       : yk_lds_pick<3, true>(kind, ld);
+  if (kind != YK_STREAM)
+    return mode == 0   ? yk_lds_pick<0, false>(kind, ld)
+           : mode == 1 ? yk_lds_pick<1, false>(kind, ld)
+                       : yk_lds_pick<3, false>(kind, ld);
+  return mode == 0   ? yk_stream_pick<0, 1>(ld, weighted)
+         : mode == 1 ? yk_stream_pick<1, 1>(ld, weighted)
+         : mode == 2 ? yk_stream_pick<2, YK_REG_R>(ld, weighted)
+                     : yk_stream_pick<3, 1>(ld, weighted);
+}
+
+// blocks a stage of the LDS-staged kernel holds (YkLdsShape::G)
+static long yk_lds_stage_blocks(int ld) { return ld <= 16 ? 8 : ld <= 32 ? 4 : ld <= 64 ? 2 : 1; }
+
+// The plan of one scan: mode 0 (k = 1), 1 (the sketch, one block in `sample`),
+// 2 (register top-R) or 3 (filtered).
+static YkPlan yk_plan(int mode, long nq, long nb, int ld, bool weighted, long sample,
+                      long min_splits, long max_split, long min_blocks, int cfg) {
+  YkPlan p = {};
   p.bstep = 32 * sample;
   const long nblocks = (nb + p.bstep - 1) / p.bstep;  // processed blocks
-  // ~8 work items per resident workgroup (512 of them: 256 CUs x 2) keeps
-  // the tail of the persistent grid short
-  const long target = yk_item_targets[cfg % 3];
-  long want = (target + p.tiles - 1) / p.tiles;
-  long maxs = (nblocks + 15) / 16;  // >= 16 processed blocks per split
+  p.kind = YK_STREAM;
+  p.waves = 4;
+  if (mode != 2 && ld <= 256 && (nq > YK_STREAM_NQ || ld > 128)) {
+    // two query tiles per wave where the chip still has work for every wave
+    p.kind = ld <= 128 && nq > 128 && (nq + 255) / 256 * nblocks >= 2048 ? YK_LDS2 : YK_LDS1;
+  } else if (mode != 2 && nq <= YK_STREAM_NQ) {
+    p.waves = nq <= 32 ? 1 : 2;
+  }
+  const long qt = (p.kind == YK_LDS2 ? 64 : 32) * p.waves;
+  p.tiles = (int)((nq + qt - 1) / qt);
+  p.slots = yk_resident_wgs((const void *)yk_scan_pick(mode, p.kind, ld, weighted), 64 * p.waves);
+  if (mode == 0 && p.kind != YK_STREAM && nb * ld <= (1L << 19) && nblocks >= 8) {
+    // k = 1 over a base of at most 2 MB, which every XCD's L2 holds (the
+    // k-means assign): even shares of the (tile, block) pairs, so that no CU
+    // waits for a last round of whole tiles (n = 1e5 points are 391 tiles for
+    // 512 workgroups).  Fewer than 8 blocks make a tile too short for the
+    // merge's launch to pay.
+    p.units = (int)nblocks;
+    p.nsplit = 1;
+    p.brange = nblocks * p.bstep;
+    const long T = (long)p.tiles * p.units;
+    if (T < p.slots) p.slots = (int)T;
+    return p;
+  }
+  // ~8 work items per resident workgroup keeps the tail of the persistent
+  // grid short, of at least min_blocks processed blocks each
+  long want = (yk_item_targets[cfg % 3] + p.tiles - 1) / p.tiles;
+  long maxs = (nblocks + min_blocks - 1) / min_blocks;
   if (want > maxs) want = maxs;
+  if ((mode == 0 || mode == 3) && p.tiles * nblocks < 96L * p.slots) {
+    // few blocks per workgroup: of the splits that fill r rounds of the
+    // resident workgroups, the one whose rounds take least (a round is a
+    // split's blocks, and ~3 more for its queries and its end)
+    long best = -1;
+    for (long r = 1; r <= 16; r++) {
+      const long s = min(nblocks, r * p.slots / p.tiles);
+      if (s < 1) continue;
+      const long per = (nblocks + s - 1) / s, n = (nblocks + per - 1) / per;
+      const long cost = (p.tiles * n + p.slots - 1) / p.slots * (per + 3);
+      if (best < 0 || cost < best) {
+        best = cost;
+        want = n;
+      }
+    }
+  }
   if (want < min_splits) want = min_splits;
   if (want > max_split) want = max_split;
   if (want > nblocks) want = nblocks;
   if (want < 1) want = 1;
   long per = (nblocks + want - 1) / want;  // processed blocks per split
-  // an item's rows stay within 2^30 bytes (buffer-load offsets are 32-bit)
-  const long max_per = (1L << 30) / (32L * 128 * 4 * sample);
+  // an item's rows stay within 2^30 bytes (the streaming kernel's buffer
+  // offsets are 32-bit)
+  const long max_per = (1L << 30) / (32L * (ld > 128 ? ld : 128) * 4 * sample);
   if (per > max_per) per = max_per;
   p.brange = per * p.bstep;
   p.nsplit = (int)((nb + p.brange - 1) / p.brange);
+  // interleaved sketch splits where the byte offsets of a split's walk (or
+  // of a stage's blocks) fit 31 bits
+  if (mode == 1) {
+    const long span = p.kind == YK_STREAM
+                          ? nb * ld * 4
+                          : (yk_lds_stage_blocks(ld) - 1) * p.bstep * p.nsplit * ld * 4 + 32L * ld * 4;
+    p.inter = span < 0x7fffffffL;
+  }
   return p;
 }
 
 extern "C" int yk_knn_plan(long nq, long nb, int d, int k, int *nsplit, int *waves, int *nblk) {
-  (void)d;
-  YkPlan p = yk_plan(nq, nb, 1, 1, k > 1 ? 256 : 4096);
+  const YkPlan p = yk_plan(k > 1 ? 3 : 0, nq, nb, yk_ld(d), false, 1, 1, 4096, 16, 0);
   *nsplit = p.nsplit;
   *waves = p.waves;
-  *nblk = p.nblk;
+  *nblk = p.kind == YK_LDS2 ? 2 : 1;
   return YK_OK;
 }
 
@@ -723,65 +1406,67 @@ static int yk_scratch(YkArena *ar, int slot, size_t bytes, void **out) {
   return YK_OK;
 }
 
-// the kernel with exactly ld/16 register-resident chunks (ld <= 128), else
-// the one streaming both operands
-template <int MODE, int R>
-static void (*yk_f32_pick(int ld, bool weighted))(ScanArgs) {
-  if (weighted && ld <= 32) return yk_scan_f32<1, 0, MODE, R>;  // no weights in NCH <= 2
-  switch (ld >> 4) {
-    case 1: return yk_scan_f32<1, 1, MODE, R>;
-    case 2: return yk_scan_f32<1, 2, MODE, R>;
-    case 3: return yk_scan_f32<1, 3, MODE, R>;
-    case 4: return yk_scan_f32<1, 4, MODE, R>;
-    case 5: return yk_scan_f32<1, 5, MODE, R>;
-    case 6: return yk_scan_f32<1, 6, MODE, R>;
-    case 7: return yk_scan_f32<1, 7, MODE, R>;
-    case 8: return yk_scan_f32<1, 8, MODE, R>;
-    default: return yk_scan_f32<1, 0, MODE, R>;
-  }
-}
-
-template <int MODE, int R>
-static int yk_launch_scan(const YkPlan &p, ScanArgs a, bool qres) {
+static int yk_launch_scan(int mode, const YkPlan &p, ScanArgs a) {
   a.brange = p.brange;
   a.bstep = p.bstep;
   a.nsplit = p.nsplit;
+  a.inter = p.inter;
+  a.units = p.units;
   a.tiles_x = p.tiles;
   a.total = p.tiles * p.nsplit;
   a.per_xcd = (a.total + 7) / 8;
-  (void)qres;
-  auto kern = yk_f32_pick<MODE, R>(a.ld, a.w != nullptr);
-  YK_TRY(yk_item_tickets(&a.tick));
-  const int per_xcd_res = yk_resident_wgs((const void *)kern, 64 * p.waves) / 8;
+  YkScanKernel kern = yk_scan_pick(mode, p.kind, a.ld, a.w != nullptr);
+  const int per_xcd_res = p.slots / 8;
   dim3 grid(8 * (a.per_xcd < per_xcd_res ? a.per_xcd : per_xcd_res)), block(64 * p.waves);
-  int tok = yk_prof_begin(MODE == 1 ? YK_PROF_F32_SKETCH : YK_PROF_FUSED);
+  a.tick = nullptr;
+  if (p.units)
+    grid.x = p.slots;
+  else if (a.per_xcd > per_xcd_res)  // more items than resident workgroups
+    YK_TRY(yk_item_tickets(&a.tick));
+  int tok = yk_prof_begin(mode == 1 ? YK_PROF_F32_SKETCH : YK_PROF_FUSED);
   hipLaunchKernelGGL(kern, grid, block, 0, yk_stream(), a);
   yk_prof_end(tok);
   YK_HIP(hipGetLastError());
   return YK_OK;
 }
 
-static int yk_sortsel(const uint64_t *src, long nq, int n, int k, int *oi, float *od,
-                      uint64_t *thr) {
-  int p2 = 1;
-  while (p2 < n) p2 <<= 1;
+// the m-th smallest of the sketch's n minima per query -> thr
+static int yk_thr(const uint64_t *src, long nq, int n, int m, int need, uint64_t *thr, int *cnt,
+                  int *flag) {
+  if (n > 4096) return yk_set_error(YK_EINVAL, "sketch of %d minima per query", n);
   int tok = yk_prof_begin(YK_PROF_MERGE);
-  hipLaunchKernelGGL(yk_sortsel_kernel, dim3((unsigned)nq), dim3(256), sizeof(uint64_t) * p2,
-                     yk_stream(), src, n, k, p2, oi, od, thr);
+  hipLaunchKernelGGL(yk_thr_kernel, dim3((unsigned)((nq + 3) / 4)), dim3(256), 0, yk_stream(), src,
+                     nq, n, m, need, thr, cnt, flag);
   yk_prof_end(tok);
   YK_HIP(hipGetLastError());
   return YK_OK;
 }
 
-// Sketch stride of the k > 16 path: every lane's minimum over its rows of
-// a 1-in-stride sample of base blocks, with >= k splits -> >= 2k distinct
+static int yk_select(const ScanArgs &a, uint64_t *thr, int k, int *assign, float *dis, int *flag) {
+  const dim3 grid((unsigned)((a.nq + 3) / 4)), block(256);
+  int tok = yk_prof_begin(YK_PROF_MERGE);
+  auto kern = k <= 64    ? yk_select_kernel<1>
+              : k <= 256 ? yk_select_kernel<4>
+              : k <= 512 ? yk_select_kernel<8>
+                         : yk_select_kernel<16>;
+  hipLaunchKernelGGL(kern, grid, block, 0, yk_stream(), a.cand, a.nq, a.cnt, thr, k, assign, dis,
+                     flag);
+  yk_prof_end(tok);
+  YK_HIP(hipGetLastError());
+  return YK_OK;
+}
+
+// Sketch stride of the filtered search: every lane's minimum over its rows
+// of a 1-in-stride sample of base blocks, with >= k splits -> >= 2k distinct
 // real keys per query.  The k-th smallest of 2k subset minima sits near
 // global rank 1.4 * stride * k, the expected candidate count; ~800 keeps
-// the filtered pass's append path rare and the list far from overflow.
+// the filtered pass's append path rare and the list far from overflow.  For
+// k <= 16, whose bound is always the proven k-th minimum, 1 in 16 (about
+// 360 candidates at k = 16).
 static long yk_sketch_stride(long nb, int k, int cfg = 0) {
   const int *sc = yk_stride_scale[(cfg / 3) % 4];
   long stride = 600L * sc[0] / sc[1] / k;
-  const long cap = sc[0] == 16 ? 16 : 8;  // the last scale may sample 1 in 16
+  const long cap = sc[0] == 16 || k <= YK_REG_R ? 16 : 8;  // the last scale may sample 1 in 16
   if (stride > cap) stride = cap;
   if (stride < 1) stride = 1;
   const long nblocks = (nb + 31) / 32;
@@ -789,16 +1474,35 @@ static long yk_sketch_stride(long nb, int k, int cfg = 0) {
   return stride;
 }
 
-// queries per pass of the k > 16 path (bounds the candidate memory)
-#define YK_LARGE_K_QB 16384L
+// the sketch's plan
+static YkPlan yk_sketch_plan(long nq, long nb, int ld, bool weighted, int k, int cfg) {
+  const long stride = yk_sketch_stride(nb, k, cfg);
+  if (k <= YK_REG_R)  // more, smaller subsets: a tighter bound
+    return yk_plan(1, nq, nb, ld, weighted, stride, 2 * k, 512, 4, cfg);
+  return yk_plan(1, nq, nb, ld, weighted, stride, k, k > 256 ? k : 256, 16, cfg);
+}
 
-// k > 16: sketch threshold, filtered scan, per-query sort (queries in batches
-// that bound the candidate memory).
-static int yk_knn_large_k(ScanArgs base, int k, bool qres, int *assign, float *dis,
-                          YkArena *ar, int cfg) {
+// queries per pass of the filtered search (bounds the candidate memory)
+#define YK_LARGE_K_QB 16384L
+// splits of the register top-R scan behind it (k <= 16)
+#define YK_FALLBACK_SPLITS 16
+
+// k > 1: sketch threshold, filtered scan, per-query select (queries in
+// batches that bound the candidate memory).  k > 16 starts from an estimated
+// bound and reads back a flag: queries that overflowed their list or were
+// left short are scanned again.  For k <= 16 the bound is the proven k-th
+// minimum, so only an overflow (thousands of rows within the bound: ties, or
+// near rows concentrated between the sampled blocks) leaves a query over,
+// and nothing is read back: the register top-16 scan is queued behind, each
+// of its workgroups leaving at once unless the flag is set.  (That scan alone
+// -- an exact FP64-normed value and a list test for every pair -- took 0.97
+// of 1.34 ms for 1,003 queries x 100,003 vectors, d = 100, k = 10, with the
+// sort of its lists 0.36 ms.)
+static int yk_knn_filtered(ScanArgs base, int k, int *assign, float *dis, YkArena *ar, int cfg) {
   const long QB = YK_LARGE_K_QB;
   const long nq_all = base.nq;
-  void *vthr, *vcnt, *vcand, *vpart, *vflag;
+  const bool small = k <= YK_REG_R, weighted = base.w != nullptr;
+  void *vthr, *vcnt, *vcand, *vpart;
   const long qb = nq_all < QB ? nq_all : QB;
   YK_TRY(yk_scratch(ar, 0, sizeof(uint64_t) * qb, &vthr));
   YK_TRY(yk_scratch(ar, 1, sizeof(int) * (qb + 64), &vcnt));
@@ -807,9 +1511,7 @@ static int yk_knn_large_k(ScanArgs base, int k, bool qres, int *assign, float *d
   uint64_t *thr = (uint64_t *)vthr;
   int *cnt = (int *)vcnt;
   int *flag = cnt + qb + 32;
-  vflag = flag;
   const long stride = yk_sketch_stride(base.nb, k, cfg);
-  const long min_splits = k;
 
   for (long q0 = 0; q0 < nq_all; q0 += QB) {
     const long nq = nq_all - q0 < QB ? nq_all - q0 : QB;
@@ -818,32 +1520,41 @@ static int yk_knn_large_k(ScanArgs base, int k, bool qres, int *assign, float *d
     a.qn = base.qn ? base.qn + q0 : nullptr;
     a.nq = nq;
     // (A) sketch: per-lane minima over a strided sample
-    YkPlan pa = yk_plan(nq, a.nb, stride, min_splits, min_splits > 256 ? min_splits : 256, cfg);
+    const YkPlan pa = yk_sketch_plan(nq, a.nb, a.ld, weighted, k, cfg);
+    const YkPlan pc = yk_plan(2, nq, a.nb, a.ld, weighted, 1, 1, YK_FALLBACK_SPLITS, 16, 0);
+    const size_t bytes_a = sizeof(uint64_t) * nq * pa.nsplit * 2;
+    const size_t bytes_c = small ? sizeof(uint64_t) * nq * pc.nsplit * 2 * YK_REG_R : 0;
     if (ar) ar->used = fixed_used;  // each pass reuses the region's partial-key piece
-    YK_TRY(yk_scratch(ar, 3, sizeof(uint64_t) * nq * pa.nsplit * 2, &vpart));
+    YK_TRY(yk_scratch(ar, 3, bytes_a > bytes_c ? bytes_a : bytes_c, &vpart));
     a.part = (uint64_t *)vpart;
-    YK_TRY((yk_launch_scan<1, 1>(pa, a, qres)));
-    // the starting bound: the m-th smallest minimum (yk_bound_rank)
-    YK_TRY(yk_sortsel(a.part, nq, pa.nsplit * 2, yk_bound_rank(k, stride), nullptr, nullptr,
-                      thr));
-    // (B) filtered scan + per-query sort, retried for overflowing queries
-    YkPlan pb = yk_plan(nq, a.nb, 1, 1, 4096, cfg);
+    YK_TRY(yk_launch_scan(1, pa, a));
+    // the starting bound: the k-th smallest minimum, or for k > 16 the m-th
+    // (yk_bound_rank)
+    const int m = small ? k : yk_bound_rank(k, stride);
+    YK_TRY(yk_thr(a.part, nq, pa.nsplit * 2, m, m, thr, cnt, flag));
+    // (B) filtered scan + per-query select
+    const YkPlan pb = yk_plan(3, nq, a.nb, a.ld, weighted, 1, 1, 4096, 16, cfg);
     a.thr = thr;
     a.cnt = cnt;
     a.cand = (uint64_t *)vcand;
-    hipLaunchKernelGGL(yk_zero_cnt_kernel, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0,
-                       yk_stream(), cnt, nq);
-    hipLaunchKernelGGL(yk_zero_cnt_kernel, dim3(1), dim3(64), 0, yk_stream(), flag, 1L);
     int tries = 0;
     for (;;) {
-      YK_TRY((yk_launch_scan<3, 1>(pb, a, qres)));
-      int tok = yk_prof_begin(YK_PROF_MERGE);
-      hipLaunchKernelGGL(yk_select_kernel, dim3((unsigned)nq), dim3(256), 0, yk_stream(), a.cand,
-                         cnt, thr, k, assign + q0 * k, dis + q0 * k, flag);
-      yk_prof_end(tok);
-      YK_HIP(hipGetLastError());
+      YK_TRY(yk_launch_scan(3, pb, a));
+      YK_TRY(yk_select(a, thr, k, assign + q0 * k, dis + q0 * k, flag));
+      if (small) {  // (C) what is left, if anything
+        a.flag = flag;
+        YK_TRY(yk_launch_scan(2, pc, a));
+        const int n = pc.nsplit * 2 * YK_REG_R;
+        int p2 = 1;
+        while (p2 < n) p2 <<= 1;
+        hipLaunchKernelGGL(yk_sortsel_kernel, dim3((unsigned)nq), dim3(256), sizeof(uint64_t) * p2,
+                           yk_stream(), a.part, n, k, p2, assign + q0 * k, dis + q0 * k, thr,
+                           flag);
+        YK_HIP(hipGetLastError());
+        break;
+      }
       int hflag = 0;
-      YK_TRY(yk_read_small(&hflag, vflag, sizeof(int)));
+      YK_TRY(yk_read_small(&hflag, flag, sizeof(int)));
       if (!hflag) break;
       if (++tries == 6)
         return yk_set_error(YK_EINVAL,
@@ -887,33 +1598,30 @@ static int yk_knn_f32_run(int type, long nq, long nb, int d, int k, const float 
   a.type = type;
   a.out_i = assign;
   a.out_d = dis;
-  const bool qres = a.ld <= 128;
-  if (k == 1) {
-    YkPlan p = yk_plan(nq, nb, 1, 1, 4096, cfg);
-    if (p.nsplit > 1) {
-      void *buf;
-      YK_TRY(yk_scratch(ar, 3, sizeof(uint64_t) * nq * p.nsplit, &buf));
-      a.part = (uint64_t *)buf;
-    }
-    YK_TRY((yk_launch_scan<0, 1>(p, a, qres)));
-    if (p.nsplit > 1) {
-      int tok = yk_prof_begin(YK_PROF_MERGE);
-      hipLaunchKernelGGL(yk_merge1_kernel, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0,
-                         yk_stream(), a.part, nq, p.nsplit, assign, dis);
-      yk_prof_end(tok);
-      YK_HIP(hipGetLastError());
-    }
-    return YK_OK;
-  }
-  if (k <= YK_REG_R) {
-    YkPlan p = yk_plan(nq, nb, 1, 1, 256, cfg);
+  if (k > 1) return yk_knn_filtered(a, k, assign, dis, ar, cfg);
+  const YkPlan p = yk_plan(0, nq, nb, a.ld, w != nullptr, 1, 1, 4096, 16, cfg);
+  const long tq = p.kind == YK_LDS2 ? 256 : 128;
+  if (p.nsplit > 1 || p.units) {
     void *buf;
-    YK_TRY(yk_scratch(ar, 3, sizeof(uint64_t) * nq * p.nsplit * 2 * YK_REG_R, &buf));
+    YK_TRY(yk_scratch(ar, 3, sizeof(uint64_t) * (p.units ? 2 * tq * p.slots : nq * p.nsplit), &buf));
     a.part = (uint64_t *)buf;
-    YK_TRY((yk_launch_scan<2, YK_REG_R>(p, a, qres)));
-    return yk_sortsel(a.part, nq, p.nsplit * 2 * YK_REG_R, k, assign, dis, nullptr);
   }
-  return yk_knn_large_k(a, k, qres, assign, dis, ar, cfg);
+  YK_TRY(yk_launch_scan(0, p, a));
+  if (p.units) {
+    int tok = yk_prof_begin(YK_PROF_MERGE);
+    hipLaunchKernelGGL(yk_merge_share_kernel, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0,
+                       yk_stream(), a.part, nq, (int)tq, (long)p.units,
+                       (long)p.tiles * p.units, (long)p.slots, assign, dis);
+    yk_prof_end(tok);
+    YK_HIP(hipGetLastError());
+  } else if (p.nsplit > 1) {
+    int tok = yk_prof_begin(YK_PROF_MERGE);
+    hipLaunchKernelGGL(yk_merge1_kernel, dim3((unsigned)((nq + 3) / 4)), dim3(256), 0, yk_stream(),
+                       a.part, nq, p.nsplit, assign, dis);
+    yk_prof_end(tok);
+    YK_HIP(hipGetLastError());
+  }
+  return YK_OK;
 }
 
 // a search through yk_time_ms
@@ -957,7 +1665,7 @@ static int yk_f32_plan(const YkF32Call &call, int *cfg, int *ran) {
   if ((double)call.nq * call.nb * call.d < (double)(1 << 29)) return YK_OK;
   const int kc = call.k == 1 ? 1 : call.k <= YK_REG_R ? 16 : 1 << yk_lg(call.k);
   char key[128];
-  snprintf(key, sizeof key, "f32:t%d:k%d:ld%d:q%d:b%d", call.type, kc, yk_ld(call.d),
+  snprintf(key, sizeof key, "f32:v2:t%d:k%d:ld%d:q%d:b%d", call.type, kc, yk_ld(call.d),
            yk_lg(call.nq), yk_lg(call.nb));
   if (yk_tune_get(key, cfg)) {
     if (*cfg < 0 || *cfg >= YK_NCFG) *cfg = 0;
@@ -969,19 +1677,17 @@ static int yk_f32_plan(const YkF32Call &call, int *cfg, int *ran) {
   long sig[YK_NCFG][3];
   int distinct = 0;
   bool dup[YK_NCFG] = {};
+  const int ld = yk_ld(call.d);
+  const bool weighted = call.w != nullptr;
   for (int i = 0; i < ncand; i++) {
     const long nqb = call.nq < YK_LARGE_K_QB ? call.nq : YK_LARGE_K_QB;
     if (call.k == 1) {
-      const YkPlan p = yk_plan(call.nq, call.nb, 1, 1, 4096, i);
-      sig[i][0] = p.nsplit, sig[i][1] = p.brange, sig[i][2] = 0;
-    } else if (call.k <= YK_REG_R) {
-      const YkPlan p = yk_plan(call.nq, call.nb, 1, 1, 256, i);
+      const YkPlan p = yk_plan(0, call.nq, call.nb, ld, weighted, 1, 1, 4096, 16, i);
       sig[i][0] = p.nsplit, sig[i][1] = p.brange, sig[i][2] = 0;
     } else {
-      const long st = yk_sketch_stride(call.nb, call.k, i);
-      const YkPlan pa = yk_plan(nqb, call.nb, st, call.k, call.k > 256 ? call.k : 256, i);
-      const YkPlan pb = yk_plan(nqb, call.nb, 1, 1, 4096, i);
-      sig[i][0] = st, sig[i][1] = pa.nsplit, sig[i][2] = pb.nsplit;
+      const YkPlan pa = yk_sketch_plan(nqb, call.nb, ld, weighted, call.k, i);
+      const YkPlan pb = yk_plan(3, nqb, call.nb, ld, weighted, 1, 1, 4096, 16, i);
+      sig[i][0] = pa.bstep, sig[i][1] = pa.nsplit, sig[i][2] = pb.nsplit;
     }
     for (int j = 0; j < i && !dup[i]; j++)
       dup[i] = !dup[j] && sig[j][0] == sig[i][0] && sig[j][1] == sig[i][1] &&
@@ -1061,21 +1767,20 @@ static int yk_noalloc_region(char **out) {
 
 // Scratch bytes one yk_knn_f32_run over nq queries takes from a region (the
 // same plans and pieces as the run itself, each rounded up to 256 bytes).
-static size_t yk_knn_f32_need(long nq, long nb, int k) {
+static size_t yk_knn_f32_need(long nq, long nb, int ld, bool weighted, int k) {
   if (k == 1) {
-    const YkPlan p = yk_plan(nq, nb, 1, 1, 4096);
+    const YkPlan p = yk_plan(0, nq, nb, ld, weighted, 1, 1, 4096, 16, 0);
+    if (p.units) return yk_align256(sizeof(uint64_t) * 2 * (p.kind == YK_LDS2 ? 256 : 128) * p.slots);
     return p.nsplit > 1 ? yk_align256(sizeof(uint64_t) * nq * p.nsplit) : 0;
   }
-  if (k <= YK_REG_R) {
-    const YkPlan p = yk_plan(nq, nb, 1, 1, 256);
-    return yk_align256(sizeof(uint64_t) * nq * p.nsplit * 2 * YK_REG_R);
-  }
   const long qb = nq < YK_LARGE_K_QB ? nq : YK_LARGE_K_QB;
-  const long stride = yk_sketch_stride(nb, k);
-  const YkPlan pa = yk_plan(qb, nb, stride, k, k > 256 ? k : 256);
+  const YkPlan pa = yk_sketch_plan(qb, nb, ld, weighted, k, 0);
+  const YkPlan pc = yk_plan(2, qb, nb, ld, weighted, 1, 1, YK_FALLBACK_SPLITS, 16, 0);
+  const size_t bytes_a = sizeof(uint64_t) * qb * pa.nsplit * 2;
+  const size_t bytes_c = k <= YK_REG_R ? sizeof(uint64_t) * qb * pc.nsplit * 2 * YK_REG_R : 0;
   return yk_align256(sizeof(uint64_t) * qb) + yk_align256(sizeof(int) * (qb + 64)) +
          yk_align256(sizeof(uint64_t) * qb * YK_CAND_CAP) +
-         yk_align256(sizeof(uint64_t) * qb * pa.nsplit * 2);
+         yk_align256(bytes_a > bytes_c ? bytes_a : bytes_c);
 }
 
 extern "C" int yk_knn_f32_noalloc(int type, long nq, long nb, int d, int k, const float *q,
@@ -1092,15 +1797,16 @@ extern "C" int yk_knn_f32_noalloc(int type, long nq, long nb, int d, int k, cons
   // query's result depends only on that query, so the passes give the
   // single call's results.
   long pass = 16384;
-  while (pass > 32 && yk_knn_f32_need(pass < nq ? pass : nq, nb, k) > YK_NOALLOC_SCRATCH_BYTES)
+  const int ld = yk_ld(d);
+  while (pass > 32 && yk_knn_f32_need(pass < nq ? pass : nq, nb, ld, w != nullptr, k) >
+                          YK_NOALLOC_SCRATCH_BYTES)
     pass >>= 1;
-  const size_t need = yk_knn_f32_need(pass < nq ? pass : nq, nb, k);
+  const size_t need = yk_knn_f32_need(pass < nq ? pass : nq, nb, ld, w != nullptr, k);
   if (need > YK_NOALLOC_SCRATCH_BYTES)
     return yk_set_error(YK_EINVAL,
                         "k=%d, nb=%ld needs %zu scratch bytes even for %ld queries at a time; "
                         "the no-allocation search holds %zu",
                         k, nb, need, pass, (size_t)YK_NOALLOC_SCRATCH_BYTES);
-  const int ld = yk_ld(d);
   for (long q0 = 0; q0 < nq; q0 += pass) {
     const long n = nq - q0 < pass ? nq - q0 : pass;
     YkArena ar = {region, (size_t)YK_NOALLOC_SCRATCH_BYTES, 0};
@@ -1241,14 +1947,15 @@ yk_bassign_res_kernel(BassignArgs a) {
       int bi = -1;
 #pragma unroll
       for (int cb = 0; cb < NBLK; cb++) {
-        float nn[16];
+        YkNormRegs nrm;
+        float (&nn)[16] = nrm.n;
 #pragma unroll
         for (int g = 0; g < 4; g++) {
           const float4 n4 = nns[(cb * 4 + g) * 64 + lane];
           nn[4 * g] = n4.x; nn[4 * g + 1] = n4.y; nn[4 * g + 2] = n4.z; nn[4 * g + 3] = n4.w;
         }
         if (32 * cb + 32 <= a.kc) {
-          yk_best1_block<false>(acc[cb], nn, qd, 32L * cb, h, false, bv, bi);
+          yk_best1_block<false>(acc[cb], nrm, qd, 32L * cb, h, false, bv, bi);
         } else {
 #pragma unroll
           for (int i = 0; i < 16; i++) {
@@ -1394,7 +2101,8 @@ int yk_batch_assign_idx(long nitems, const int *item_inst, const int *item_tile,
   a.qidx = qidx;
   a.total = (int)nitems;
   a.per_xcd = (a.total + 7) / 8;
-  auto kern = yk_f32_pick<0, 1>(a.ld, false);
+  // (the points are the kernel's queries: 128 per item, four waves)
+  auto kern = yk_scan_pick(0, a.ld <= 256 ? YK_LDS1 : YK_STREAM, a.ld, false);
   YK_TRY(yk_item_tickets(&a.tick));
   const int per_res = yk_resident_wgs((const void *)kern, 256) / 8;
   dim3 grid(8 * (a.per_xcd < per_res ? a.per_xcd : per_res)), block(256);

@@ -29,3 +29,21 @@ def test_upload_roundtrip(ya, n, d):
     ya.check(ya.lib().yk_download_vectors(back.ctypes.data, V.vec.ptr, n, d), "download")
     V.free()
     assert np.array_equal(back.view(np.uint32), x.view(np.uint32))
+
+
+@pytest.mark.parametrize("n,d", [(1, 1), (5, 3), (2055, 157), (3, 1000), (409601, 41), (120000, 48)])
+def test_copies_roundtrip_and_pad_columns(ya, n, d):
+    """Rows spread to and collected from the padded layout (one dense piece,
+    and 67 MB in two), and an unpadded set of 23 MB read back in slices: every
+    byte comes back and the pad columns are zero."""
+    from yael_amd import device
+    rng = np.random.default_rng(n + d)
+    x = rng.standard_normal((n, d)).astype(np.float32)
+    print("copies n=%d d=%d (%.1f MB)" % (n, d, x.nbytes / 2**20), flush=True)
+    V = device.DeviceSet(x)
+    back = np.empty_like(x)
+    ya.check(ya.lib().yk_download_vectors(back.ctypes.data, V.vec.ptr, n, d), "download")
+    raw = V.vec.to_host(np.float32, (n, V.ld))
+    V.free()
+    assert np.array_equal(back, x)
+    assert np.array_equal(raw[:, :d], x) and not raw[:, d:].any()

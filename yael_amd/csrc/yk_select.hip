@@ -1541,7 +1541,8 @@ static int yk_knn_filtered(ScanArgs base, int k, int *assign, float *dis, YkAren
     for (;;) {
       YK_TRY(yk_launch_scan(3, pb, a));
       YK_TRY(yk_select(a, thr, k, assign + q0 * k, dis + q0 * k, flag));
-      if (small) {  // (C) what is left, if anything
+      if (small) {  // (C) what is left, if anything (a base that fits a list leaves nothing)
+        if (a.nb <= YK_CAND_CAP) break;
         a.flag = flag;
         YK_TRY(yk_launch_scan(2, pc, a));
         const int n = pc.nsplit * 2 * YK_REG_R;

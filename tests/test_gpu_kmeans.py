@@ -310,3 +310,28 @@ def test_kmeanspp_float_runs_golden(ya):
                                     init="kmeans++", output="all")
     assert abs(q - float(gl["ret"])) <= 2e-3 * abs(float(gl["ret"])), (q, gl["ret"])
     assert (asg == gl["assign"]).mean() > 0.98
+
+
+@pytest.mark.parametrize("n,d,k,ne,heavy", [
+    (3000, 8, 40, 7, 0), (9000, 5, 1024, 300, 0), (9000, 20, 1025, 120, 0), (60000, 4, 5000, 900, 0),
+    (70000, 4, 20000, 990, 0), (60000, 4, 300, 50, 40000), (70000, 4, 300, 50, 55000)])
+def test_device_split_bitexact(ya, oracle, n, d, k, ne, heavy):
+    """One step that empties ne clusters (centroids repeated), with the split
+    probabilities over one to sixty-four elements per thread; a cluster of
+    40,000 equal points makes the smallest probability too small for exact
+    sums, one of 55,000 wraps nassign^2 - 1 negative: both go to the host's
+    split.  Integer data: the oracle's centroids bit for bit."""
+    rng = np.random.default_rng(n + k)
+    v = rng.integers(0, 200, (n, d)).astype(np.float32)
+    if heavy:
+        v[:heavy] = 7
+    u = np.unique(v, axis=0)
+    init = u[rng.permutation(len(u))[:k]].copy()
+    init[0] = 7
+    init[rng.permutation(np.arange(1, k))[:ne]] = init[0]
+    print("device split n=%d k=%d ne=%d heavy=%d" % (n, k, ne, heavy), flush=True)
+    q_o, c_o, d_o, a_o, n_o = oracle.kmeans(v, k, 1, flags=0x100000 | 0x10000, seed=3, init=init)
+    c, q, dis, a, na = ya.kmeans(v, k, niter=1, seed=3, verbose=False, init_centroids=init,
+                                 output="all")
+    assert (na == 0).sum() >= ne and np.array_equal(na, n_o) and np.array_equal(a, a_o)
+    assert np.array_equal(c.view(np.int32), c_o.view(np.int32))

@@ -8,8 +8,11 @@
  * initialisation (kmeans.c:15-20), the empty-cluster split with its rand_r /
  * gaussrand_r streams (kmeans.c:166-209), the abandon and stop rules
  * (kmeans.c:300-313) and the best-of-redo bookkeeping (kmeans.c:416-428).
- * Per iteration the host reads back k counts and one double; the centroid
- * matrix crosses the bus only in an iteration that splits a cluster.
+ * Per iteration the host reads back k counts and one double; an iteration
+ * that splits clusters also sends the split's draws (the donors are chosen
+ * and their rows shared out on the device; for k > 65,536, or where the
+ * choice needs the reference's sequential rounding, the centroid matrix is
+ * brought to the host and back).
  *
  * Assign precision: for large k the assign step takes the precision form
  * (yk_knn_bf16 with k = 1, k' = 8): a BF16 MFMA pass keeps each point's 8
@@ -19,6 +22,7 @@
  * result is the FP32 form's, bit for bit, either way.
  */
 #include <math.h>
+#include <pthread.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -86,6 +90,82 @@ int yh_reassign_empty(int d, int k, float *cent, long ldc, const int *nassign, u
   free(eps);
   free(p);
   return nre;
+}
+
+/* the split's perturbation directions: eps row e from its own stream gs[e]
+ * (kmeans.c:190-195); slices of the rows on up to YH_SPLIT_THREADS threads */
+#define YH_SPLIT_THREADS 8
+typedef struct {
+  int e0, e1, d;
+  const unsigned *gs;
+  float *eps;
+} yh_eps_job;
+
+static void *yh_eps_worker(void *arg) {
+  yh_eps_job *j = (yh_eps_job *)arg;
+  for (int e = j->e0; e < j->e1; e++) {
+    unsigned gs = j->gs[e];
+    for (int l = 0; l < j->d; l++) j->eps[(long)e * j->d + l] = (float)yh_gaussrand_r(&gs);
+  }
+  return NULL;
+}
+
+static void yh_eps_rows(int ne, int d, const unsigned *gs, float *eps) {
+  yh_eps_job job[YH_SPLIT_THREADS];
+  pthread_t th[YH_SPLIT_THREADS];
+  int started[YH_SPLIT_THREADS] = {0};
+  /* a thread is worth starting for ~4096 deviates (~0.3 ms) */
+  long nt = (long)ne * d / 4096;
+  if (nt > YH_SPLIT_THREADS) nt = YH_SPLIT_THREADS;
+  if (nt > ne) nt = ne;
+  if (nt < 1) nt = 1;
+  for (int t = 0; t < nt; t++) {
+    job[t] = (yh_eps_job){(int)((long)ne * t / nt), (int)((long)ne * (t + 1) / nt), d, gs, eps};
+    if (t > 0) started[t] = pthread_create(&th[t], NULL, yh_eps_worker, &job[t]) == 0;
+  }
+  yh_eps_worker(&job[0]);
+  for (int t = 1; t < nt; t++) {
+    if (started[t])
+      pthread_join(th[t], NULL);
+    else
+      yh_eps_worker(&job[t]);
+  }
+}
+
+/* The split on the device: the draws are the reference's streams in its
+ * order, the choice of the donors runs while the directions are drawn.  *done
+ * = 0: not done (nothing changed), the host's split takes over. */
+#define YH_SPLIT_MAX_K 65536
+static int yh_split_device(int d, int k, float *cent, const int *counts, const int *hcounts, int ne,
+                           unsigned seed, int *done) {
+  *done = 0;
+  if (k < 2 || k > YH_SPLIT_MAX_K) return YK_OK;
+  void *ws = yh_buf(YH_KM_SPLIT, yk_split_ws_bytes(ne, d));
+  if (!ws) return YK_ENOMEM;
+  double *rd = (double *)malloc(sizeof(double) * (size_t)ne);
+  unsigned *gs = (unsigned *)malloc(sizeof(unsigned) * (size_t)ne);
+  int *empties = (int *)malloc(sizeof(int) * (size_t)ne);
+  float *eps = (float *)malloc(sizeof(float) * (size_t)ne * d);
+  int rc = YK_OK;
+  if (!rd || !gs || !empties || !eps) rc = yk_set_error_c(YK_ENOMEM, "host malloc");
+  if (rc == YK_OK) {
+    for (int c = 0, e = 0; c < k; c++) {
+      if (hcounts[c] != 0) continue;
+      empties[e] = c;
+      rd[e] = yh_drand_r(&seed);
+      gs[e++] = (unsigned)rand_r(&seed);
+    }
+    rc = yk_split_pick(counts, k, ne, rd, empties, ws);
+  }
+  if (rc == YK_OK) {
+    yh_eps_rows(ne, d, gs, eps);
+    rc = yk_split_apply(cent, d, ne, eps, ws, done);
+  }
+  free(rd);
+  free(gs);
+  free(empties);
+  free(eps);
+  return rc;
 }
 
 /* The first k entries of the Fisher-Yates shuffle of vector.c:226-253 are
@@ -230,7 +310,14 @@ static int yh_kmeans_core(int d, int n, int k, int niter, int flags, int verbose
     for (int c = 0; c < k; c++) nempty += hcounts[c] == 0;
     unsigned split_seed = (unsigned)rand_r(&seed);
     int nre = 0;
-    if (nempty) {
+    int split = 0;
+    if (nempty && (rc = yh_split_device(d, k, m->c, m->counts, hcounts, nempty, split_seed,
+                                        &split)) != YK_OK)
+      return rc;
+    if (split) {
+      nre = nempty;
+      if (verbose) fprintf(stderr, "# kmeans warning: %d empty clusters -> split\n", nre);
+    } else if (nempty) {
       if ((rc = yk_memcpy_d2h(hcent, m->c, sizeof(float) * (size_t)k * ld)) != YK_OK) return rc;
       nre = yh_reassign_empty(d, k, hcent, ld, hcounts, split_seed);
       if ((rc = yk_memcpy_h2d(m->c, hcent, sizeof(float) * (size_t)k * ld)) != YK_OK) return rc;

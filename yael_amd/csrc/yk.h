@@ -153,6 +153,16 @@ int yk_kmeans_update_async(long n, int k, int d, const float *v, const int *assi
                            float *cent, int *counts, int normalize, void *ws);
 int yk_kmeans_readback_checked(const int *counts, int k, int *counts_host, const float *dis,
                                long n, double *obj_host, void *ws, void *upd_ws);
+/* The empty-cluster split on the device (kmeans.c:166-209) for k <= 65536:
+ * yk_split_pick enqueues the choice of the ne donors from the cluster sizes
+ * (device) and the split's ne uniform draws (host arrays: rd, and the empty
+ * clusters in ascending order); yk_split_apply shares the donors' rows out
+ * with the perturbation directions eps (ne x d, host) and waits.  *done = 0:
+ * the choice needs the reference's sequential rounding, nothing was changed.
+ * ws: yk_split_ws_bytes(ne, d) of device memory. */
+size_t yk_split_ws_bytes(int ne, int d);
+int yk_split_pick(const int *counts, int k, int ne, const double *rd, const int *empties, void *ws);
+int yk_split_apply(float *cent, int d, int ne, const float *eps, void *ws, int *done);
 /* k-means++ step: best[j] = min(best[j], squared distance of point j to
  * point s) for j < n (first: best starts at HUGE_VAL); vn: the points'
  * double norms (yk_norms out_d); host_copy (optional, from yk_host_alloc)

@@ -579,6 +579,215 @@ extern "C" int yk_kmeans_readback_checked(const int *counts, int k, int *counts_
   return err ? yk_kmeans_nearest_error() : YK_OK;
 }
 
+// ---------------------------------------------------------------------------
+// The empty-cluster split (kmeans.c:166-209).  The sequential part is the
+// choice of the donors: per empty cluster a walk of the uniform draw down the
+// split probabilities p, the donor's set to 0, and p normalised again in L1
+// norm, every element rounded to float: O(k) per empty cluster (64 us on the
+// host at k = 65,536, 1,865 clusters in one iteration: 120 of a 163 ms call).
+// One workgroup holds p in registers, thread t a run of elements in index
+// order, and takes the empty clusters one after the other: ~3 us each.
+//
+// The reference's sums and walk are sequential in double.  Here they are
+// prefix sums, equal to them because every partial sum is exact: the floats p
+// are multiples of 2^-52 (the smallest positive one is at least 2^-28 at
+// first, and 65,536 roundings of the sum cannot halve it) and their sum is
+// below 2, so 53 bits hold every partial sum in any order, and the draws
+// (multiples of 2^-31) less such sums as well.  Where that does not
+// hold (a smaller probability, a negative one from the 32-bit wrap of
+// nassign^2 - 1, or the walk ending on the last cluster with nothing left
+// there) *flag is set and the host does the split.
+
+// p normalised and summed per thread: p[i] = float(p[i] * inv)
+template <int PT>
+__device__ __forceinline__ double yk_split_scale(float (&p)[PT], double inv) {
+  double s = 0.0;
+#pragma unroll
+  for (int i = 0; i < PT; i++) {
+    p[i] = (float)((double)p[i] * inv);
+    s += (double)p[i];
+  }
+  return s;
+}
+
+template <int PT>
+__global__ __launch_bounds__(1024) void yk_split_pick_kernel(const int *__restrict__ counts, int k,
+                                                             const double *__restrict__ rd, int ne,
+                                                             int *__restrict__ pick, int *flag) {
+  __shared__ double wsum[16];
+  __shared__ double s_left;  // the probabilities' sum without the donor's
+  __shared__ int s_bad;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  if (t == 0) s_bad = 0;
+  float p[PT];
+  double s = 0.0;
+#pragma unroll
+  for (int i = 0; i < PT; i++) {
+    const int c = t * PT + i;
+    const unsigned u = c < k ? (unsigned)counts[c] : 0u;
+    p[i] = u < 2 ? 0.f : (float)(int)(u * u - 1u);
+    s += (double)p[i];
+  }
+  // inclusive scan over the threads (exact, see above); *tot: the total
+  auto scan = [&](double x, double *tot) {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const double y = __shfl_up(x, o);
+      if (lane >= o) x += y;
+    }
+    if (lane == 63) wsum[wave] = x;
+    __syncthreads();
+    double before = 0.0, all = 0.0;
+#pragma unroll
+    for (int w = 0; w < 16; w++) {
+      const double v = wsum[w];
+      if (w < wave) before += v;
+      all += v;
+    }
+    *tot = all;
+    return x + before;
+  };
+  double tot;
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < PT; i++) bad |= p[i] < 0.f;
+  scan(s, &tot);
+  s = yk_split_scale<PT>(p, 1.0 / tot);
+#pragma unroll
+  for (int i = 0; i < PT; i++) bad |= p[i] > 0.f && p[i] < 0x1p-28f;
+  if (bad || !(tot > 0.0)) s_bad = 1;
+  __syncthreads();  // also: wsum is free again
+  for (int e = 0; e < ne && !s_bad; e++) {
+    const double incl = scan(s, &tot);
+    const double r = rd[e];
+    // the first j < k - 1 whose prefix exceeds the draw, else k - 1
+    const double before = incl - s;
+    const int last = k - 1;
+    const bool mine_last = last / PT == t;
+    // (a donor below k - 1 lies in the first thread whose prefix, without
+    // element k - 1, exceeds the draw)
+    double cum = before;
+    int j = -1;
+    double pj = 0.0;
+    if (before <= r && (incl > r || mine_last)) {
+#pragma unroll
+      for (int i = 0; i < PT; i++) {
+        const int c = t * PT + i;
+        if (c < last && j < 0) {
+          cum += (double)p[i];
+          if (cum > r) {
+            j = c;
+            pj = (double)p[i];
+            p[i] = 0.f;
+          }
+        }
+      }
+      if (j < 0 && mine_last) {  // nothing before k - 1
+#pragma unroll
+        for (int i = 0; i < PT; i++)
+          if (t * PT + i == last) {
+            j = last;
+            pj = (double)p[i];
+            p[i] = 0.f;
+          }
+      }
+    }
+    if (j >= 0) {
+      pick[e] = j;
+      s_left = tot - pj;
+      if (!(pj > 0.0) || !(tot - pj > 0.0)) s_bad = 1;  // an empty donor, or none left
+    }
+    __syncthreads();
+    s = yk_split_scale<PT>(p, 1.0 / s_left);
+    __syncthreads();  // every thread has read s_left and s_bad's state
+  }
+  if (t == 0) *flag = s_bad;
+}
+
+// the donors' rows shared out: one wave per empty cluster (kmeans.c:186-203).
+// The donors are distinct and none is empty, so the order is free.  The
+// double sum of float squares goes through the columns in order.
+__global__ __launch_bounds__(256) void yk_split_rows_kernel(float *__restrict__ cent, int d, int ld,
+                                                            const int *__restrict__ empties,
+                                                            const int *__restrict__ pick, int ne,
+                                                            const float *__restrict__ eps,
+                                                            const int *__restrict__ flag) {
+  const int lane = threadIdx.x & 63;
+  const int e = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (e >= ne || *flag) return;
+  float *cc = cent + (long)empties[e] * ld, *cj = cent + (long)pick[e] * ld;
+  double nr = 0.0;
+  for (int j0 = 0; j0 < d; j0 += 64) {
+    const float x = j0 + lane < d ? cj[j0 + lane] : 0.0f;
+    const float sq = __fmul_rn(x, x);
+    const int m = d - j0 < 64 ? d - j0 : 64;
+    for (int t = 0; t < m; t++) nr = __dadd_rn(nr, (double)__shfl(sq, t));
+  }
+  const double s = __dmul_rn(__dsqrt_rn(nr), 0.0000001);
+  for (int l = lane; l < d; l += 64) {
+    const float el = (float)__dmul_rn((double)eps[(long)e * d + l], s), x = cj[l];
+    cj[l] = __fadd_rn(x, el);
+    cc[l] = __fsub_rn(x, el);
+  }
+}
+
+extern "C" size_t yk_split_ws_bytes(int ne, int d) {
+  return 256 + yk_align(sizeof(double) * (size_t)ne) + 2 * yk_align(sizeof(int) * (size_t)ne) +
+         yk_align(sizeof(float) * (size_t)ne * d);
+}
+
+struct SplitWs {
+  int *flag;
+  double *rd;
+  int *empties, *pick;
+  float *eps;
+};
+static SplitWs yk_split_layout(void *ws, int ne) {
+  SplitWs w;
+  char *p = (char *)ws;
+  w.flag = (int *)p;
+  p += 256;
+  w.rd = (double *)p;
+  p += yk_align(sizeof(double) * (size_t)ne);
+  w.empties = (int *)p;
+  p += yk_align(sizeof(int) * (size_t)ne);
+  w.pick = (int *)p;
+  p += yk_align(sizeof(int) * (size_t)ne);
+  w.eps = (float *)p;
+  return w;
+}
+
+extern "C" int yk_split_pick(const int *counts, int k, int ne, const double *rd,
+                             const int *empties, void *ws) {
+  YK_TRY(yk_init());
+  if (ne < 1 || k < 2 || k > 65536)
+    return yk_set_error(YK_EINVAL, "yk_split_pick: %d empty clusters of %d", ne, k);
+  const SplitWs w = yk_split_layout(ws, ne);
+  YK_TRY(yk_memcpy_h2d(w.rd, rd, sizeof(double) * (size_t)ne));
+  YK_TRY(yk_memcpy_h2d(w.empties, empties, sizeof(int) * (size_t)ne));
+  auto kern = k <= 1024    ? yk_split_pick_kernel<1>
+              : k <= 4096  ? yk_split_pick_kernel<4>
+              : k <= 16384 ? yk_split_pick_kernel<16>
+                           : yk_split_pick_kernel<64>;
+  hipLaunchKernelGGL(kern, dim3(1), dim3(1024), 0, yk_stream(), counts, k, w.rd, ne, w.pick,
+                     w.flag);
+  YK_HIP(hipGetLastError());
+  return YK_OK;
+}
+
+extern "C" int yk_split_apply(float *cent, int d, int ne, const float *eps, void *ws, int *done) {
+  YK_TRY(yk_init());
+  const SplitWs w = yk_split_layout(ws, ne);
+  YK_TRY(yk_memcpy_h2d(w.eps, eps, sizeof(float) * (size_t)ne * d));
+  hipLaunchKernelGGL(yk_split_rows_kernel, dim3((unsigned)((ne + 3) / 4)), dim3(256), 0,
+                     yk_stream(), cent, d, yk_ld(d), w.empties, w.pick, ne, w.eps, w.flag);
+  YK_HIP(hipGetLastError());
+  int flag = 0;
+  YK_TRY(yk_read_small(&flag, w.flag, sizeof(int)));
+  *done = !flag;
+  return YK_OK;
+}
+
 // workspace pointer of the objective partials (for callers that keep the
 // objective on the device)
 double *yk_ws_obj(void *ws, long n, int k) { return yk_ws_layout(ws, n, k).obj; }

@@ -139,14 +139,17 @@ extern "C" int yk_host_free(void *p) {
 // largest readback through the pinned landing buffer of yk_read_small (one
 // memcpy of it costs less than the second wait of a pageable copy)
 #define YK_READ_SMALL ((size_t)256 << 10)
-#define YK_STAGE_MIN_D2H ((size_t)16 << 20)
+// smallest copies through the staging threads: down 4 MB (17 GB/s plain, 22
+// staged; 32 MB 17 and 38), up 16 MB (37 and 43; plain is ahead below)
+#define YK_STAGE_MIN_DOWN ((size_t)4 << 20)
+#define YK_STAGE_MIN_UP ((size_t)16 << 20)
 static int yk_copy_staged(char *dev, char *host, size_t bytes, bool up);
 
 extern "C" int yk_memcpy_d2h(void *dst, const void *src, size_t bytes) {
   YK_TRY(yk_init());
   if (!bytes) return YK_OK;
   if (bytes <= YK_READ_SMALL) return yk_read_small(dst, src, bytes);
-  if (bytes >= YK_STAGE_MIN_D2H) return yk_copy_staged((char *)src, (char *)dst, bytes, false);
+  if (bytes >= YK_STAGE_MIN_DOWN) return yk_copy_staged((char *)src, (char *)dst, bytes, false);
   YK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, g_stream));
   YK_HIP(hipStreamSynchronize(g_stream));
   return YK_OK;
@@ -223,15 +226,18 @@ extern "C" int yk_sync(void) {
   return YK_OK;
 }
 
-// Large copies from and to pageable host memory: YK_STAGE_THREADS host threads
-// each take a contiguous slice and push it through two pinned buffers of
-// YK_STAGE_BYTES on a stream of their own (default priority), the host copy
-// of one buffer overlapping the DMA of the other.  The pinned buffers (128 MB
-// in all) are allocated at the first large copy and kept until the process
-// ends; a mutex keeps one staged copy at a time.
-#define YK_STAGE_THREADS 8
+// Copies of YK_STAGE_MIN_* bytes and more from and to pageable host memory: up
+// to YK_STAGE_THREADS host threads, one per YK_STAGE_SLICE bytes, each take a
+// contiguous slice and push it through two pinned buffers on a stream of
+// their own (default priority), the host copy of one buffer overlapping the
+// DMA of the other.  (A plain copy to pageable memory goes in 1 MB pieces, 20
+// us on the bus and ~70 us between them.  256 MB: 17 GB/s plain, 51 with four
+// threads, 42 with eight.)  The pinned buffers (64 MB in all)
+// are allocated at the first such copy and kept until the process ends; a
+// mutex keeps one staged copy at a time.
+#define YK_STAGE_THREADS 4
+#define YK_STAGE_SLICE ((size_t)2 << 20)
 #define YK_STAGE_BYTES ((size_t)8 << 20)
-#define YK_STAGE_MIN ((size_t)64 << 20)
 static pthread_mutex_t g_stage_mu = PTHREAD_MUTEX_INITIALIZER;
 static void *g_stage_buf[YK_STAGE_THREADS][2];
 static hipStream_t g_stage_st[YK_STAGE_THREADS];
@@ -249,6 +255,9 @@ struct YkStageJob {
 static void *yk_stage_worker(void *arg) {
   YkStageJob *j = (YkStageJob *)arg;
   size_t pend[2] = {0, 0}, at[2] = {0, 0};  // bytes in flight through each buffer, their place
+  // two pieces of a slice or more, so that the buffers overlap
+  size_t piece = (j->bytes / 2 + 4095) & ~(size_t)4095;
+  if (piece > YK_STAGE_BYTES) piece = YK_STAGE_BYTES;
   auto settle = [&](int b) {  // the buffer's DMA is done; down: its bytes go to the host
     if (!pend[b]) return hipSuccess;
     const hipError_t e = hipEventSynchronize(g_stage_ev[j->t][b]);
@@ -258,7 +267,7 @@ static void *yk_stage_worker(void *arg) {
   };
   size_t off = 0;
   for (int b = 0; off < j->bytes && j->err == hipSuccess; b ^= 1) {
-    const size_t n = j->bytes - off < YK_STAGE_BYTES ? j->bytes - off : YK_STAGE_BYTES;
+    const size_t n = j->bytes - off < piece ? j->bytes - off : piece;
     void *buf = g_stage_buf[j->t][b];
     hipError_t e = settle(b);
     if (e == hipSuccess && j->up) memcpy(buf, j->host + off, n);
@@ -296,7 +305,9 @@ static int yk_copy_staged(char *dev, char *host, size_t bytes, bool up) {
   pthread_mutex_lock(&g_stage_mu);
   int rc = yk_stage_setup();
   if (rc == YK_OK) {
-    const size_t per = (bytes / YK_STAGE_THREADS + 4095) & ~(size_t)4095;
+    size_t ways = bytes / YK_STAGE_SLICE;
+    if (ways > YK_STAGE_THREADS) ways = YK_STAGE_THREADS;
+    const size_t per = (bytes / ways + 4095) & ~(size_t)4095;
     YkStageJob job[YK_STAGE_THREADS];
     pthread_t th[YK_STAGE_THREADS];
     int started[YK_STAGE_THREADS] = {0}, nt = 0;
@@ -387,7 +398,7 @@ static int yk_dense_copy(float *dev, float *host, long n, int d, bool up) {
       YK_TRY(yk_memcpy_d2h(host + i * d, buf, bytes));
       continue;
     }
-    if (bytes >= YK_STAGE_MIN_D2H)
+    if (bytes >= YK_STAGE_MIN_UP)
       YK_TRY(yk_copy_staged((char *)buf, (char *)(host + i * d), bytes, true));
     else
       YK_HIP(hipMemcpyAsync(buf, host + i * d, bytes, hipMemcpyHostToDevice, g_stream));
@@ -412,7 +423,7 @@ extern "C" int yk_upload_vectors(float *dst, const float *src, long n, int d) {
     pthread_mutex_unlock(&g_dense_mu);
     return rc;
   }
-  if (bytes >= YK_STAGE_MIN) return yk_copy_staged((char *)dst, (char *)src, bytes, true);
+  if (bytes >= YK_STAGE_MIN_UP) return yk_copy_staged((char *)dst, (char *)src, bytes, true);
   YK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, g_stream));
   YK_HIP(hipStreamSynchronize(g_stream));
   return YK_OK;

@@ -151,6 +151,32 @@ def test_starting_bound_underflow(dev):
     assert counts == [3, 1]
 
 
+@pytest.mark.parametrize("typ", [2, 16])
+def test_captured_lists_certify(dev, typ):
+    """k' = k leaves nearly every query uncertified at first; the keys that
+    the filtered pass captured up to its bound (about 256 per query here, more
+    or fewer than the 8 k' the second look takes) certify them without
+    another search: one filtered pass, one sketch."""
+    import ctypes
+    import yael_amd
+    rng = np.random.default_rng(31)
+    b = rng.standard_normal((40000, 64)).astype(np.float32)
+    q = rng.standard_normal((300, 64)).astype(np.float32)
+    lib = yael_amd.lib()
+    lib.yk_prof_enable(1)
+    lib.yk_prof_reset()
+    try:
+        assert same_as_fp32(dev, q, b, 32, 32, typ) == 0
+        counts = []
+        for slot in (6, 7, 4):  # filtered-pass scans, sketch scans, re-ranks
+            tot, cnt = ctypes.c_double(), ctypes.c_long()
+            lib.yk_prof_get(slot, ctypes.byref(tot), ctypes.byref(cnt))
+            counts.append(cnt.value)
+    finally:
+        lib.yk_prof_enable(0)
+    assert counts == [1, 1, 2]
+
+
 def test_small_base(dev):
     rng = np.random.default_rng(10)
     b = mixture(rng, 50, 16, 4, 10)

@@ -40,6 +40,8 @@
 #include <stdio.h>
 #include <stdlib.h>
 
+#include <type_traits>
+
 #include "yk.h"
 #include "yk_dev.h"
 #include "yk_wsel.h"
@@ -1072,7 +1074,7 @@ __global__ __launch_bounds__(256) void yk_bf_rsel_thr_kernel(const uint64_t *__r
 template <int E, int E2>
 __device__ __forceinline__ void yk_rsel_cand(const uint64_t *p, int m, int n, int kp, int lane,
                                              uint64_t *lds, uint64_t *dst, uint64_t *thr,
-                                             int *cnt, int *flag) {
+                                             uint64_t *bnd, int *cnt, int *flag) {
   if (n < kp && *thr != YK_KEY_NONE) {
     // fewer than kp keys within the starting bound (an estimated one: under
     // a proven bound, or under an overflow's, kp keys or more are within
@@ -1102,11 +1104,15 @@ __device__ __forceinline__ void yk_rsel_cand(const uint64_t *p, int m, int n, in
     return;
   }
   yk_wave_topk<E, E2>(v, kp, lane, lds, dst);
-  if (lane == 0) *thr = 0;
+  if (lane == 0) {
+    *bnd = *thr;
+    *thr = 0;
+  }
 }
 
 // The filtered pass's candidate lists: per query (thr != 0) the kp smallest
-// of its captured keys, sorted, to cand_out, and thr cleared.  A list that
+// of its captured keys, sorted, to cand_out, and thr cleared (its value kept
+// in bnd: the list holds every key up to it).  A list that
 // overflowed YK_CAND_CAP gets a tighter bound and the flag; one with fewer
 // than kp keys (under an estimated starting bound) gets no bound and the
 // flag.  Either way the query's list is written empty until its next pass.
@@ -1114,8 +1120,8 @@ __device__ __forceinline__ void yk_rsel_cand(const uint64_t *p, int m, int n, in
 template <int E2>
 __global__ __launch_bounds__(256) void yk_bf_rsel_cand_kernel(const uint64_t *__restrict__ cand,
                                                               long nq, int *cnt, uint64_t *thr,
-                                                              int kp, uint64_t *cand_out,
-                                                              int *flag) {
+                                                              uint64_t *bnd, int kp,
+                                                              uint64_t *cand_out, int *flag) {
   __shared__ uint64_t lds[4][64 * E2];
   const long q = blockIdx.x * 4L + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1125,15 +1131,57 @@ __global__ __launch_bounds__(256) void yk_bf_rsel_cand_kernel(const uint64_t *__
   const uint64_t *p = cand + q * (long)YK_CAND_CAP;
   uint64_t *dst = cand_out + q * kp;
   if (m <= 256)
-    yk_rsel_cand<4, E2>(p, m, n, kp, lane, lds[wave], dst, thr + q, cnt + q, flag);
+    yk_rsel_cand<4, E2>(p, m, n, kp, lane, lds[wave], dst, thr + q, bnd + q, cnt + q, flag);
   else if (m <= 512)
-    yk_rsel_cand<8, E2>(p, m, n, kp, lane, lds[wave], dst, thr + q, cnt + q, flag);
+    yk_rsel_cand<8, E2>(p, m, n, kp, lane, lds[wave], dst, thr + q, bnd + q, cnt + q, flag);
   else if (m <= 1024)
-    yk_rsel_cand<16, E2>(p, m, n, kp, lane, lds[wave], dst, thr + q, cnt + q, flag);
+    yk_rsel_cand<16, E2>(p, m, n, kp, lane, lds[wave], dst, thr + q, bnd + q, cnt + q, flag);
   else if (m <= 2048)
-    yk_rsel_cand<32, E2>(p, m, n, kp, lane, lds[wave], dst, thr + q, cnt + q, flag);
+    yk_rsel_cand<32, E2>(p, m, n, kp, lane, lds[wave], dst, thr + q, bnd + q, cnt + q, flag);
   else
-    yk_rsel_cand<64, E2>(p, m, n, kp, lane, lds[wave], dst, thr + q, cnt + q, flag);
+    yk_rsel_cand<64, E2>(p, m, n, kp, lane, lds[wave], dst, thr + q, bnd + q, cnt + q, flag);
+}
+
+// Wider lists for the queries the certificate left over: query list[i]'s
+// kp smallest captured keys, sorted, to cand_out[i], and in rest[i] the key
+// that bounds every other key of the base from below -- the kp-th of them, or
+// where the whole capture fits, the bound it was captured under.  One wave
+// per query.
+template <int E2>
+__global__ __launch_bounds__(256) void yk_bf_widen_kernel(
+    const uint64_t *__restrict__ cand, const int *__restrict__ cnt,
+    const uint64_t *__restrict__ bnd, const int *__restrict__ list, long nlist, int kp,
+    uint64_t *__restrict__ cand_out, uint64_t *__restrict__ rest) {
+  __shared__ uint64_t lds[4][64 * E2];
+  const long i = blockIdx.x * 4L + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (i >= nlist) return;
+  const long q = list[i];
+  const int m = min(cnt[q], YK_CAND_CAP);
+  const uint64_t *p = cand + q * (long)YK_CAND_CAP;
+  uint64_t *dst = cand_out + i * kp;
+  auto pick = [&](auto e) {
+    constexpr int E = decltype(e)::value;
+    uint64_t v[E], w[E2];
+    yk_wave_load<E>(p, m, lane, v);
+    yk_wave_topk_reg<E, E2>(v, kp, lane, lds[wave], w);
+#pragma unroll
+    for (int s = 0; s < E2; s++) {
+      const int t = lane * E2 + s;
+      if (t < kp) dst[t] = w[s];
+      if (t == kp - 1) rest[i] = m > kp ? w[s] : bnd[q];
+    }
+  };
+  if (m <= 256)
+    pick(std::integral_constant<int, 4>());
+  else if (m <= 512)
+    pick(std::integral_constant<int, 8>());
+  else if (m <= 1024)
+    pick(std::integral_constant<int, 16>());
+  else if (m <= 2048)
+    pick(std::integral_constant<int, 32>());
+  else
+    pick(std::integral_constant<int, 64>());
 }
 
 // yk_bf_sortsel_kernel for n <= 1024 keys per query: four queries per
@@ -1207,19 +1255,22 @@ __device__ __forceinline__ bool yk_rerank_needed(const uint64_t *cq, int kp, int
   return kk != YK_KEY_NONE && (double)yk_fkey_inv((uint32_t)(kk >> 32)) <= bound;
 }
 
+//
+// With qlist, query i of the call (its lists and ex) is query qlist[i] of
+// the queries and results: the second look at the uncertified ones.
 template <int NCH>
 __global__ __launch_bounds__(64) void yk_rerank_tile_kernel(
     const float *__restrict__ q, const double *__restrict__ qn, const float *__restrict__ b,
     const float *__restrict__ bn, int ld, int type, const uint64_t *__restrict__ cand, int kp,
     int k, const float4 *__restrict__ qstats, const float4 *__restrict__ bmax, float gam_bf,
-    float gam_32, uint64_t *__restrict__ ex) {
-  const long qi = blockIdx.y;
+    float gam_32, const int *__restrict__ qlist, uint64_t *__restrict__ ex) {
+  const long qi = blockIdx.y, qr = qlist ? qlist[qi] : qi;
   const int t0 = blockIdx.x * 32;
   const int lane = threadIdx.x, r = lane & 31, h = lane >> 5;
   const bool dot = type == YK_DOT;
   const uint64_t *cq = cand + qi * kp;
   double ebf, e32, bound;
-  yk_rerank_bound(dot, qstats[qi], *bmax, gam_bf, gam_32, cq[k - 1], &ebf, &e32, &bound);
+  yk_rerank_bound(dot, qstats[qr], *bmax, gam_bf, gam_32, cq[k - 1], &ebf, &e32, &bound);
   if (!yk_rerank_needed(cq, kp, t0, bound)) return;
   // A candidate whose first-pass value is above the bound cannot be among
   // the k nearest (its FP32-form value exceeds the k-th's, as for a whole
@@ -1232,7 +1283,7 @@ __global__ __launch_bounds__(64) void yk_rerank_tile_kernel(
   const uint64_t key = ci < kp ? cq[ci] : YK_KEY_NONE;
   const long row = beyond(key) ? 0 : (long)(uint32_t)key;
   const float *bp = b + row * ld + h * 8;
-  const float *qp = q + qi * ld + h * 8;
+  const float *qp = q + qr * ld + h * 8;
   const int nch = NCH > 0 ? NCH : ld >> 4;
   f32x16 acc;
 #pragma unroll
@@ -1279,7 +1330,7 @@ __global__ __launch_bounds__(64) void yk_rerank_tile_kernel(
   }
   // column 0 (lanes 0 and 32) holds the tile's candidate rows 8g + 4h + e
   if (r == 0) {
-    const double qnd = dot ? 0.0 : qn[qi];
+    const double qnd = dot ? 0.0 : qn[qr];
 #pragma unroll
     for (int i = 0; i < 16; i++) {
       const int cidx = t0 + 8 * (i >> 2) + 4 * h + (i & 3);
@@ -1324,22 +1375,23 @@ __device__ __forceinline__ void yk_rerank_finish(const uint64_t *exq, int nproc,
 __global__ __launch_bounds__(256) void yk_rerank_fin_kernel(
     const uint64_t *__restrict__ cand, long n, long nb, int type, int kp, int k,
     const float4 *__restrict__ qstats, const float4 *__restrict__ bmax, float gam_bf,
-    float gam_32, const uint64_t *__restrict__ ex, int *out_i, float *out_d, int *unc_list,
-    int *n_unc) {
+    float gam_32, const int *__restrict__ qlist, const uint64_t *__restrict__ rest,
+    const uint64_t *__restrict__ ex, int *out_i, float *out_d, int *unc_list, int *n_unc) {
   __shared__ uint64_t kth_s[4];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const long qi = blockIdx.x * 4L + wave;
   if (qi >= n) return;
+  const long qr = qlist ? qlist[qi] : qi;
   const uint64_t *cq = cand + qi * kp;
   double ebf, e32, bound;
-  yk_rerank_bound(type == YK_DOT, qstats[qi], *bmax, gam_bf, gam_32, cq[k - 1], &ebf, &e32,
+  yk_rerank_bound(type == YK_DOT, qstats[qr], *bmax, gam_bf, gam_32, cq[k - 1], &ebf, &e32,
                   &bound);
   int nproc = 0;  // candidates re-ranked: the leading tiles that start within the bound
   for (int t0 = 0; yk_rerank_needed(cq, kp, t0, bound); t0 += 32) nproc = min(kp, t0 + 32);
   const int m = max(nproc, k);
   const uint64_t *exq = ex + qi * kp;
-  int *oi = out_i + qi * k;
-  float *od = out_d + qi * k;
+  int *oi = out_i + qr * k;
+  float *od = out_d + qr * k;
   uint64_t *kth = kth_s + wave;
   if (m <= 256)
     yk_rerank_finish<4>(exq, nproc, k, lane, oi, od, kth);
@@ -1350,11 +1402,12 @@ __global__ __launch_bounds__(256) void yk_rerank_fin_kernel(
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
   if (lane == 0) {
-    // the first pass kept the kp smallest keys; fewer than kp real ones means
-    // every base vector was a candidate
-    const uint64_t last = cq[kp - 1], fk = *kth;
+    // the first pass kept the kp smallest keys, or every key up to rest[qi];
+    // fewer than kp real ones, or no such bound, means every base vector was
+    // a candidate
+    const uint64_t last = rest ? rest[qi] : cq[kp - 1], fk = *kth;
     bool ok;
-    if (last == YK_KEY_NONE || kp >= nb) {
+    if (last == YK_KEY_NONE || (!rest && kp >= nb)) {
       ok = true;
     } else if (fk == YK_KEY_NONE) {
       ok = false;
@@ -1363,7 +1416,7 @@ __global__ __launch_bounds__(256) void yk_rerank_fin_kernel(
       const float Fk = yk_fkey_inv((uint32_t)(fk >> 32));
       ok = (double)Fk < (double)Tb - ebf - e32;
     }
-    if (!ok) unc_list[atomicAdd(n_unc, 1)] = (int)qi;
+    if (!ok) unc_list[atomicAdd(n_unc, 1)] = (int)qr;
   }
 }
 
@@ -1607,6 +1660,18 @@ static int yk_bnb(int mode, int nch, int r = YK_REG_R) {
   return mode != 2 && nch >= 1 && nch <= 9 ? 3 : 2;
 }
 
+// The sketch's plan: at least kp splits, each giving 4 subset minima per
+// query.  A split of the long-vector kernel gives 4 per wave of its
+// workgroup, so kp / 8 splits do, and 128 keep the minima of a query within
+// the 4,096 that one wave selects from in registers (with 512 splits for
+// k' = 512 a workgroup sorted 16,384 keys per query: 1.53 ms for 917 queries).
+static BPlan yk_bsketch_plan(long nq, long nb, int ldh, long stride, int kp) {
+  const int nch = ldh >> 4;
+  const long per = nch > 16 ? YK_TW : 1;
+  const long least = (kp + per - 1) / per, most = per > 1 ? 128 : 256;
+  return yk_bplan(nq, nb, yk_bnb(1, nch), stride, least, least > most ? least : most, 64L * ldh);
+}
+
 // streaming kernel with exactly nch register-resident chunks (nch <= 16),
 // else the one streaming both operands
 template <int MODE, int R>
@@ -1708,7 +1773,13 @@ static int yk_bf_sortsel(const uint64_t *src, long nq, int n, int kp, uint64_t *
 // call enqueues one filtered pass and returns without waiting; with resume
 // (after the caller read the flag set) it repeats the filtered pass for the
 // overflowed queries with their tighter bounds, waiting on the flag each time.
-static int yk_bf16_candidates(Bf16Args a, int kp, uint64_t *cand_out, int *ovf, bool resume) {
+// The captured lists, their lengths and bounds (cap) stay until the next call.
+struct YkCaptured {
+  const uint64_t *cand, *bnd;
+  const int *cnt;
+};
+static int yk_bf16_candidates(Bf16Args a, int kp, uint64_t *cand_out, int *ovf, bool resume,
+                              YkCaptured *cap) {
   const long nq = a.nq;
   void *vpart;
   if (kp <= YK_REG_R) {
@@ -1738,17 +1809,17 @@ static int yk_bf16_candidates(Bf16Args a, int kp, uint64_t *cand_out, int *ovf, 
     return YK_OK;
   }
   void *vthr, *vcnt, *vcand;
-  YK_TRY(yk_bscratch(1, sizeof(uint64_t) * nq, &vthr));
+  YK_TRY(yk_bscratch(1, sizeof(uint64_t) * nq * 2, &vthr));
   YK_TRY(yk_bscratch(2, sizeof(int) * (nq + 64), &vcnt));
   YK_TRY(yk_bscratch(3, sizeof(uint64_t) * nq * YK_CAND_CAP, &vcand));
-  uint64_t *thr = (uint64_t *)vthr;
+  uint64_t *thr = (uint64_t *)vthr, *bnd = thr + nq;
   int *cnt = (int *)vcnt;
+  *cap = {(const uint64_t *)vcand, bnd, cnt};
   if (!resume) {
     // sketch: per-lane minima over a 1-in-stride sample, >= kp splits (same
     // reasoning as the FP32 form in yk_select.hip)
     const long stride = yk_bsketch_stride(a.nb, kp);
-    BPlan pa = yk_bplan(nq, a.nb, yk_bnb(1, a.ldh >> 4), stride, kp, kp > 256 ? kp : 256,
-                        64L * a.ldh);
+    const BPlan pa = yk_bsketch_plan(nq, a.nb, a.ldh, stride, kp);
     // per query and split: 2 lane halves x 2 block parities of minima, and
     // for long vectors that per wave of the tiled kernel's workgroup
     const int nsub = (a.ldh >> 4) > 16 ? 4 * YK_TW : 4;
@@ -1770,13 +1841,13 @@ static int yk_bf16_candidates(Bf16Args a, int kp, uint64_t *cand_out, int *ovf, 
     const dim3 g4((unsigned)((nq + 3) / 4));
     if (kp <= 256)
       hipLaunchKernelGGL(yk_bf_rsel_cand_kernel<4>, g4, dim3(256), 0, yk_stream(), a.cand, nq, cnt,
-                         thr, kp, cand_out, ovf);
+                         thr, bnd, kp, cand_out, ovf);
     else if (kp <= 512)
       hipLaunchKernelGGL(yk_bf_rsel_cand_kernel<8>, g4, dim3(256), 0, yk_stream(), a.cand, nq, cnt,
-                         thr, kp, cand_out, ovf);
+                         thr, bnd, kp, cand_out, ovf);
     else
       hipLaunchKernelGGL(yk_bf_rsel_cand_kernel<16>, g4, dim3(256), 0, yk_stream(), a.cand, nq,
-                         cnt, thr, kp, cand_out, ovf);
+                         cnt, thr, bnd, kp, cand_out, ovf);
     YK_HIP(hipGetLastError());
     if (!resume) break;
     int hflag = 0;
@@ -1868,8 +1939,7 @@ extern "C" int yk_knn_bf16(int type, long nq, long nb, int d, int k, int kp, con
         sig[i][0] = p.nsplit, sig[i][1] = p.brange, sig[i][2] = 0;
       } else {
         const long st = yk_bsketch_stride(nb, kp);
-        const BPlan pa =
-            yk_bplan(nqb, nb, yk_bnb(1, nch), st, kp, kp > 256 ? kp : 256, 64L * ldh);
+        const BPlan pa = yk_bsketch_plan(nqb, nb, ldh, st, kp);
         const BPlan pb = yk_bplan(nqb, nb, yk_bnb(3, nch), 1, 1, 4096, 64L * ldh);
         sig[i][0] = st, sig[i][1] = pa.nsplit, sig[i][2] = pb.nsplit;
       }
@@ -1919,10 +1989,11 @@ static int yk_knn_bf16_run(int type, long nq, long nb, int d, int k, int kp, con
   void *vcand, *vunc;
   const long qb = nq < QB ? nq : QB;
   YK_TRY(yk_bscratch(4, sizeof(uint64_t) * qb * kp, &vcand));
-  YK_TRY(yk_bscratch(5, sizeof(int) * (qb + 64), &vunc));
+  YK_TRY(yk_bscratch(5, sizeof(int) * (2 * qb + 64), &vunc));
   // the uncertified count and the candidate-overflow flag side by side: one
   // read after the re-rank brings both back
-  int *unc = (int *)vunc, *nunc = unc + qb + 32, *ovf = nunc + 1;
+  int *const unc1 = (int *)vunc, *const unc2 = unc1 + qb;
+  int *nunc = unc2 + qb + 32, *ovf = nunc + 1, *nunc2 = nunc + 2;
   const int ld = yk_ld(d), ldh = yk_bf16_ld(d, type);
   const float gam_bf = 2.0f * (ldh + 8) * 0x1p-23f, gam_32 = 2.0f * (ld + 8) * 0x1p-23f;
   int total_fb = 0;
@@ -1946,9 +2017,14 @@ static int yk_knn_bf16_run(int type, long nq, long nb, int d, int k, int kp, con
       YK_HIP(hipGetLastError());
       a.qf = (const uint16_t *)vqf;
     }
-    hipLaunchKernelGGL(yk_bf_zero_kernel, dim3(1), dim3(64), 0, yk_stream(), nunc, 2L);
-    YK_TRY(yk_bf16_candidates(a, kp, (uint64_t *)vcand, ovf, false));
-    auto rerank = [&]() -> int {
+    hipLaunchKernelGGL(yk_bf_zero_kernel, dim3(1), dim3(64), 0, yk_stream(), nunc, 3L);
+    YkCaptured cap = {};
+    YK_TRY(yk_bf16_candidates(a, kp, (uint64_t *)vcand, ovf, false, &cap));
+    // the re-rank of the batch's lists, or of the m lists of kp candidates of
+    // the queries qlist (their other rows at or above rest), certified or not
+    // to ulist
+    auto rerank = [&](const uint64_t *cand, int kp, const int *qlist, long m,
+                      const uint64_t *rest, void *vex, int *ulist, int *nu) -> int {
       int tok = yk_prof_begin(YK_PROF_RERANK);
       if (kp <= 8) {
         void (*rk4)(const float *, const double *, const float *, const float *, long, int, int,
@@ -1965,15 +2041,15 @@ static int yk_knn_bf16_run(int type, long nq, long nb, int d, int k, int kp, con
           case 8: rk4 = yk_rerank4_kernel<8>; break;
           default: rk4 = yk_rerank4_kernel<0>; break;
         }
-        hipLaunchKernelGGL(rk4, dim3((unsigned)((n + 3) / 4)), dim3(64), 0, yk_stream(),
+        hipLaunchKernelGGL(rk4, dim3((unsigned)((m + 3) / 4)), dim3(64), 0, yk_stream(),
                            q + q0 * ld, qn ? qn + q0 : nullptr, b, bn, nb, ld, type,
-                           (const uint64_t *)vcand, n, kp, k, (const float4 *)qstats + q0,
+                           cand, m, kp, k, (const float4 *)qstats + q0,
                            (const float4 *)bstats_max, gam_bf, gam_32, assign + q0 * k,
-                           dis + q0 * k, unc, nunc);
+                           dis + q0 * k, ulist, nu);
       } else {
         void (*rt)(const float *, const double *, const float *, const float *, int, int,
                    const uint64_t *, int, int, const float4 *, const float4 *, float, float,
-                   uint64_t *);
+                   const int *, uint64_t *);
         switch (ld >> 4) {
           case 1: rt = yk_rerank_tile_kernel<1>; break;
           case 2: rt = yk_rerank_tile_kernel<2>; break;
@@ -1985,40 +2061,63 @@ static int yk_knn_bf16_run(int type, long nq, long nb, int d, int k, int kp, con
           case 8: rt = yk_rerank_tile_kernel<8>; break;
           default: rt = yk_rerank_tile_kernel<0>; break;
         }
-        void *vex;
-        YK_TRY(yk_bscratch(8, sizeof(uint64_t) * (size_t)n * kp, &vex));
-        hipLaunchKernelGGL(rt, dim3((unsigned)((kp + 31) / 32), (unsigned)n), dim3(64), 0,
+        hipLaunchKernelGGL(rt, dim3((unsigned)((kp + 31) / 32), (unsigned)m), dim3(64), 0,
                            yk_stream(), q + q0 * ld, qn ? qn + q0 : nullptr, b, bn, ld, type,
-                           (const uint64_t *)vcand, kp, k, (const float4 *)qstats + q0,
-                           (const float4 *)bstats_max, gam_bf, gam_32, (uint64_t *)vex);
-        hipLaunchKernelGGL(yk_rerank_fin_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0,
-                           yk_stream(), (const uint64_t *)vcand, n, nb, type, kp, k,
-                           (const float4 *)qstats + q0, (const float4 *)bstats_max, gam_bf,
-                           gam_32, (const uint64_t *)vex, assign + q0 * k, dis + q0 * k, unc,
-                           nunc);
+                           cand, kp, k, (const float4 *)qstats + q0, (const float4 *)bstats_max,
+                           gam_bf, gam_32, qlist, (uint64_t *)vex);
+        hipLaunchKernelGGL(yk_rerank_fin_kernel, dim3((unsigned)((m + 3) / 4)), dim3(256), 0,
+                           yk_stream(), cand, m, nb, type, kp, k, (const float4 *)qstats + q0,
+                           (const float4 *)bstats_max, gam_bf, gam_32, qlist, rest,
+                           (const uint64_t *)vex, assign + q0 * k, dis + q0 * k, ulist, nu);
       }
       yk_prof_end(tok);
       YK_HIP(hipGetLastError());
       return YK_OK;
     };
-    YK_TRY(rerank());
+    void *vex = nullptr;
+    if (kp > 8) YK_TRY(yk_bscratch(8, sizeof(uint64_t) * (size_t)n * kp, &vex));
+    auto rerank_all = [&]() {
+      return rerank((const uint64_t *)vcand, kp, nullptr, n, nullptr, vex, unc1, nunc);
+    };
+    YK_TRY(rerank_all());
     int hv[2] = {0, 0};
     YK_TRY(yk_read_small(hv, nunc, sizeof(hv)));
     if (hv[1]) {
       // a query's capture overflowed (massive ties): its list was empty in
       // this re-rank; the filtered pass again for such queries, then the
       // re-rank of the batch again
-      YK_TRY(yk_bf16_candidates(a, kp, (uint64_t *)vcand, ovf, true));
+      YK_TRY(yk_bf16_candidates(a, kp, (uint64_t *)vcand, ovf, true, &cap));
       hipLaunchKernelGGL(yk_bf_zero_kernel, dim3(1), dim3(64), 0, yk_stream(), nunc, 1L);
-      YK_TRY(rerank());
+      YK_TRY(rerank_all());
       YK_TRY(yk_read_small(hv, nunc, sizeof(int)));
     }
-    const int hn = hv[0];
-    // Uncertified queries, first level: the precision form again on just
-    // those queries with 8x the candidates (the certificate's margin grows
-    // with the k'-th first-pass value); what that level cannot certify goes
-    // to the FP32 form there.  The result is the FP32 form's either way.
+    int hn = hv[0];
+    const int *unc = unc1;
     const int kp2 = (int)min((long)min(8 * kp, YK_KMAX), nb);
+    // Uncertified queries, first: the filtered pass captured every key up to
+    // its bound, several times k' of them, so 8x the candidates (or all that
+    // were captured) are at hand; the certificate's margin grows with the
+    // last one's value.  (Searching again with 8 k' took 4.7 of 24.1 ms for
+    // 917 of 1e4 queries x 1e6 unit rows, d = 960, k' = 64.)
+    if (hn > 0 && kp > YK_REG_R && kp2 > kp) {
+      const size_t szl = yk_b256(sizeof(uint64_t) * (size_t)hn * kp2);
+      void *vw;
+      YK_TRY(yk_bscratch(6, 2 * szl + sizeof(uint64_t) * hn, &vw));
+      uint64_t *wide = (uint64_t *)vw, *wex = (uint64_t *)((char *)vw + szl),
+               *rest = (uint64_t *)((char *)vw + 2 * szl);
+      const auto widen = kp2 <= 256   ? yk_bf_widen_kernel<4>
+                         : kp2 <= 512 ? yk_bf_widen_kernel<8>
+                                      : yk_bf_widen_kernel<16>;
+      hipLaunchKernelGGL(widen, dim3((unsigned)((hn + 3) / 4)), dim3(256), 0, yk_stream(),
+                         cap.cand, cap.cnt, cap.bnd, unc, (long)hn, kp2, wide, rest);
+      YK_HIP(hipGetLastError());
+      YK_TRY(rerank(wide, kp2, unc, hn, rest, wex, unc2, nunc2));
+      YK_TRY(yk_read_small(&hn, nunc2, sizeof(int)));
+      unc = unc2;
+    }
+    // What is left, first level: the precision form again on just those
+    // queries with 8x the candidates; what that level cannot certify goes
+    // to the FP32 form there.  The result is the FP32 form's either way.
     if (hn > 0 && g_bs_level == 0 && kp2 > kp) {
       // each piece starts on a 256-byte boundary: the gathers write and the
       // nested search reads them with 16-byte vector accesses

@@ -586,7 +586,9 @@ extern "C" int yk_kmeans_readback_checked(const int *counts, int k, int *counts_
 // norm, every element rounded to float: O(k) per empty cluster (64 us on the
 // host at k = 65,536, 1,865 clusters in one iteration: 120 of a 163 ms call).
 // One workgroup holds p in registers, thread t a run of elements in index
-// order, and takes the empty clusters one after the other: ~3 us each.
+// order, and takes the empty clusters one after the other: ~4 us each at
+// k = 65,536, of which the normalisation's five instructions per element on
+// one CU are half.
 //
 // The reference's sums and walk are sequential in double.  Here they are
 // prefix sums, equal to them because every partial sum is exact: the floats p
@@ -598,15 +600,27 @@ extern "C" int yk_kmeans_readback_checked(const int *counts, int k, int *counts_
 // nassign^2 - 1, or the walk ending on the last cluster with nothing left
 // there) *flag is set and the host does the split.
 
+// Each pass converts its p[i] anew: kept from one pass for the next, the
+// doubles of 64 elements alone fill the thread's 128 registers, and p went to
+// scratch memory (with the donor's thread walking its elements one by one:
+// 6.3 us per empty cluster).
+template <int PT>
+__device__ __forceinline__ void yk_split_pass(float (&p)[PT]) {
+#pragma unroll
+  for (int i = 0; i < PT; i++) asm volatile("" : "+v"(p[i]));
+}
+
 // p normalised and summed per thread: p[i] = float(p[i] * inv)
 template <int PT>
 __device__ __forceinline__ double yk_split_scale(float (&p)[PT], double inv) {
   double s = 0.0;
+  yk_split_pass<PT>(p);
 #pragma unroll
   for (int i = 0; i < PT; i++) {
     p[i] = (float)((double)p[i] * inv);
     s += (double)p[i];
   }
+  yk_split_pass<PT>(p);
   return s;
 }
 
@@ -616,6 +630,7 @@ __global__ __launch_bounds__(1024) void yk_split_pick_kernel(const int *__restri
                                                              int *__restrict__ pick, int *flag) {
   __shared__ double wsum[16];
   __shared__ double s_left;  // the probabilities' sum without the donor's
+  __shared__ float s_run[PT];  // the donor's thread's elements
   __shared__ int s_bad;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   if (t == 0) s_bad = 0;
@@ -660,42 +675,43 @@ __global__ __launch_bounds__(1024) void yk_split_pick_kernel(const int *__restri
   for (int e = 0; e < ne && !s_bad; e++) {
     const double incl = scan(s, &tot);
     const double r = rd[e];
-    // the first j < k - 1 whose prefix exceeds the draw, else k - 1
+    // The donor is the first j < k - 1 whose prefix exceeds the draw, else
+    // k - 1.  A donor below k - 1 lies in the first thread whose prefix,
+    // without element k - 1, exceeds the draw; that thread's elements are
+    // spread over its wave, a lane each, for their prefixes.
     const double before = incl - s;
     const int last = k - 1;
-    const bool mine_last = last / PT == t;
-    // (a donor below k - 1 lies in the first thread whose prefix, without
-    // element k - 1, exceeds the draw)
-    double cum = before;
-    int j = -1;
-    double pj = 0.0;
-    if (before <= r && (incl > r || mine_last)) {
+    const bool own = before <= r && (incl > r || last / PT == t);
+    const uint64_t owns = __builtin_amdgcn_ballot_w64(own);
+    if (owns) {  // (one wave)
+      const int src = __builtin_ctzll(owns), c0 = ((wave << 6) + src) * PT;
+      if (own) {
 #pragma unroll
-      for (int i = 0; i < PT; i++) {
-        const int c = t * PT + i;
-        if (c < last && j < 0) {
-          cum += (double)p[i];
-          if (cum > r) {
-            j = c;
-            pj = (double)p[i];
-            p[i] = 0.f;
-          }
-        }
+        for (int i = 0; i < PT; i++) s_run[i] = p[i];
       }
-      if (j < 0 && mine_last) {  // nothing before k - 1
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const double x = lane < PT ? (double)s_run[lane] : 0.0;
+      const bool below = lane < PT && c0 + lane < last;
+      double cum = below ? x : 0.0;
 #pragma unroll
-        for (int i = 0; i < PT; i++)
-          if (t * PT + i == last) {
-            j = last;
-            pj = (double)p[i];
-            p[i] = 0.f;
-          }
+      for (int o = 1; o < (PT < 64 ? PT : 64); o <<= 1) {
+        const double y = __shfl_up(cum, o);
+        if (lane >= o) cum += y;
       }
-    }
-    if (j >= 0) {
-      pick[e] = j;
-      s_left = tot - pj;
-      if (!(pj > 0.0) || !(tot - pj > 0.0)) s_bad = 1;  // an empty donor, or none left
+      cum += __shfl(before, src);
+      const uint64_t hit = __builtin_amdgcn_ballot_w64(below && cum > r);
+      // (no hit: nothing before k - 1, whose thread this is)
+      const int at = hit ? __builtin_ctzll(hit) : last - c0;
+      const double pj = __shfl(x, at);
+      if (own) {
+        pick[e] = c0 + at;
+        s_left = tot - pj;
+        if (!(pj > 0.0) || !(tot - pj > 0.0)) s_bad = 1;  // an empty donor, or none left
+#pragma unroll
+        for (int i = 0; i < PT; i++) p[i] = i == at ? 0.f : p[i];
+      }
     }
     __syncthreads();
     s = yk_split_scale<PT>(p, 1.0 / s_left);

@@ -527,3 +527,27 @@ def test_small_k_overflow_and_nan(ya, oracle, nq, k):
         want = np.lexsort((np.arange(nb), np.where(np.isnan(dist), np.inf, dist)))[:k]
         assert np.array_equal(gi[i], want), i
     assert (gi[-1] == -1).all()
+
+
+@pytest.mark.parametrize("scale", [0, -60, 50])
+@pytest.mark.parametrize("d,nb", [(16, 1), (16, 31), (24, 50), (32, 256), (64, 300), (128, 33),
+                                  (128, 1024), (200, 300)])
+def test_k1_near_ties(ya, d, nb, scale):
+    """k = 1 where the block's minimum and its first row are found apart.
+    Points on a plane with small integer coordinates times 2^scale: every
+    distance is exact, most queries have several rows at the least distance
+    or one unit from it, and at 2^50 most distances are past 1e30 (no row).
+    The first of the nearest rows has to win, with its exact value; base sizes
+    around the 32-row blocks (rows past the base never win)."""
+    rng = np.random.default_rng(nb + d)
+    b = np.zeros((nb, d), np.float32)
+    q = np.zeros((300, d), np.float32)
+    b[:, [0, d - 1]] = 1400 - rng.integers(0, 12, (nb, 2))
+    q[:, [0, d - 1]] = 1400 - rng.integers(0, 12, (300, 2))
+    dist = ((q[:, None].astype(np.float64) - b) ** 2).sum(2) * 2.0 ** (2 * scale)
+    gi, gd = ya.knn(np.ldexp(q, scale), np.ldexp(b, scale), 1)
+    near = dist.min(1)
+    want = np.where(near < np.float32(1e30), dist.argmin(1), -1)
+    print("k=1 near ties: d", d, "nb", nb, "scale", scale, flush=True)
+    assert np.array_equal(gi[:, 0], want)
+    assert np.array_equal(gd[:, 0], np.where(want < 0, 1e30, near).astype(np.float32))

@@ -121,15 +121,19 @@ __device__ __forceinline__ void yk_reg_insert(uint64_t (&t)[R], uint64_t x) {
   t[0] = x < t[0] ? x : t[0];
 }
 
-// A lane's 16 row norms, in registers or (the LDS-staged kernel) read from
-// LDS where they are used: value i's norm is float 8 (i >> 2) + (i & 3) of
-// the lane half's block norms.
+// A lane's 16 row norms, in registers or (the kernels that stage them) read
+// from LDS where they are used: value i's norm is entry 8 (i >> 2) + (i & 3)
+// of the lane half's block norms.  dbl: the norm as a double, held as one in
+// LDS (a conversion per value and block less).
 struct YkNormRegs {
   float n[16];
   __device__ __forceinline__ float operator[](int i) const { return n[i]; }
+  __device__ __forceinline__ double dbl(int i) const { return n[i]; }
 };
 struct YkNormLds {
   const float *p;
+  const double *pd;
+  __device__ __forceinline__ double dbl(int i) const { return pd[8 * (i >> 2) + (i & 3)]; }
   __device__ __forceinline__ float operator[](int i) const { return p[8 * (i >> 2) + (i & 3)]; }
   __device__ __forceinline__ float pick(int is) const { return p[8 * (is >> 2) + (is & 3)]; }
 };
@@ -173,12 +177,21 @@ __device__ __forceinline__ int yk_pick16(const f32x16 &acc, const float (&m)[16]
 // first blocks go without: a wave runs the exact pass when any of its 64
 // lanes may improve, which at block j of a range happens with probability
 // about 1 - (1 - 1/(j+1))^64, so early blocks would pay for both.  The exact
-// pass takes the exact FP64-normed expression for all 16 values, branch-free,
-// in ascending row order with a strict '<' (the smallest index wins a tie).
+// pass takes the exact FP64-normed expression for all 16 values and their
+// minimum; where a lane improves, the first row of that value is looked up
+// (the smallest index wins a tie).  What counts is the number of vector
+// instructions: they do not overlap with the FP32 MFMAs of the SIMD's other
+// waves (d = 16, k = 256: the matrix unit busy 46% and vector instructions
+// issuing 58% of the cycles; the norms read as doubles and the row found after
+// the minimum: 8 sub-spaces of 1e6 points, 10 iterations 16.3 -> 15.4 ms).
+// Rows past the base are zeros with a norm of YK_FAR_NORM: no such value is
+// below 1e30, where bv starts.
 // (Picking out the lanes' one candidate by the approximations first, to
 // evaluate one exact value per lane, measured slower: 26.8 against 18.2 ms
 // for the 8 sub-spaces of 1e6 points, d = 16, k = 256, 10 iterations -- the
 // selects cost as much as the FP64 operations they replace.)
+#define YK_FAR_NORM 1e36f
+
 template <bool DOT, class Norms>
 __device__ __forceinline__ void yk_best1_block(const f32x16 &acc, const Norms &nn, double qnd,
                                                long bb, int h, bool test, float &bv, int &bi) {
@@ -201,27 +214,26 @@ __device__ __forceinline__ void yk_best1_block(const f32x16 &acc, const Norms &n
   }
   double qd = qnd;
   asm volatile("" : "+v"(qd));
-  // value i sits at row bb + 4 h + 8 (i >> 2) + (i & 3); values 0-7 and 8-15
-  // as two chains, the first also holding the earlier blocks' best.  (The
-  // fused form rounds as bn+qn - 2 acc does: 2 acc is exact, and where it
-  // would overflow the norms' sum has too.)
-  float b0 = bv, b1 = bv;
-  int o0 = -1, o1 = -1;
+  // value i sits at row bb + 4 h + 8 (i >> 2) + (i & 3).  (The fused form
+  // rounds as bn+qn - 2 acc does: 2 acc is exact, and where it would
+  // overflow the norms' sum has too.)
+  float v[16], mm = INFINITY;
 #pragma unroll
-  for (int i = 0; i < 8; i++) {
-    const float v0 = DOT ? acc[i] : __builtin_fmaf(-2.0f, acc[i], (float)(qd + (double)nn[i]));
-    const float v1 =
-        DOT ? acc[i + 8] : __builtin_fmaf(-2.0f, acc[i + 8], (float)(qd + (double)nn[i + 8]));
-    const bool t0 = v0 < b0, t1 = v1 < b1;
-    b0 = t0 ? v0 : b0;
-    o0 = t0 ? 8 * (i >> 2) + (i & 3) : o0;
-    b1 = t1 ? v1 : b1;
-    o1 = t1 ? 16 + 8 * (i >> 2) + (i & 3) : o1;
+  for (int i = 0; i < 16; i++) {
+    v[i] = DOT ? acc[i] : __builtin_fmaf(-2.0f, acc[i], (float)(qd + nn.dbl(i)));
+    mm = fminf(mm, v[i]);
   }
-  const bool t = b1 < b0;
-  bv = t ? b1 : b0;
-  const int bo = t ? o1 : o0;
-  if (bo >= 0) bi = (int)bb + 4 * h + bo;
+  if (!(mm < bv)) return;
+  int bo = 0;
+#pragma unroll
+  for (int i = 15; i >= 0; i--) bo = v[i] == mm ? 8 * (i >> 2) + (i & 3) : bo;
+  // (of a +0 and a -0, which only the dot product has, the first one's bits)
+  if (DOT && mm == 0.0f) {
+#pragma unroll
+    for (int i = 15; i >= 0; i--) mm = v[i] == 0.0f ? v[i] : mm;
+  }
+  bv = mm;
+  bi = (int)bb + 4 * h + bo;
 }
 
 // the largest of a lane's 16 row norms
@@ -647,6 +659,7 @@ yk_scan_f32_lds(ScanArgs a0) {
   using S = YkLdsShape<NCH>;
   constexpr int U = S::U, G = S::G, KL = S::KL, NL = S::NL, CST = S::CST;
   constexpr int ld = 16 * NCH, TQ = 128 * NB;
+  constexpr bool BEST1 = MODE != 3 && !WT;  // yk_best1_block
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, h = lane >> 5;
@@ -654,6 +667,7 @@ yk_scan_f32_lds(ScanArgs a0) {
   struct Shared {
     float4 tile[2][G * 32 * U];
     float norm[2][G * 32];
+    double normd[2][BEST1 ? G * 32 : 1];
     float wt[2][WT ? G * 32 : 1];
     uint64_t cstage[MODE == 3 ? 4 * NB * 64 * CST : 1];
     int item;
@@ -793,7 +807,7 @@ yk_scan_f32_lds(ScanArgs a0) {
           yk_load_lds16(rs, sm.tile[buf] + 64 * (4 * i + wave), voff[i]);
       if (tid < 32 * G) {
         const long nr = row + (tid >> 5) * bstep + (tid & 31);
-        if (!dot) ld_n = nr < nb32 ? a.bn[nr] : 0.f;
+        if (!dot) ld_n = nr < (BEST1 ? a.nb : nb32) ? a.bn[nr] : BEST1 ? YK_FAR_NORM : 0.f;
         if (WT) ld_w = nr < nb32 ? a.w[nr] : 0.f;
       }
     };
@@ -801,12 +815,14 @@ yk_scan_f32_lds(ScanArgs a0) {
     auto store = [&](int buf) {
       if (tid < 32 * G) {
         sm.norm[buf][tid] = ld_n;
+        if (BEST1) sm.normd[buf][tid] = (double)ld_n;
         if (WT) sm.wt[buf][tid] = ld_w;
       }
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
     };
 
-    auto block = [&](const float4 *tp, const float *np, const float *wp, long bb, bool test) {
+    auto block = [&](const float4 *tp, const float *np, const double *npd, const float *wp,
+                     long bb, bool test) {
       f32x16 acc[NB];
 #pragma unroll
       for (int j = 0; j < NB; j++)
@@ -835,15 +851,16 @@ yk_scan_f32_lds(ScanArgs a0) {
           }
         __builtin_amdgcn_sched_barrier(0);
       }
-      const YkNormLds nn = {np};
+      const YkNormLds nn = {np, npd};
 #pragma unroll
       for (int j = 0; j < NB; j++) {
         if constexpr (MODE != 3) {
+          if (!WT && !dot) {
+            yk_best1_block<false>(acc[j], nn, qnd[j], bb, h, test, bv[j], bi[j]);
+            continue;
+          }
           if (!WT && bb + 32 <= bend) {
-            if (dot)
-              yk_best1_block<true>(acc[j], nn, qnd[j], bb, h, test, bv[j], bi[j]);
-            else
-              yk_best1_block<false>(acc[j], nn, qnd[j], bb, h, test, bv[j], bi[j]);
+            yk_best1_block<true>(acc[j], nn, qnd[j], bb, h, test, bv[j], bi[j]);
             continue;
           }
         }
@@ -901,7 +918,7 @@ yk_scan_f32_lds(ScanArgs a0) {
           // (the value's weighted approximation less its error, against the
           // bound: a lane's one such value by itself, several by the loop)
           const float limw = lim + 1e-36f;
-          const YkNormLds ww = {wp};
+          const YkNormLds ww = {wp, nullptr};
           int cnt = 0, is = 0;
           float as = acc[j][0];
 #pragma unroll
@@ -934,6 +951,7 @@ yk_scan_f32_lds(ScanArgs a0) {
           const long bb = bbeg + ((long)st * G + g) * bstep;
           if (bb >= bend) break;
           block(sm.tile[buf] + (g * 32 + r) * U, sm.norm[buf] + g * 32 + 4 * h,
+                sm.normd[buf] + (BEST1 ? g * 32 + 4 * h : 0),
                 sm.wt[buf] + (WT ? g * 32 + 4 * h : 0), bb, st * G + g >= 48);
         }
       }
@@ -1854,7 +1872,7 @@ yk_bassign_res_kernel(BassignArgs a) {
   const int ibeg = xcd * a.per_xcd, iend = min(a.nuitems, ibeg + a.per_xcd);
   const int ld = a.ld;
   __shared__ float4 cfs[NBLK * 2 * NCH * 64];
-  __shared__ float4 nns[NBLK * 4 * 64];
+  __shared__ double nns[NBLK * 32];
   __shared__ int s_item;
   auto next_item = [&](int it) {
     __syncthreads();  // also: every wave is done with the staged centroids
@@ -1873,17 +1891,16 @@ yk_bassign_res_kernel(BassignArgs a) {
     // centroid fragments and norms, staged in LDS once for the workgroup
     // in the lanes' order: fragment entry (cb, half-chunk q, lane) holds row
     // 32 cb + r, dimensions 16 (q / 2) + 8 h + 4 (q % 2) .. + 3 (rows past kc
-    // clamped to the last, masked below); norm entry (cb, g, lane) rows
-    // 32 cb + 8 g + 4 h .. + 3
+    // are zeros of norm YK_FAR_NORM)
     for (int i = threadIdx.x; i < NBLK * 2 * NCH * 64; i += blockDim.x) {
       const int ln = i & 63, q = (i >> 6) % (2 * NCH), cb = (i >> 6) / (2 * NCH);
-      const float *row = cb0 + (long)min(32 * cb + (ln & 31), a.kc - 1) * ld + (ln >> 5) * 8;
-      cfs[i] = *(const float4 *)(row + 16 * (q >> 1) + 4 * (q & 1));
+      const int cr = 32 * cb + (ln & 31);
+      const float *row = cb0 + (long)cr * ld + (ln >> 5) * 8;
+      cfs[i] = cr < a.kc ? *(const float4 *)(row + 16 * (q >> 1) + 4 * (q & 1))
+                         : make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    for (int i = threadIdx.x; i < NBLK * 4 * 64; i += blockDim.x) {
-      const int ln = i & 63, g = (i >> 6) & 3, cb = i >> 8;
-      nns[i] = *(const float4 *)(cnb + 32 * cb + 8 * g + 4 * (ln >> 5));
-    }
+    for (int i = threadIdx.x; i < NBLK * 32; i += blockDim.x)
+      nns[i] = (double)(i < a.kc ? cnb[i] : YK_FAR_NORM);
     __syncthreads();
     const long step = 32L * nwave;
     long pb = p0 + 32L * wave;
@@ -1948,26 +1965,8 @@ yk_bassign_res_kernel(BassignArgs a) {
       int bi = -1;
 #pragma unroll
       for (int cb = 0; cb < NBLK; cb++) {
-        YkNormRegs nrm;
-        float (&nn)[16] = nrm.n;
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-          const float4 n4 = nns[(cb * 4 + g) * 64 + lane];
-          nn[4 * g] = n4.x; nn[4 * g + 1] = n4.y; nn[4 * g + 2] = n4.z; nn[4 * g + 3] = n4.w;
-        }
-        if (32 * cb + 32 <= a.kc) {
-          yk_best1_block<false>(acc[cb], nrm, qd, 32L * cb, h, false, bv, bi);
-        } else {
-#pragma unroll
-          for (int i = 0; i < 16; i++) {
-            const int bidx = 32 * cb + 8 * (i >> 2) + 4 * h + (i & 3);
-            const float v = (float)(qd + (double)nn[i]) - 2.0f * acc[cb][i];
-            if (bidx < a.kc && v < bv) {
-              bv = v;
-              bi = bidx;
-            }
-          }
-        }
+        const YkNormLds nn = {nullptr, nns + 32 * cb + 4 * h};
+        yk_best1_block<false>(acc[cb], nn, qd, 32L * cb, h, false, bv, bi);
       }
       const float ov = __shfl_xor(bv, 32);
       const int oi = __shfl_xor(bi, 32);

@@ -170,14 +170,16 @@ __global__ __launch_bounds__(1024) void yk_cs_scan_kernel(int *__restrict__ mat,
   if (t == 1023) offsets[k] = part[1023];
 }
 
-// Pass 3: wave w places segment w's points.  Per 64-point chunk (all the
-// segment's clusters loaded at once), a bitonic sort of the keys (cluster
-// << 6 | lane) puts the chunk's points with equal clusters next to each
-// other in lane order; a point's place in its cluster is the cluster's
-// start, plus the earlier segments' counts of it, plus this segment's
-// running count of it (LDS, per wave, updated chunk by chunk in order),
-// plus its rank in its run: the sort is stable.  The chunks' ranks are
-// computed first and their gathers and stores issued together.
+// Pass 3: wave w places segment w's points, 64 at a time (all the segment's
+// clusters loaded at once).  A point's place is the next free one of its
+// cluster for this segment (LDS, per wave: the cluster's start plus the earlier
+// segments' counts of it, advanced chunk by chunk in order) plus the number
+// of lanes below with the same cluster: the sort is stable.  The lanes of a
+// cluster are found by one ballot per bit of the cluster number, eleven at
+// most.  What bounds it is the serial work of a segment's wave (98 of them for
+// 1e5 points): with a bitonic sort of each chunk's clusters, 21 dependent
+// shuffles, the kernel took 22.6 us at k = 1,024 (21.6 us for 2e4 points,
+// k = 50), now 11.7 (5.3).
 __global__ __launch_bounds__(256) void yk_cs_scatter_kernel(const int *__restrict__ assign, long n,
                                                             int k, long nseg,
                                                             const int *__restrict__ mat,
@@ -189,50 +191,34 @@ __global__ __launch_bounds__(256) void yk_cs_scatter_kernel(const int *__restric
   const long seg = blockIdx.x * 4L + wave;
   if (seg >= nseg) return;
   int *run = lr + wave * k;
-  for (int c = lane; c < k; c += 64) run[c] = 0;
   const long p0 = seg * YK_CS_SEG;
-  unsigned key[NJ];
+  int a[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; j++) {
     const long p = p0 + 64 * j + lane;
-    const int a = p < n ? assign[p] : -1;
-    key[j] = (unsigned)a < (unsigned)k ? ((unsigned)a << 6) | (unsigned)lane : 0xffffffffu;
+    a[j] = p < n ? assign[p] : -1;
   }
-  int pos[NJ];
+  for (int c = lane; c < k; c += 64) run[c] = offsets[c] + mat[seg * k + c];
+  uint64_t same[NJ];  // the chunk's lanes of the lane's cluster
 #pragma unroll
-  for (int j = 0; j < NJ; j++) {
-    unsigned kk = key[j];
+  for (int j = 0; j < NJ; j++)
+    same[j] = __builtin_amdgcn_ballot_w64((unsigned)a[j] < (unsigned)k);
+  for (int b = 0; (k - 1) >> b; b++) {
 #pragma unroll
-    for (int size = 2; size <= 64; size <<= 1) {
-#pragma unroll
-      for (int stride = size >> 1; stride > 0; stride >>= 1) {
-        const unsigned other = __shfl_xor(kk, stride);
-        const bool up = (lane & size) == 0, lower = (lane & stride) == 0;
-        kk = (lower == up) ? min(kk, other) : max(kk, other);
-      }
+    for (int j = 0; j < NJ; j++) {
+      const uint64_t m = __builtin_amdgcn_ballot_w64(a[j] >> b & 1);
+      same[j] &= a[j] >> b & 1 ? m : ~m;
     }
-    key[j] = kk;
-    const bool valid = kk != 0xffffffffu;
-    const int c = (int)(kk >> 6);
-    const int prev = __shfl_up(c, 1), next = __shfl_down(c, 1);
-    const bool start = lane == 0 || prev != c, end = lane == 63 || next != c;
-    int st = start ? lane : 0;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(st, o);
-      if (lane >= o) st = max(st, v);
-    }
-    const int rank = lane - st;
-    int base = 0;
-    if (valid) base = run[c];
-    if (valid && end) run[c] = base + rank + 1;
-    pos[j] = base + rank;
   }
 #pragma unroll
   for (int j = 0; j < NJ; j++) {
-    if (key[j] == 0xffffffffu) continue;
-    const int c = (int)(key[j] >> 6);
-    perm[offsets[c] + mat[seg * k + c] + pos[j]] = (int)(p0 + 64 * j + (key[j] & 63));
+    if ((unsigned)a[j] >= (unsigned)k) continue;
+    const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(same[j] >> 32),
+                                               __builtin_amdgcn_mbcnt_lo((unsigned)same[j], 0u));
+    const int cnt = __popcll(same[j]);
+    const int pos = run[a[j]] + rank;
+    if (rank == cnt - 1) run[a[j]] = pos + 1;
+    perm[pos] = (int)(p0 + 64 * j + lane);
   }
 }
 
@@ -360,33 +346,37 @@ __global__ __launch_bounds__(256) void yk_segsum_kernel(const float *__restrict_
 // (one per lane; nsl = ceil(d / 64) waves per cluster): at d = 128 twice the
 // waves of yk_segsum_kernel for the same rows, each column still summed in
 // point order, so the bits are that kernel's.  No normalisation (that needs
-// the whole row in one wave).
+// the whole row in one wave).  Bound by the latency of a cluster's rows, so
+// 32 of them are in flight (eight: 29.8 us at n = 1e5, k = 1,024, d = 128 and
+// 27.8 us at n = 2e4, k = 50, d = 32; now 21.3 and 20.1).
 __global__ __launch_bounds__(256) void yk_segsum_cols_kernel(const float *__restrict__ v, int d,
                                                              int ld, int k, int nsl,
                                                              const int *__restrict__ offsets,
                                                              const int *__restrict__ perm,
                                                              float *__restrict__ cent) {
+  constexpr int B = 32;  // rows in flight
   const int lane = threadIdx.x & 63;
-  const long g = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const long g = (long)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (g >= (long)k * nsl) return;
   const long c = g / nsl;
   const int j = (int)(g % nsl) * 64 + lane;
-  const int jl = j < d ? j : 0;  // lanes past d load column 0 and discard it
+  const float *vj = v + (j < d ? j : 0);  // lanes past d load column 0 and discard it
   const int beg = offsets[c], end = offsets[c + 1];
   const double inv = 1.0 / (double)(end - beg);
   double s = 0.0;
+  int next = beg + lane < end ? perm[beg + lane] : 0;
   for (int pb = beg; pb < end; pb += 64) {
-    const int nb = end - pb < 64 ? end - pb : 64;
-    const int pidx = lane < nb ? perm[pb + lane] : 0;
-    int t = 0;
-    for (; t + 8 <= nb; t += 8) {
-      float x[8];
+    const int nb = end - pb < 64 ? end - pb : 64, pidx = next;
+    if (pb + 64 + lane < end) next = perm[pb + 64 + lane];
+    for (int t = 0; t < nb; t += B) {
+      float x[B];
+      // (past the cluster's end: its last row again, added as zero)
 #pragma unroll
-      for (int u = 0; u < 8; u++) x[u] = v[(long)__shfl(pidx, t + u) * ld + jl];
+      for (int u = 0; u < B; u++)
+        x[u] = vj[(long)__builtin_amdgcn_readlane(pidx, t + u < nb ? t + u : nb - 1) * ld];
 #pragma unroll
-      for (int u = 0; u < 8; u++) s += (double)x[u];
+      for (int u = 0; u < B; u++) s += t + u < nb ? (double)x[u] : 0.0;
     }
-    for (; t < nb; t++) s += (double)v[(long)__shfl(pidx, t) * ld + jl];
   }
   if (j < d) cent[c * ld + j] = (float)(s * inv);
 }

@@ -576,7 +576,7 @@ extern "C" int yk_kmeans_readback_checked(const int *counts, int k, int *counts_
 // norm, every element rounded to float: O(k) per empty cluster (64 us on the
 // host at k = 65,536, 1,865 clusters in one iteration: 120 of a 163 ms call).
 // One workgroup holds p in registers, thread t a run of elements in index
-// order, and takes the empty clusters one after the other: ~4 us each at
+// order, and takes the empty clusters one after the other: 3.9 us each at
 // k = 65,536, of which the normalisation's five instructions per element on
 // one CU are half.
 //
@@ -614,6 +614,26 @@ __device__ __forceinline__ double yk_split_scale(float (&p)[PT], double inv) {
   return s;
 }
 
+// inclusive scan over the wave's lanes: shifts inside the rows of 16 lanes,
+// then the rows' last lanes broadcast (data-parallel moves: a scan by
+// shuffles through LDS, six dependent round trips, took 0.5 us)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double yk_dpp_f64(double x) {
+  const uint64_t u = (uint64_t)__double_as_longlong(x);
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)u, CTRL, ROWS, 0xf, false);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), CTRL, ROWS, 0xf, false);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+__device__ __forceinline__ double yk_wave_scan_f64(double x) {
+  x += yk_dpp_f64<0x111, 0xf>(x);  // row_shr:1
+  x += yk_dpp_f64<0x112, 0xf>(x);  // row_shr:2
+  x += yk_dpp_f64<0x114, 0xf>(x);  // row_shr:4
+  x += yk_dpp_f64<0x118, 0xf>(x);  // row_shr:8
+  x += yk_dpp_f64<0x142, 0xa>(x);  // row_bcast:15 into rows 1 and 3
+  x += yk_dpp_f64<0x143, 0xc>(x);  // row_bcast:31 into rows 2 and 3
+  return x;
+}
+
 template <int PT>
 __global__ __launch_bounds__(1024) void yk_split_pick_kernel(const int *__restrict__ counts, int k,
                                                              const double *__restrict__ rd, int ne,
@@ -635,11 +655,7 @@ __global__ __launch_bounds__(1024) void yk_split_pick_kernel(const int *__restri
   }
   // inclusive scan over the threads (exact, see above); *tot: the total
   auto scan = [&](double x, double *tot) {
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const double y = __shfl_up(x, o);
-      if (lane >= o) x += y;
-    }
+    x = yk_wave_scan_f64(x);
     if (lane == 63) wsum[wave] = x;
     __syncthreads();
     double before = 0.0, all = 0.0;
@@ -684,13 +700,7 @@ __global__ __launch_bounds__(1024) void yk_split_pick_kernel(const int *__restri
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       const double x = lane < PT ? (double)s_run[lane] : 0.0;
       const bool below = lane < PT && c0 + lane < last;
-      double cum = below ? x : 0.0;
-#pragma unroll
-      for (int o = 1; o < (PT < 64 ? PT : 64); o <<= 1) {
-        const double y = __shfl_up(cum, o);
-        if (lane >= o) cum += y;
-      }
-      cum += __shfl(before, src);
+      const double cum = yk_wave_scan_f64(below ? x : 0.0) + __shfl(before, src);
       const uint64_t hit = __builtin_amdgcn_ballot_w64(below && cum > r);
       // (no hit: nothing before k - 1, whose thread this is)
       const int at = hit ? __builtin_ctzll(hit) : last - c0;

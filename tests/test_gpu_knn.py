@@ -551,3 +551,22 @@ def test_k1_near_ties(ya, d, nb, scale):
     print("k=1 near ties: d", d, "nb", nb, "scale", scale, flush=True)
     assert np.array_equal(gi[:, 0], want)
     assert np.array_equal(gd[:, 0], np.where(want < 0, 1e30, near).astype(np.float32))
+
+
+@pytest.mark.parametrize("nq,d,typ,weighted", [(512, 704, 2, False), (513, 688, 2, False),
+                                               (513, 704, 2, False), (600, 960, 16, False),
+                                               (530, 701, 2, True)])
+@pytest.mark.parametrize("k", [2, 16])
+def test_long_vectors_small_k_bitexact(ya, oracle, nq, d, typ, weighted, k):
+    """k <= 16 on both sides of the lines (704 padded dimensions, 512 queries)
+    past which the register lists answer alone.  Integer data (weights are
+    powers of two): the oracle's lists bit for bit."""
+    rng = np.random.default_rng(nq + d + k)
+    nb = 5003
+    b = rng.integers(0, 9, (nb, d)).astype(np.float32)
+    q = rng.integers(0, 9, (nq, d)).astype(np.float32)
+    w = 2.0 ** rng.integers(-2, 3, nb).astype(np.float32) if weighted else None
+    print("long small k", nq, d, typ, weighted, k, flush=True)
+    gi, gd = ya.knn(q, b, k, distance_type=typ, weights=w)
+    oi, od = oracle.knn_full(typ, b, q, k, w)
+    parity.check_knn(typ, q, b, k, gi, gd, oi, od, w=w, exact=True, label="long%d_%d_%d" % (nq, d, k))

@@ -1067,17 +1067,17 @@ __device__ void yk_block_bitonic(uint64_t *s, int p2) {
 }
 
 // The k smallest of each query's n keys (src + q*n), sorted: the end of the
-// register top-R scan, for the queries the filtered pass left (*flag != 0,
-// thr[q] != 0).
+// register top-R scan, for every query or (with flag and thr) those that the
+// filtered pass left (*flag != 0, thr[q] != 0).
 __global__ __launch_bounds__(256) void yk_sortsel_kernel(const uint64_t *__restrict__ src,
                                                          int n, int k, int p2, int *out_i,
                                                          float *out_d,
                                                          const uint64_t *__restrict__ thr,
                                                          const int *__restrict__ flag) {
   extern __shared__ uint64_t s[];
-  if (*flag == 0) return;
+  if (flag && *flag == 0) return;
   const long q = blockIdx.x;
-  if (thr[q] == 0) return;
+  if (thr && thr[q] == 0) return;
   const uint64_t *p = src + q * (long)n;
   for (int i = threadIdx.x; i < p2; i += blockDim.x) s[i] = i < n ? p[i] : YK_KEY_NONE;
   __syncthreads();
@@ -1322,6 +1322,10 @@ static YkPlan yk_plan(int mode, long nq, long nb, int ld, bool weighted, long sa
   const long qt = (p.kind == YK_LDS2 ? 64 : 32) * p.waves;
   p.tiles = (int)((nq + qt - 1) / qt);
   p.slots = yk_resident_wgs((const void *)yk_scan_pick(mode, p.kind, ld, weighted), 64 * p.waves);
+  // the filtered scan of vectors too long for registers streams its queries
+  // too, from beyond the L2: three workgroups per CU (1e4 queries x 1e5, d =
+  // 960, k = 100: 37.9 ms; the four that fit 40.6, two 38.8)
+  if (mode == 3 && ld > 256 && p.waves == 4 && p.slots > 768) p.slots = 768;
   if (mode == 0 && p.kind != YK_STREAM && nb * ld <= (1L << 19) && nblocks >= 8) {
     // k = 1 over a base of at most 2 MB, which every XCD's L2 holds (the
     // k-means assign): even shares of the (tile, block) pairs, so that no CU
@@ -1598,6 +1602,33 @@ static int yk_knn_f32_check(int *type, long nq, long nb, int k) {
 
 // The FP32 search of nq queries, scratch from ar (nullptr: the grow-only
 // buffers).
+// k <= 16 by the register top-16 scan alone: many long vectors, where the
+// sketch's sixteenth of the MFMAs costs more than the lists' insertions save
+// (1e4 queries x 4e5, k = 10: d = 960 142 ms and 150 through the filter; 5,000
+// x 1e5, d = 512: 9.04 and 8.58; 100 x 1e6, d = 960: 6.16 and 4.52).
+static bool yk_knn_by_lists(int k, int ld, long nq) {
+  return k > 1 && k <= YK_REG_R && ld >= 704 && nq > 512;
+}
+static YkPlan yk_lists_plan(long nq, long nb, int ld, bool weighted, int cfg) {
+  return yk_plan(2, nq, nb, ld, weighted, 1, 1, 256, 16, cfg);
+}
+static int yk_knn_lists(ScanArgs a, int k, int *assign, float *dis, int cfg) {
+  const YkPlan p = yk_lists_plan(a.nq, a.nb, a.ld, a.w != nullptr, cfg);
+  const int n = p.nsplit * 2 * YK_REG_R;
+  void *buf;
+  YK_TRY(yk_scratch(nullptr, 3, sizeof(uint64_t) * a.nq * n, &buf));
+  a.part = (uint64_t *)buf;
+  YK_TRY(yk_launch_scan(2, p, a));
+  int p2 = 1;
+  while (p2 < n) p2 <<= 1;
+  int tok = yk_prof_begin(YK_PROF_MERGE);
+  hipLaunchKernelGGL(yk_sortsel_kernel, dim3((unsigned)a.nq), dim3(256), sizeof(uint64_t) * p2,
+                     yk_stream(), a.part, n, k, p2, assign, dis, nullptr, nullptr);
+  yk_prof_end(tok);
+  YK_HIP(hipGetLastError());
+  return YK_OK;
+}
+
 static int yk_knn_f32_run(int type, long nq, long nb, int d, int k, const float *q,
                           const double *qn, const float *b, const float *bn, const float *w,
                           int *assign, float *dis, YkArena *ar, int cfg = 0) {
@@ -1617,6 +1648,8 @@ static int yk_knn_f32_run(int type, long nq, long nb, int d, int k, const float 
   a.type = type;
   a.out_i = assign;
   a.out_d = dis;
+  // (without allocation the scratch is sized for the filtered search)
+  if (!ar && yk_knn_by_lists(k, a.ld, nq)) return yk_knn_lists(a, k, assign, dis, cfg);
   if (k > 1) return yk_knn_filtered(a, k, assign, dis, ar, cfg);
   const YkPlan p = yk_plan(0, nq, nb, a.ld, w != nullptr, 1, 1, 4096, 16, cfg);
   const long tq = p.kind == YK_LDS2 ? 256 : 128;
@@ -1700,8 +1733,10 @@ static int yk_f32_plan(const YkF32Call &call, int *cfg, int *ran) {
   const bool weighted = call.w != nullptr;
   for (int i = 0; i < ncand; i++) {
     const long nqb = call.nq < YK_LARGE_K_QB ? call.nq : YK_LARGE_K_QB;
-    if (call.k == 1) {
-      const YkPlan p = yk_plan(0, call.nq, call.nb, ld, weighted, 1, 1, 4096, 16, i);
+    if (call.k == 1 || yk_knn_by_lists(call.k, ld, call.nq)) {
+      const YkPlan p = call.k > 1
+                           ? yk_lists_plan(call.nq, call.nb, ld, weighted, i)
+                           : yk_plan(0, call.nq, call.nb, ld, weighted, 1, 1, 4096, 16, i);
       sig[i][0] = p.nsplit, sig[i][1] = p.brange, sig[i][2] = 0;
     } else {
       const YkPlan pa = yk_sketch_plan(nqb, call.nb, ld, weighted, call.k, i);

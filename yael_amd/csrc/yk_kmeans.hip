@@ -859,9 +859,9 @@ extern "C" int yk_kpp_update(const float *v, long n, int d, const double *vn, lo
 // present) adds the counts, or takes the workgroup's places in the node's
 // list, where LDS atomics hand them out.  (A global atomic per point queues
 // at a level of few nodes: 1e6 points through two levels of 32 children,
-// d = 128: 28.1 of the descent's 28.8 ms; the whole descent now 0.575 ms.)  Levels of more than
-// YK_HQ_LDS_NODES nodes (a 32 KB table) keep the atomic per point: their
-// addresses are many.
+// d = 128: 28.1 of the descent's 28.8 ms; the whole descent now 0.44 ms.)
+// Levels of more than YK_HQ_LDS_NODES nodes (a 32 KB table) keep the atomic
+// per point: their addresses are many.
 #define YK_HQ_LDS_NODES 8192
 #define YK_HQ_SEG 4096  // points per workgroup: 16 per thread
 

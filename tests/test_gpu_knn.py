@@ -570,3 +570,35 @@ def test_long_vectors_small_k_bitexact(ya, oracle, nq, d, typ, weighted, k):
     gi, gd = ya.knn(q, b, k, distance_type=typ, weights=w)
     oi, od = oracle.knn_full(typ, b, q, k, w)
     parity.check_knn(typ, q, b, k, gi, gd, oi, od, w=w, exact=True, label="long%d_%d_%d" % (nq, d, k))
+
+
+@pytest.mark.parametrize("nq,d", [(64, 40), (65, 40), (300, 40), (5, 200), (70, 270)])
+@pytest.mark.parametrize("nb", [3000, 4096, 4097, 20000])
+@pytest.mark.parametrize("k", [10, 60])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_minus_infinity_is_a_distance(ya, nq, d, nb, k, weighted):
+    """Half of the base at -inf (a component of -inf under the dot product, or
+    a weight of -inf), or five rows of it: -inf is the least of the values, so
+    the starting bound of the filtered pass may be -inf itself, and the rows
+    at it are returned, lowest index first.  Query counts on both sides of 64,
+    base sizes on both sides of a candidate list's 4,096 places."""
+    rng = np.random.default_rng(nb + nq + k)
+    b = rng.integers(1, 20, (nb, d)).astype(np.float32)
+    q = rng.integers(1, 20, (nq, d)).astype(np.float32)
+    q[:, 0] = 30  # no row at distance 0, whose weighted value would be NaN
+    for low in (nb // 2, 5):
+        rows = np.sort(rng.permutation(nb)[:low])
+        if weighted:
+            typ, w, bb = 2, np.ones(nb, np.float32), b
+            w[rows] = -np.inf
+            dist = ((q * q).sum(1)[:, None] + (b * b).sum(1)[None]) - 2 * (q @ b.T)
+        else:
+            typ, w, bb = 16, None, b.copy()
+            bb[rows, 7] = -np.inf
+            dist = q @ b.T
+        dist[:, rows] = -np.inf
+        print("-inf", nq, d, nb, k, "weighted" if weighted else "dot", "rows", low, flush=True)
+        gi, gd = ya.knn(q, bb, k, distance_type=typ, weights=w)
+        want = np.argsort(dist, axis=1, kind="stable")[:, :k]
+        assert np.array_equal(gi, want)
+        assert np.array_equal(gd, np.take_along_axis(dist, want, 1))

@@ -758,7 +758,9 @@ yk_scan_f32_lds(ScanArgs a0) {
       bi[j] = -1;
       ncs[j] = 0;
       // MODE 3: the bound's value (its row is looked up where a value equals
-      // it); 0: the query is already final
+      // it); a query that is already final (T = 0), or past the last one, has
+      // -inf here, which a bound's value may be too: a value equal to it
+      // enters by its whole key only (no key is <= 0)
       const uint64_t T = MODE == 3 ? a.thr[qrow[j]] : 0;
       Tv[j] = T == 0 || !qok[j] ? -INFINITY
                                 : (T == YK_KEY_NONE ? INFINITY : yk_fkey_inv((uint32_t)(T >> 32)));
@@ -880,9 +882,9 @@ yk_scan_f32_lds(ScanArgs a0) {
               bv[j] = v;
               bi[j] = (int)bidx;
             }
-          } else if (bidx < bend && v <= Tv[j] && Tv[j] > -INFINITY) {  // (drops NaN)
+          } else if (bidx < bend && v <= Tv[j]) {  // (drops NaN)
             const uint64_t key = yk_key(v, (int)bidx);
-            if (v < Tv[j] || key <= a.thr[qrow[j]]) {
+            if (v < Tv[j] || (qok[j] && key <= a.thr[qrow[j]])) {
               const int n = ncs[j];
               cs[(j * 64 + lane) * CST + n] = key;
               if (n + 1 == CST) {
@@ -904,13 +906,14 @@ yk_scan_f32_lds(ScanArgs a0) {
             if (lim < INFINITY) continue;
           }
           // m_i <= th for every value that may enter: qf + m_i - slack <=
-          // lim, with twice the slack for the roundings of this line
+          // lim, with twice the slack for the roundings of this line (an
+          // infinite lim: no such line, every value is tested)
           int is;
           float as;
           const int cnt = yk_pick16(acc[j], m, dot ? lim : lim - qf + 2.0f * slack, is, as);
           if (cnt == 1) {
             enter(exact(as, nn.pick(is)), is);
-          } else if (cnt > 1 || !(lim < INFINITY)) {
+          } else if (cnt > 1 || !(fabsf(lim) < INFINITY)) {
 #pragma unroll
             for (int i = 0; i < 16; i++) enter(exact(acc[j][i], nn[i]), i);
           }

@@ -602,3 +602,36 @@ def test_minus_infinity_is_a_distance(ya, nq, d, nb, k, weighted):
         want = np.argsort(dist, axis=1, kind="stable")[:, :k]
         assert np.array_equal(gi, want)
         assert np.array_equal(gd, np.take_along_axis(dist, want, 1))
+
+
+@pytest.mark.parametrize("nq", [5, 100, 300])
+@pytest.mark.parametrize("k", [2, 16])
+def test_small_k_list_overflow(ya, nq, k):
+    """k <= 16 with more rows strictly below a query's starting bound than its
+    candidate list holds (4,096): 6,000 near rows, none of them in the blocks
+    that the sketch samples (every 16th block of 32 rows at this size), so the
+    register top-16 scan queued behind answers.  Every other query has 64 near
+    rows in sampled blocks of their own, is answered by the first pass and
+    shares its wave with the overflowing ones."""
+    rng = np.random.default_rng(k + nq)
+    nb, d, cap, near = 40000, 24, 4096, 64
+    b = rng.integers(100, 200, (nb, d)).astype(np.float32)
+    block = np.arange(nb) // 32
+    sampled = block % 16 == 0
+    rows = rng.permutation(np.flatnonzero(~sampled))[:6000]
+    b[rows] = rng.integers(0, 3, (len(rows), d))
+    at = 32 * rng.permutation(np.flatnonzero(np.arange(nb // 32) % 16 == 0))[:near]
+    b[at + rng.integers(0, 32, near)] = 300 + rng.integers(0, 2, (near, d))
+    q = rng.integers(0, 2, (nq, d)).astype(np.float32)
+    q[1::2] += 300
+    dist = (q * q).sum(1)[:, None] + (b * b).sum(1)[None] - 2 * (q @ b.T)  # exact
+    for i in range(nq):
+        if i % 2 == 0:  # below every sampled row, so below any bound from them
+            assert (dist[i] < dist[i, sampled].min()).sum() > cap
+        else:  # a row in each of 64 blocks: k subsets' minima or more are theirs
+            assert (dist[i] <= np.sort(dist[i, sampled])[near - 1]).sum() == near
+    print("list overflow", nq, k, flush=True)
+    gi, gd = ya.knn(q, b, k)
+    want = np.argsort(dist, axis=1, kind="stable")[:, :k]
+    assert np.array_equal(gi, want)
+    assert np.array_equal(gd, np.take_along_axis(dist, want, 1))

@@ -1163,19 +1163,22 @@ __device__ __forceinline__ void yk_cand_topk(const uint64_t *p, int m, int n, in
 // admits, any bound) gets no bound, its count reset and the flag: its next
 // pass admits every value (and overflows, the overflow's bound then being a
 // proven one); a query with fewer than k keys and no bound has no more to
-// find.  (The keys are held in registers and the k-th found by ballot
+// find.  `last`: no scan follows, so every query's outputs are written here
+// (the caller knows that no list overflows, and that the bound admits k keys).
+// (The keys are held in registers and the k-th found by ballot
 // counts, as in the precision form: 1e4 lists of ~700 keys, k = 100, 0.049
 // -> 0.012 ms against a workgroup's bitonic sort per query.)
 template <int E2>
 __global__ __launch_bounds__(256) void yk_select_kernel(const uint64_t *__restrict__ cand, long nq,
                                                         int *cnt, uint64_t *thr, int k,
-                                                        int *out_i, float *out_d, int *flag) {
+                                                        int *out_i, float *out_d, int *flag,
+                                                        int last) {
   __shared__ uint64_t lds[4][64 * E2];
   const long q = blockIdx.x * 4L + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (q >= nq || thr[q] == 0) return;
   const int n = cnt[q];
-  if (n < k && thr[q] != YK_KEY_NONE) {
+  if (!last && n < k && thr[q] != YK_KEY_NONE) {
     if (lane == 0) {
       thr[q] = YK_KEY_NONE;
       cnt[q] = 0;
@@ -1467,7 +1470,8 @@ static int yk_thr(const uint64_t *src, long nq, int n, int m, int need, uint64_t
   return YK_OK;
 }
 
-static int yk_select(const ScanArgs &a, uint64_t *thr, int k, int *assign, float *dis, int *flag) {
+static int yk_select(const ScanArgs &a, uint64_t *thr, int k, int *assign, float *dis, int *flag,
+                     int last) {
   const dim3 grid((unsigned)((a.nq + 3) / 4)), block(256);
   int tok = yk_prof_begin(YK_PROF_MERGE);
   auto kern = k <= 64    ? yk_select_kernel<1>
@@ -1475,7 +1479,7 @@ static int yk_select(const ScanArgs &a, uint64_t *thr, int k, int *assign, float
               : k <= 512 ? yk_select_kernel<8>
                          : yk_select_kernel<16>;
   hipLaunchKernelGGL(kern, grid, block, 0, yk_stream(), a.cand, a.nq, a.cnt, thr, k, assign, dis,
-                     flag);
+                     flag, last);
   yk_prof_end(tok);
   YK_HIP(hipGetLastError());
   return YK_OK;
@@ -1563,11 +1567,16 @@ static int yk_knn_filtered(ScanArgs base, int k, int *assign, float *dis, YkAren
     a.cnt = cnt;
     a.cand = (uint64_t *)vcand;
     int tries = 0;
+    // k <= 16 and a base that fits a list: no list overflows, and the proven
+    // bound leaves no query short (the sketch and the filtered scan evaluate
+    // the same expression), so the queued scan and its sort would find the flag
+    // unset: two launches, 3.3 of the 35 - 55 us of such a search
+    const bool last = small && a.nb <= YK_CAND_CAP;
     for (;;) {
       YK_TRY(yk_launch_scan(3, pb, a));
-      YK_TRY(yk_select(a, thr, k, assign + q0 * k, dis + q0 * k, flag));
-      if (small) {  // (C) what is left, if anything (a base that fits a list leaves nothing)
-        if (a.nb <= YK_CAND_CAP) break;
+      YK_TRY(yk_select(a, thr, k, assign + q0 * k, dis + q0 * k, flag, last));
+      if (last) break;
+      if (small) {  // (C) what is left, if anything
         a.flag = flag;
         YK_TRY(yk_launch_scan(2, pc, a));
         const int n = pc.nsplit * 2 * YK_REG_R;

@@ -635,3 +635,29 @@ def test_small_k_list_overflow(ya, nq, k):
     want = np.argsort(dist, axis=1, kind="stable")[:, :k]
     assert np.array_equal(gi, want)
     assert np.array_equal(gd, np.take_along_axis(dist, want, 1))
+
+
+@pytest.mark.parametrize("nq,nb,d", [(200, 38743, 4096), (200, 38744, 4096), (128, 61000, 4096),
+                                     (129, 60066, 4090), (513, 5003, 704)])
+@pytest.mark.parametrize("k", [2, 16])
+@pytest.mark.parametrize("typ,weighted", [(2, False), (16, False), (2, True)])
+def test_long_vectors_lists_line(ya, nq, nb, d, k, typ, weighted):
+    """k <= 16 on both sides of the line past which the register lists answer
+    alone (more than 128 queries, nq nb ld^2 of 1.3e14).  Integer data (weights
+    are powers of two), so every value is exact in FP32: the k least by (value,
+    index)."""
+    rng = np.random.default_rng(nq + nb + d + k)
+    b = rng.integers(0, 9, (nb, d)).astype(np.float32)
+    q = rng.integers(0, 9, (nq, d)).astype(np.float32)
+    dist = q @ b.T
+    if typ == 2:
+        dist = ((q * q).sum(1)[:, None] + (b * b).sum(1)[None]) - 2 * dist
+    w = None
+    if weighted:
+        w = 2.0 ** rng.integers(-2, 3, nb).astype(np.float32)
+        dist *= w
+    print("lists line", nq, nb, d, k, typ, weighted, flush=True)
+    gi, gd = ya.knn(q, b, k, distance_type=typ, weights=w)
+    want = np.argsort(dist, axis=1, kind="stable")[:, :k]
+    assert np.array_equal(gi, want)
+    assert np.array_equal(gd, np.take_along_axis(dist, want, 1))

@@ -93,3 +93,28 @@ def test_noalloc_rejects_what_the_search_rejects():
         assert L.yk_last_error()
     for x in (bs, qs, oi, od):
         x.free()
+
+
+def test_noalloc_lists_in_passes():
+    """Long vectors, k <= 16, in two passes of the register lists: 1,024
+    queries, which fill the array, and the 76 left over."""
+    from yael_amd.device import DeviceSet
+    rng = np.random.default_rng(5)
+    nq, nb, d, k = 1100, 131072, 1024, 10
+    print("case lists in passes", nq, nb, d, k, flush=True)
+    b = rng.random((nb, d), dtype=np.float32)
+    q = rng.random((nq, d), dtype=np.float32)
+    bs, qs = DeviceSet(b), DeviceSet(q)
+    bs.compute_norms()
+    qs.compute_norms()
+    want_i, want_d = _search("yk_knn_f32", 2, qs, bs, k)
+    got_i, got_d = _search("yk_knn_f32_noalloc", 2, qs, bs, k)
+    bs.free()
+    qs.free()
+    assert np.array_equal(got_i, want_i)
+    assert np.array_equal(got_d.view(np.int32), want_d.view(np.int32))
+    # and 64-bit distances of a few queries
+    for i in (0, 1023, 1024, 1099):
+        dist = ((b - q[i]).astype(np.float64) ** 2).sum(1)
+        near = np.argsort(dist, kind="stable")[:k]
+        assert np.allclose(dist[got_i[i]], dist[near], rtol=1e-5)

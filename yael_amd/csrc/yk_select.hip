@@ -1612,23 +1612,31 @@ static int yk_knn_f32_check(int *type, long nq, long nb, int k) {
   return nq <= 0 ? 1 : YK_OK;
 }
 
-// The FP32 search of nq queries, scratch from ar (nullptr: the grow-only
-// buffers).
-// k <= 16 by the register top-16 scan alone: many long vectors, where the
-// sketch's sixteenth of the MFMAs costs more than the lists' insertions save
-// (1e4 queries x 4e5, k = 10: d = 960 142 ms and 150 through the filter; 5,000
-// x 1e5, d = 512: 9.04 and 8.58; 100 x 1e6, d = 960: 6.16 and 4.52).
-static bool yk_knn_by_lists(int k, int ld, long nq) {
-  return k > 1 && k <= YK_REG_R && ld >= 704 && nq > 512;
+// k <= 16 by the register top-16 scan alone: large searches of long vectors,
+// where the sketch's sixteenth of the MFMAs and the filter's fewer waves cost
+// more than the lists' insertions save.  Both routes stream from memory there
+// (d > 256); a tile of 128 queries or fewer, and d <= 256, are the filter's.
+// The line is where the two meet, in 538 shapes of 65 .. 10,000 queries, 2e4 ..
+// 1e6 rows and d = 272 .. 2,048, k = 10 (2 and 16 alike), filter and lists in ms:
+//   d = 400: 4,000 x 1e5 5.32 / 5.63, 10,000 x 4e5 60.1 / 57.8
+//   d = 640: 1,000 x 4e5 8.18 / 8.17, 4,000 x 4e5 41.7 / 38.5
+//   d = 960: 1,000 x 1e5 3.30 / 3.82, 4,000 x 1e5 14.95 / 14.07
+//   d = 1536: 1,000 x 1e5 5.46 / 5.98, 768 x 4e5 16.3 / 15.4
+// Past it the lists take 0.91 - 1.0 of the filter's time, before it 1.0 - 3.6
+// times as long; the rule is 0.4% from the faster of the two on average and
+// at worst 8% (160 queries, one wave of a second tile).
+static bool yk_knn_by_lists(int k, int ld, long nq, long nb) {
+  return k > 1 && k <= YK_REG_R && ld > 256 && nq > 128 &&
+         (double)nq * (double)nb * ld * ld >= 1.3e14;
 }
 static YkPlan yk_lists_plan(long nq, long nb, int ld, bool weighted, int cfg) {
   return yk_plan(2, nq, nb, ld, weighted, 1, 1, 256, 16, cfg);
 }
-static int yk_knn_lists(ScanArgs a, int k, int *assign, float *dis, int cfg) {
+static int yk_knn_lists(ScanArgs a, int k, int *assign, float *dis, YkArena *ar, int cfg) {
   const YkPlan p = yk_lists_plan(a.nq, a.nb, a.ld, a.w != nullptr, cfg);
   const int n = p.nsplit * 2 * YK_REG_R;
   void *buf;
-  YK_TRY(yk_scratch(nullptr, 3, sizeof(uint64_t) * a.nq * n, &buf));
+  YK_TRY(yk_scratch(ar, 3, sizeof(uint64_t) * a.nq * n, &buf));
   a.part = (uint64_t *)buf;
   YK_TRY(yk_launch_scan(2, p, a));
   int p2 = 1;
@@ -1641,9 +1649,11 @@ static int yk_knn_lists(ScanArgs a, int k, int *assign, float *dis, int cfg) {
   return YK_OK;
 }
 
+// The FP32 search of nq queries, scratch from ar (nullptr: the grow-only
+// buffers); lists: yk_knn_by_lists
 static int yk_knn_f32_run(int type, long nq, long nb, int d, int k, const float *q,
                           const double *qn, const float *b, const float *bn, const float *w,
-                          int *assign, float *dis, YkArena *ar, int cfg = 0) {
+                          int *assign, float *dis, bool lists, YkArena *ar, int cfg = 0) {
   if (k > YK_KMAX) {  // beyond the on-chip selection: distance rows + radix select
     if (ar) return yk_set_error(YK_EINVAL, "k=%d > %d needs allocated scratch", k, YK_KMAX);
     return yk_knn_bigk(type, nq, nb, d, k, q, qn, b, bn, w, assign, dis);
@@ -1660,8 +1670,7 @@ static int yk_knn_f32_run(int type, long nq, long nb, int d, int k, const float 
   a.type = type;
   a.out_i = assign;
   a.out_d = dis;
-  // (without allocation the scratch is sized for the filtered search)
-  if (!ar && yk_knn_by_lists(k, a.ld, nq)) return yk_knn_lists(a, k, assign, dis, cfg);
+  if (lists) return yk_knn_lists(a, k, assign, dis, ar, cfg);
   if (k > 1) return yk_knn_filtered(a, k, assign, dis, ar, cfg);
   const YkPlan p = yk_plan(0, nq, nb, a.ld, w != nullptr, 1, 1, 4096, 16, cfg);
   const long tq = p.kind == YK_LDS2 ? 256 : 128;
@@ -1703,7 +1712,7 @@ struct YkF32Call {
 static int yk_f32_call(void *p) {
   const YkF32Call &c = *(const YkF32Call *)p;
   return yk_knn_f32_run(c.type, c.nq, c.nb, c.d, c.k, c.q, c.qn, c.b, c.bn, c.w, c.assign, c.dis,
-                        nullptr, c.cfg);
+                        yk_knn_by_lists(c.k, yk_ld(c.d), c.nq, c.nb), nullptr, c.cfg);
 }
 
 // log2 bucket of a size (shape classes of the tuning cache)
@@ -1745,7 +1754,7 @@ static int yk_f32_plan(const YkF32Call &call, int *cfg, int *ran) {
   const bool weighted = call.w != nullptr;
   for (int i = 0; i < ncand; i++) {
     const long nqb = call.nq < YK_LARGE_K_QB ? call.nq : YK_LARGE_K_QB;
-    if (call.k == 1 || yk_knn_by_lists(call.k, ld, call.nq)) {
+    if (call.k == 1 || yk_knn_by_lists(call.k, ld, call.nq, call.nb)) {
       const YkPlan p = call.k > 1
                            ? yk_lists_plan(call.nq, call.nb, ld, weighted, i)
                            : yk_plan(0, call.nq, call.nb, ld, weighted, 1, 1, 4096, 16, i);
@@ -1791,7 +1800,8 @@ extern "C" int yk_knn_f32(int type, long nq, long nb, int d, int k, const float 
   int cfg = 0, ran = 0;
   YK_TRY(yk_f32_plan(call, &cfg, &ran));
   if (ran) return YK_OK;
-  return yk_knn_f32_run(type, nq, nb, d, k, q, qn, b, bn, w, assign, dis, nullptr, cfg);
+  return yk_knn_f32_run(type, nq, nb, d, k, q, qn, b, bn, w, assign, dis,
+                        yk_knn_by_lists(k, yk_ld(d), nq, nb), nullptr, cfg);
 }
 
 // ---------------------------------------------------------------------------
@@ -1833,7 +1843,10 @@ static int yk_noalloc_region(char **out) {
 
 // Scratch bytes one yk_knn_f32_run over nq queries takes from a region (the
 // same plans and pieces as the run itself, each rounded up to 256 bytes).
-static size_t yk_knn_f32_need(long nq, long nb, int ld, bool weighted, int k) {
+static size_t yk_knn_f32_need(long nq, long nb, int ld, bool weighted, int k, bool lists) {
+  if (lists)
+    return yk_align256(sizeof(uint64_t) * nq * 2 * YK_REG_R *
+                       yk_lists_plan(nq, nb, ld, weighted, 0).nsplit);
   if (k == 1) {
     const YkPlan p = yk_plan(0, nq, nb, ld, weighted, 1, 1, 4096, 16, 0);
     if (p.units) return yk_align256(sizeof(uint64_t) * 2 * (p.kind == YK_LDS2 ? 256 : 128) * p.slots);
@@ -1862,12 +1875,17 @@ extern "C" int yk_knn_f32_noalloc(int type, long nq, long nb, int d, int k, cons
   // power-of-two pass (at most 16384 queries) whose scratch fits.  Each
   // query's result depends only on that query, so the passes give the
   // single call's results.
+  // (the route is the first pass's for them all)
   long pass = 16384;
   const int ld = yk_ld(d);
-  while (pass > 32 && yk_knn_f32_need(pass < nq ? pass : nq, nb, ld, w != nullptr, k) >
-                          YK_NOALLOC_SCRATCH_BYTES)
-    pass >>= 1;
-  const size_t need = yk_knn_f32_need(pass < nq ? pass : nq, nb, ld, w != nullptr, k);
+  bool lists;
+  size_t need;
+  for (;; pass >>= 1) {
+    const long n = pass < nq ? pass : nq;
+    lists = yk_knn_by_lists(k, ld, n, nb);
+    need = yk_knn_f32_need(n, nb, ld, w != nullptr, k, lists);
+    if (need <= YK_NOALLOC_SCRATCH_BYTES || pass <= 32) break;
+  }
   if (need > YK_NOALLOC_SCRATCH_BYTES)
     return yk_set_error(YK_EINVAL,
                         "k=%d, nb=%ld needs %zu scratch bytes even for %ld queries at a time; "
@@ -1877,7 +1895,7 @@ extern "C" int yk_knn_f32_noalloc(int type, long nq, long nb, int d, int k, cons
     const long n = nq - q0 < pass ? nq - q0 : pass;
     YkArena ar = {region, (size_t)YK_NOALLOC_SCRATCH_BYTES, 0};
     YK_TRY(yk_knn_f32_run(type, n, nb, d, k, q + q0 * ld, qn ? qn + q0 : nullptr, b, bn, w,
-                          assign + q0 * k, dis + q0 * k, &ar));
+                          assign + q0 * k, dis + q0 * k, lists, &ar));
   }
   return YK_OK;
 }

@@ -1738,8 +1738,12 @@ static int yk_f32_plan(const YkF32Call &call, int *cfg, int *ran) {
   if ((double)call.nq * call.nb * call.d < (double)(1 << 29)) return YK_OK;
   const int kc = call.k == 1 ? 1 : call.k <= YK_REG_R ? 16 : 1 << yk_lg(call.k);
   char key[128];
-  snprintf(key, sizeof key, "f32:v2:t%d:k%d:ld%d:q%d:b%d", call.type, kc, yk_ld(call.d),
-           yk_lg(call.nq), yk_lg(call.nb));
+  // (a plan of one route, or of the weighted kernels, says nothing of the
+  // other's: both may meet within a bucket of sizes)
+  snprintf(key, sizeof key, "f32:v2:t%d:k%d:ld%d:q%d:b%d%s%s", call.type, kc, yk_ld(call.d),
+           yk_lg(call.nq), yk_lg(call.nb),
+           yk_knn_by_lists(call.k, yk_ld(call.d), call.nq, call.nb) ? ":lists" : "",
+           call.w ? ":w" : "");
   if (yk_tune_get(key, cfg)) {
     if (*cfg < 0 || *cfg >= YK_NCFG) *cfg = 0;
     return YK_OK;

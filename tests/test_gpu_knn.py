@@ -638,12 +638,13 @@ def test_small_k_list_overflow(ya, nq, k):
 
 
 @pytest.mark.parametrize("nq,nb,d", [(200, 38743, 4096), (200, 38744, 4096), (128, 61000, 4096),
-                                     (129, 60066, 4090), (513, 5003, 704)])
+                                     (129, 60066, 4090), (129, 21254, 4096), (192, 14281, 4096),
+                                     (513, 5003, 704)])
 @pytest.mark.parametrize("k", [2, 16])
 @pytest.mark.parametrize("typ,weighted", [(2, False), (16, False), (2, True)])
 def test_long_vectors_lists_line(ya, nq, nb, d, k, typ, weighted):
     """k <= 16 on both sides of the line past which the register lists answer
-    alone (more than 128 queries, nq nb ld^2 of 1.3e14).  Integer data (weights
+    alone (more than 128 queries; nq nb ld^2 of 1.3e14, up to 192 queries 4.6e13).  Integer data (weights
     are powers of two), so every value is exact in FP32: the k least by (value,
     index)."""
     rng = np.random.default_rng(nq + nb + d + k)

@@ -1616,18 +1616,23 @@ static int yk_knn_f32_check(int *type, long nq, long nb, int k) {
 // where the sketch's sixteenth of the MFMAs and the filter's fewer waves cost
 // more than the lists' insertions save.  Both routes stream from memory there
 // (d > 256); a tile of 128 queries or fewer, and d <= 256, are the filter's.
-// The line is where the two meet, in 538 shapes of 65 .. 10,000 queries, 2e4 ..
+// The line is where the two meet, in 518 shapes of 65 .. 10,000 queries, 2e4 ..
 // 1e6 rows and d = 272 .. 2,048, k = 10 (2 and 16 alike), filter and lists in ms:
 //   d = 400: 4,000 x 1e5 5.32 / 5.63, 10,000 x 4e5 60.1 / 57.8
 //   d = 640: 1,000 x 4e5 8.18 / 8.17, 4,000 x 4e5 41.7 / 38.5
 //   d = 960: 1,000 x 1e5 3.30 / 3.82, 4,000 x 1e5 14.95 / 14.07
 //   d = 1536: 1,000 x 1e5 5.46 / 5.98, 768 x 4e5 16.3 / 15.4
 // Past it the lists take 0.91 - 1.0 of the filter's time, before it 1.0 - 3.6
-// times as long; the rule is 0.4% from the faster of the two on average and
-// at worst 8% (160 queries, one wave of a second tile).
+// times as long.  Up to 192 queries the second tile's idle waves cost the
+// filter's two scans more than the lists' one, and the line lies lower (124
+// shapes more):
+//   144 queries: 4e5, d = 960 3.67 / 3.36, 1e6, d = 704 6.60 / 6.18
+//   192 queries: 1e5, d = 1536 1.63 / 1.88, 4e5, d = 1536 5.91 / 5.58
+// Over all of them the rule is 0.5% from the faster route on average, 12% at
+// worst (its own line: 129 queries x 2e5, d = 960).
 static bool yk_knn_by_lists(int k, int ld, long nq, long nb) {
   return k > 1 && k <= YK_REG_R && ld > 256 && nq > 128 &&
-         (double)nq * (double)nb * ld * ld >= 1.3e14;
+         (double)nq * (double)nb * ld * ld >= (nq <= 192 ? 4.6e13 : 1.3e14);
 }
 static YkPlan yk_lists_plan(long nq, long nb, int ld, bool weighted, int cfg) {
   return yk_plan(2, nq, nb, ld, weighted, 1, 1, 256, 16, cfg);

@@ -15,8 +15,9 @@ hipStream_t yk_stream(void);
 int yk_read_small(void *dst, const void *src, size_t bytes);
 int yk_prof_setup(void);
 // Workgroups of `block` threads that fit on the whole device at once for
-// kernel `fn` (occupancy x CU count), at least 8 and a multiple of 8.
-int yk_resident_wgs(const void *fn, int block);
+// kernel `fn` (occupancy, at most `most` where given, x CU count), at least 8
+// and a multiple of 8.
+int yk_resident_wgs(const void *fn, int block, int most = 0);
 int yk_prof_begin(int slot);
 void yk_prof_end(int tok);
 

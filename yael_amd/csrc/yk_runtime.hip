@@ -566,16 +566,16 @@ extern "C" int yk_prof_get(int which, double *total_ms, long *count) {
 
 #define YK_OCC_CACHE 256
 static const void *g_occ_fn[YK_OCC_CACHE];
-static int g_occ_block[YK_OCC_CACHE], g_occ_val[YK_OCC_CACHE], g_occ_n = 0;
+static int g_occ_block[YK_OCC_CACHE], g_occ_val[YK_OCC_CACHE], g_occ_n = 0;  // val: per CU
 static int g_cu_count = 0;
 static pthread_mutex_t g_occ_mu = PTHREAD_MUTEX_INITIALIZER;
 
-int yk_resident_wgs(const void *fn, int block) {
+int yk_resident_wgs(const void *fn, int block, int most) {
   pthread_mutex_lock(&g_occ_mu);
-  int res = 0;
+  int per_cu = 0;
   for (int i = 0; i < g_occ_n; i++)
-    if (g_occ_fn[i] == fn && g_occ_block[i] == block) res = g_occ_val[i];
-  if (!res) {
+    if (g_occ_fn[i] == fn && g_occ_block[i] == block) per_cu = g_occ_val[i];
+  if (!per_cu) {
     if (!g_cu_count) {
       hipDeviceProp_t p;
       if (hipGetDeviceProperties(&p, 0) == hipSuccess) {
@@ -585,22 +585,20 @@ int yk_resident_wgs(const void *fn, int block) {
         g_cu_count = 256;
       }
     }
-    int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, block, 0) != hipSuccess) {
       (void)hipGetLastError();  // consumed: one workgroup per CU is assumed instead
       per_cu = 1;
     }
     if (per_cu < 1) per_cu = 1;
-    res = per_cu * g_cu_count;
-    res = res < 8 ? 8 : res & ~7;
     if (g_occ_n < YK_OCC_CACHE) {
       g_occ_fn[g_occ_n] = fn;
       g_occ_block[g_occ_n] = block;
-      g_occ_val[g_occ_n++] = res;
+      g_occ_val[g_occ_n++] = per_cu;
     }
   }
+  const int res = (most > 0 && per_cu > most ? most : per_cu) * g_cu_count;
   pthread_mutex_unlock(&g_occ_mu);
-  return res;
+  return res < 8 ? 8 : res & ~7;
 }
 
 // ---------------------------------------------------------------------------

@@ -1327,11 +1327,12 @@ static YkPlan yk_plan(int mode, long nq, long nb, int ld, bool weighted, long sa
   }
   const long qt = (p.kind == YK_LDS2 ? 64 : 32) * p.waves;
   p.tiles = (int)((nq + qt - 1) / qt);
-  p.slots = yk_resident_wgs((const void *)yk_scan_pick(mode, p.kind, ld, weighted), 64 * p.waves);
   // the filtered scan of vectors too long for registers streams its queries
   // too, from beyond the L2: three workgroups per CU (1e4 queries x 1e5, d =
   // 960, k = 100: 37.9 ms; the four that fit 40.6, two 38.8)
-  if (mode == 3 && ld > 256 && p.waves == 4 && p.slots > 768) p.slots = 768;
+  const int most = mode == 3 && ld > 256 && p.waves == 4 ? 3 : 0;
+  p.slots = yk_resident_wgs((const void *)yk_scan_pick(mode, p.kind, ld, weighted), 64 * p.waves,
+                            most);
   if (mode == 0 && p.kind != YK_STREAM && nb * ld <= (1L << 19) && nblocks >= 8) {
     // k = 1 over a base of at most 2 MB, which every XCD's L2 holds (the
     // k-means assign): even shares of the (tile, block) pairs, so that no CU
@@ -2136,7 +2137,7 @@ int yk_batch_assign_res(int ninst, int d, int kc, int kpad, int chunk, const flo
   YK_TRY(yk_item_tickets(&a.tick));
   // (two workgroups per CU: a third, where the registers allow it, made an
   // iteration's assign 0.387 instead of 0.380 ms)
-  const int per_res = (int)min((long)yk_resident_wgs((const void *)kern, 256) / 8, 64L);
+  const int per_res = yk_resident_wgs((const void *)kern, 256, 2) / 8;
   // The update's chunk is chosen for the update; whole chunks as work items
   // left the last of ~1.4 rounds half empty (2e6 points, 1,094 chunks for 768
   // workgroups: 0.412 ms, now 0.380).  At least six items a workgroup, of

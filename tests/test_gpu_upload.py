@@ -47,3 +47,35 @@ def test_copies_roundtrip_and_pad_columns(ya, n, d):
     V.free()
     assert np.array_equal(back, x)
     assert np.array_equal(raw[:, :d], x) and not raw[:, d:].any()
+
+
+@pytest.mark.parametrize("n,d", [(1, 65), (500, 128), (600, 100), (2100, 128), (9001, 128),
+                                 (11000, 100), (50000, 128), (180001, 100)])
+def test_copies_of_pinned_host_memory(ya, n, d):
+    """Host memory from yk_host_alloc, below and above the sizes at which
+    pageable memory goes through the landing buffer (256 KB), the staging
+    threads (4 and 16 MB) and the dense pieces (64 MB), dense and padded."""
+    import ctypes
+    from yael_amd import device
+    L, vp = ya.lib(), ctypes.c_void_p
+    rng = np.random.default_rng(n + d)
+    x = rng.standard_normal((n, d)).astype(np.float32)
+    p = vp()
+    ya.check(L.yk_host_alloc(ctypes.byref(p), 2 * x.nbytes), "host_alloc")
+    src, dst = np.frombuffer((ctypes.c_char * (2 * x.nbytes)).from_address(p.value),
+                             np.float32).reshape(2, n, d)
+    src[:], dst[:] = x, 0
+    print("pinned n=%d d=%d (%.1f MB)" % (n, d, x.nbytes / 2**20), flush=True)
+    V = device.DeviceSet(shape=(n, d))
+    ya.check(L.yk_upload_vectors(V.vec.ptr, src.ctypes.data_as(vp), n, d), "upload")
+    ya.check(L.yk_download_vectors(dst.ctypes.data_as(vp), V.vec.ptr, n, d), "download")
+    raw = V.vec.to_host(np.float32, (n, V.ld))
+    assert np.array_equal(raw[:, :d], x) and not raw[:, d:].any()
+    assert np.array_equal(dst, x)
+    if V.ld == d:
+        dst[:] = 0
+        ya.check(L.yk_memcpy_d2h(dst.ctypes.data_as(vp), V.vec.ptr, x.nbytes), "d2h")
+        assert np.array_equal(dst, x)
+    V.free()
+    del src, dst
+    ya.check(L.yk_host_free(p), "host_free")

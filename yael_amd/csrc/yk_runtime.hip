@@ -145,11 +145,26 @@ extern "C" int yk_host_free(void *p) {
 #define YK_STAGE_MIN_UP ((size_t)16 << 20)
 static int yk_copy_staged(char *dev, char *host, size_t bytes, bool up);
 
+// Memory at p that HIP knows (pinned or mapped host memory, or a device's): the
+// DMA reaches it by itself, and a detour through the pinned buffers only costs
+// a host copy (to pinned memory, plain and staged: 4 MB 0.082 and 0.154 ms, 32
+// MB 0.60 and 0.80; 256 KB through the landing buffer 0.019 instead of 0.013).
+static bool yk_known_to_hip(const void *p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();  // consumed: ordinary host memory
+    return false;
+  }
+  return a.type != hipMemoryTypeUnregistered;
+}
+
 extern "C" int yk_memcpy_d2h(void *dst, const void *src, size_t bytes) {
   YK_TRY(yk_init());
   if (!bytes) return YK_OK;
-  if (bytes <= YK_READ_SMALL) return yk_read_small(dst, src, bytes);
-  if (bytes >= YK_STAGE_MIN_DOWN) return yk_copy_staged((char *)src, (char *)dst, bytes, false);
+  if (bytes <= 256 || (bytes <= YK_READ_SMALL && !yk_known_to_hip(dst)))
+    return yk_read_small(dst, src, bytes);
+  if (bytes >= YK_STAGE_MIN_DOWN && !yk_known_to_hip(dst))
+    return yk_copy_staged((char *)src, (char *)dst, bytes, false);
   YK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, g_stream));
   YK_HIP(hipStreamSynchronize(g_stream));
   return YK_OK;
@@ -379,14 +394,30 @@ static int yk_dense_buffer(size_t bytes, float **out) {
   return YK_OK;
 }
 
+// the rows by one 2-D copy: to pinned memory (256 KB 0.012 ms, in two steps
+// 0.029; 32 MB 0.55 and 0.67), and where no dense buffer is to be had
+static int yk_copy_2d(float *dev, float *host, long n, int d, bool up) {
+  const size_t dev_row = sizeof(float) * (size_t)yk_ld(d), row = sizeof(float) * (size_t)d;
+  if (up) {
+    YK_TRY(yk_memset(dev, 0, dev_row * (size_t)n));
+    YK_HIP(hipMemcpy2DAsync(dev, dev_row, host, row, row, n, hipMemcpyHostToDevice, g_stream));
+  } else {
+    YK_HIP(hipMemcpy2DAsync(host, row, dev, dev_row, row, n, hipMemcpyDeviceToHost, g_stream));
+  }
+  YK_HIP(hipStreamSynchronize(g_stream));
+  return YK_OK;
+}
+
 static int yk_dense_copy(float *dev, float *host, long n, int d, bool up) {
   const int ld = yk_ld(d);
+  const bool known = yk_known_to_hip(host);
+  if (known && !up) return yk_copy_2d(dev, host, n, d, false);
   const size_t row = sizeof(float) * (size_t)d;
   long step = (long)(YK_DENSE_BYTES / row);  // rows per copy
   if (step < 1) step = 1;
   if (step > n) step = n;
   float *buf;
-  YK_TRY(yk_dense_buffer(row * (size_t)step, &buf));
+  if (yk_dense_buffer(row * (size_t)step, &buf) != YK_OK) return yk_copy_2d(dev, host, n, d, up);
   for (long i = 0; i < n; i += step) {
     const long m = n - i < step ? n - i : step;
     const size_t bytes = row * (size_t)m;
@@ -398,7 +429,7 @@ static int yk_dense_copy(float *dev, float *host, long n, int d, bool up) {
       YK_TRY(yk_memcpy_d2h(host + i * d, buf, bytes));
       continue;
     }
-    if (bytes >= YK_STAGE_MIN_UP)
+    if (bytes >= YK_STAGE_MIN_UP && !known)
       YK_TRY(yk_copy_staged((char *)buf, (char *)(host + i * d), bytes, true));
     else
       YK_HIP(hipMemcpyAsync(buf, host + i * d, bytes, hipMemcpyHostToDevice, g_stream));
@@ -423,7 +454,8 @@ extern "C" int yk_upload_vectors(float *dst, const float *src, long n, int d) {
     pthread_mutex_unlock(&g_dense_mu);
     return rc;
   }
-  if (bytes >= YK_STAGE_MIN_UP) return yk_copy_staged((char *)dst, (char *)src, bytes, true);
+  if (bytes >= YK_STAGE_MIN_UP && !yk_known_to_hip(src))
+    return yk_copy_staged((char *)dst, (char *)src, bytes, true);
   YK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, g_stream));
   YK_HIP(hipStreamSynchronize(g_stream));
   return YK_OK;

@@ -152,3 +152,23 @@ def test_quantize_ordering_paths_vs_oracle(hk, tmp_path, nlevel, bf, d, n):
     v[n // 2] = np.nan
     want[n // 2] = -1
     assert np.array_equal(t.quantize(v), want)
+
+
+@pytest.mark.parametrize("nlevel,bf,n", [(3, 30, 1), (3, 30, 40), (4, 12, 129), (3, 90, 8163),
+                                         (3, 90, 8164)])
+def test_quantize_few_points_of_many_nodes(hk, tmp_path, nlevel, bf, n):
+    """Fewer points than a level's nodes, where the level has no more work
+    items than points (n), and each side of the size from which it is counted
+    by nodes (8,100 of them and one for every 128 points).  Integer trees and
+    points: the oracle's leaves."""
+    from oracle_bind import Oracle
+    rng = np.random.default_rng(nlevel * 1000 + n)
+    d = 8
+    levels = [np.rint(rng.uniform(0, 200, (bf ** (l + 1), d))).astype(np.float32)
+              for l in range(nlevel)]
+    v = np.rint(rng.uniform(0, 200, (n, d))).astype(np.float32)
+    path = tmp_path / "int.hkm"
+    _tree_file(path, levels, bf)
+    t = hk.hkm_read(path)
+    print("hkm_quantize nlevel=%d bf=%d n=%d" % (nlevel, bf, n), flush=True)
+    assert np.array_equal(t.quantize(v), Oracle().hkm_quantize(levels, bf, v))

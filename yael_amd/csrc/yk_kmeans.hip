@@ -1054,8 +1054,9 @@ static int yk_hq_descend(const float *v, const double *vn, long n, int d, int nl
   long lvl = 0, nn = 1;  // first centroid row of the level, its parent nodes
   for (int l = 0; l < nlevel; l++) {
     // an upper bound of the level's work items: nothing is read back, the
-    // items past the last one are skipped
-    const long nitems = l == 0 ? (n + 127) / 128 : n / 128 + nn;
+    // items past the last one are skipped (no more than points either: a
+    // node without any has no item)
+    const long nitems = l == 0 ? (n + 127) / 128 : min(n, n / 128 + nn);
     const unsigned gi = (unsigned)((nitems + 255) / 256);
     if (l == 0) {
       hipLaunchKernelGGL(yk_hq_root_kernel, dim3(gi), dim3(256), 0, st, n, nitems, off, item_inst,

@@ -134,21 +134,22 @@ static void yh_eps_rows(int ne, int d, const unsigned *gs, float *eps) {
 
 /* The split on the device: the draws are the reference's streams in its
  * order, the choice of the donors runs while the directions are drawn.  *done
- * = 0: not done (nothing changed), the host's split takes over. */
+ * = 0: not done (nothing changed; also where there is no memory for it), the
+ * host's split takes over. */
 #define YH_SPLIT_MAX_K 65536
 static int yh_split_device(int d, int k, float *cent, const int *counts, const int *hcounts, int ne,
                            unsigned seed, int *done) {
   *done = 0;
   if (k < 2 || k > YH_SPLIT_MAX_K) return YK_OK;
   void *ws = yh_buf(YH_KM_SPLIT, yk_split_ws_bytes(ne, d));
-  if (!ws) return YK_ENOMEM;
+  if (!ws) return YK_OK;
   double *rd = (double *)malloc(sizeof(double) * (size_t)ne);
   unsigned *gs = (unsigned *)malloc(sizeof(unsigned) * (size_t)ne);
   int *empties = (int *)malloc(sizeof(int) * (size_t)ne);
   float *eps = (float *)malloc(sizeof(float) * (size_t)ne * d);
+  const int room = rd && gs && empties && eps;
   int rc = YK_OK;
-  if (!rd || !gs || !empties || !eps) rc = yk_set_error_c(YK_ENOMEM, "host malloc");
-  if (rc == YK_OK) {
+  if (room) {
     for (int c = 0, e = 0; c < k; c++) {
       if (hcounts[c] != 0) continue;
       empties[e] = c;
@@ -157,7 +158,7 @@ static int yh_split_device(int d, int k, float *cent, const int *counts, const i
     }
     rc = yk_split_pick(counts, k, ne, rd, empties, ws);
   }
-  if (rc == YK_OK) {
+  if (room && rc == YK_OK) {
     yh_eps_rows(ne, d, gs, eps);
     rc = yk_split_apply(cent, d, ne, eps, ws, done);
   }

@@ -118,3 +118,14 @@ def test_noalloc_lists_in_passes():
         dist = ((b - q[i]).astype(np.float64) ** 2).sum(1)
         near = np.argsort(dist, kind="stable")[:k]
         assert np.allclose(dist[got_i[i]], dist[near], rtol=1e-5)
+
+
+@pytest.mark.parametrize("typ,k,first,second", [
+    (2, 10, (5000, 3000, 40), (2100, 4096, 24)),     # lists of nb places, several passes
+    (2, 16, (3700, 4097, 32), (1793, 9000, 64)),     # 4,096 places; one query left over
+    (16, 2, (16500, 100, 20), (16384, 1001, 16)),    # more than 16,384 queries
+    (2, 40, (5001, 2047, 48), (2600, 4500, 32))])
+def test_noalloc_passes(typ, k, first, second):
+    """Passes that are no power of two, and candidate lists no longer than the
+    base: the results of the allocating search, bit for bit."""
+    test_noalloc_matches_allocating_search("passes%d" % k, typ, k, False, first, second)

@@ -61,7 +61,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // word 3 of a raw (untyped, stride 0) buffer descriptor on gfx9-family GPUs
 #define YK_BUF_DWORD3 0x00020000
 
-#define YK_CAND_CAP 4096  // candidate keys kept per query (MODE 3)
+#define YK_CAND_CAP 4096  // candidate keys kept per query at most (MODE 3)
 #define YK_CSTAGE 8       // MODE 3: keys staged in LDS per (lane, query tile)
 #define YK_REG_R 16       // register top-R of MODE 2
 
@@ -86,7 +86,8 @@ struct ScanArgs {
   uint64_t *part;  // MODE 0: [nq][nsplit]; MODE 2: [nq][nsplit][2][R]
   const uint64_t *thr;  // MODE 3: per-query threshold key (0 = inactive)
   int *cnt;             // MODE 3: per-query candidate count
-  uint64_t *cand;       // MODE 3: [nq][YK_CAND_CAP]
+  uint64_t *cand;       // MODE 3: [nq][cap]
+  int cap;              // places of a query's list (yk_cand_cap)
   // batched form (item_inst != NULL): work item -> (instance, point tile);
   // q/qn/out_* are the concatenated points of all instances, b/bn the
   // instances' centroid sets (kpad rows apart), nb is unused
@@ -336,7 +337,7 @@ __global__ __launch_bounds__(256) void yk_scan_f32(ScanArgs a0) {
     const int base = atomicAdd(&a.cnt[qrow[j]], n);
     const uint64_t *src = cs + (j * 64 + lane) * YK_CSTAGE;
     for (int s_ = 0; s_ < n; s_++)
-      if (base + s_ < YK_CAND_CAP) a.cand[qrow[j] * YK_CAND_CAP + base + s_] = src[s_];
+      if (base + s_ < a.cap) a.cand[qrow[j] * a.cap + base + s_] = src[s_];
   };
   uint64_t top[NB][MODE == 2 ? R : 1];
   uint64_t T[NB];
@@ -782,7 +783,7 @@ yk_scan_f32_lds(ScanArgs a0) {
       const int base = atomicAdd(&a.cnt[qrow[j]], n);
       const uint64_t *src = cs + (j * 64 + lane) * CST;
       for (int s_ = 0; s_ < n; s_++)
-        if (base + s_ < YK_CAND_CAP) a.cand[(long)qrow[j] * YK_CAND_CAP + base + s_] = src[s_];
+        if (base + s_ < a.cap) a.cand[(long)qrow[j] * a.cap + base + s_] = src[s_];
     };
 
     // wave load i of a stage: lane l stores unit 64 (4 i + wave) + l of the
@@ -1136,7 +1137,7 @@ __device__ __forceinline__ void yk_cand_topk(const uint64_t *p, int m, int n, in
                                              int *cnt, int *flag) {
   uint64_t v[E];
   yk_wave_load<E>(p, m, lane, v);
-  if (n > YK_CAND_CAP) {
+  if (n > m) {  // the list overflowed
     const uint64_t x = yk_wave_kth<E>(v, k, false);
     if (lane == 0) {
       *thr = x;
@@ -1169,8 +1170,8 @@ __device__ __forceinline__ void yk_cand_topk(const uint64_t *p, int m, int n, in
 // counts, as in the precision form: 1e4 lists of ~700 keys, k = 100, 0.049
 // -> 0.012 ms against a workgroup's bitonic sort per query.)
 template <int E2>
-__global__ __launch_bounds__(256) void yk_select_kernel(const uint64_t *__restrict__ cand, long nq,
-                                                        int *cnt, uint64_t *thr, int k,
+__global__ __launch_bounds__(256) void yk_select_kernel(const uint64_t *__restrict__ cand, int cap,
+                                                        long nq, int *cnt, uint64_t *thr, int k,
                                                         int *out_i, float *out_d, int *flag,
                                                         int last) {
   __shared__ uint64_t lds[4][64 * E2];
@@ -1186,8 +1187,8 @@ __global__ __launch_bounds__(256) void yk_select_kernel(const uint64_t *__restri
     }
     return;
   }
-  const int m = n < YK_CAND_CAP ? n : YK_CAND_CAP;
-  const uint64_t *p = cand + q * (long)YK_CAND_CAP;
+  const int m = n < cap ? n : cap;
+  const uint64_t *p = cand + q * (long)cap;
   int *oi = out_i + q * k;
   float *od = out_d + q * k;
   if (m <= 256)
@@ -1479,7 +1480,7 @@ static int yk_select(const ScanArgs &a, uint64_t *thr, int k, int *assign, float
               : k <= 256 ? yk_select_kernel<4>
               : k <= 512 ? yk_select_kernel<8>
                          : yk_select_kernel<16>;
-  hipLaunchKernelGGL(kern, grid, block, 0, yk_stream(), a.cand, a.nq, a.cnt, thr, k, assign, dis,
+  hipLaunchKernelGGL(kern, grid, block, 0, yk_stream(), a.cand, a.cap, a.nq, a.cnt, thr, k, assign, dis,
                      flag, last);
   yk_prof_end(tok);
   YK_HIP(hipGetLastError());
@@ -1512,6 +1513,12 @@ static YkPlan yk_sketch_plan(long nq, long nb, int ld, bool weighted, int k, int
   return yk_plan(1, nq, nb, ld, weighted, stride, k, k > 256 ? k : 256, 16, cfg);
 }
 
+// places of a query's candidate list: no more than the base has rows (whole
+// lists for bases of 100 and 1,000 rows left the no-allocation search's 64 MB
+// room for 1,024 queries a pass: 16,384 queries, d = 32, 0.41 and 0.42 ms, now
+// 0.089 and 0.132)
+static int yk_cand_cap(long nb) { return nb < YK_CAND_CAP ? (int)((nb + 7) & ~7L) : YK_CAND_CAP; }
+
 // queries per pass of the filtered search (bounds the candidate memory)
 #define YK_LARGE_K_QB 16384L
 // splits of the register top-R scan behind it (k <= 16)
@@ -1532,11 +1539,16 @@ static int yk_knn_filtered(ScanArgs base, int k, int *assign, float *dis, YkAren
   const long QB = YK_LARGE_K_QB;
   const long nq_all = base.nq;
   const bool small = k <= YK_REG_R, weighted = base.w != nullptr;
+  // k <= 16 and a base that fits a list: no list overflows, and the proven
+  // bound leaves no query short (the sketch and the filtered scan evaluate
+  // the same expression), so the queued scan and its sort would find the flag
+  // unset: two launches, 3.3 of the 35 - 55 us of such a search
+  const bool last = small && base.nb <= YK_CAND_CAP;
   void *vthr, *vcnt, *vcand, *vpart;
   const long qb = nq_all < QB ? nq_all : QB;
   YK_TRY(yk_scratch(ar, 0, sizeof(uint64_t) * qb, &vthr));
   YK_TRY(yk_scratch(ar, 1, sizeof(int) * (qb + 64), &vcnt));
-  YK_TRY(yk_scratch(ar, 2, sizeof(uint64_t) * qb * YK_CAND_CAP, &vcand));
+  YK_TRY(yk_scratch(ar, 2, sizeof(uint64_t) * qb * yk_cand_cap(base.nb), &vcand));
   const size_t fixed_used = ar ? ar->used : 0;
   uint64_t *thr = (uint64_t *)vthr;
   int *cnt = (int *)vcnt;
@@ -1553,7 +1565,7 @@ static int yk_knn_filtered(ScanArgs base, int k, int *assign, float *dis, YkAren
     const YkPlan pa = yk_sketch_plan(nq, a.nb, a.ld, weighted, k, cfg);
     const YkPlan pc = yk_plan(2, nq, a.nb, a.ld, weighted, 1, 1, YK_FALLBACK_SPLITS, 16, 0);
     const size_t bytes_a = sizeof(uint64_t) * nq * pa.nsplit * 2;
-    const size_t bytes_c = small ? sizeof(uint64_t) * nq * pc.nsplit * 2 * YK_REG_R : 0;
+    const size_t bytes_c = small && !last ? sizeof(uint64_t) * nq * pc.nsplit * 2 * YK_REG_R : 0;
     if (ar) ar->used = fixed_used;  // each pass reuses the region's partial-key piece
     YK_TRY(yk_scratch(ar, 3, bytes_a > bytes_c ? bytes_a : bytes_c, &vpart));
     a.part = (uint64_t *)vpart;
@@ -1567,12 +1579,8 @@ static int yk_knn_filtered(ScanArgs base, int k, int *assign, float *dis, YkAren
     a.thr = thr;
     a.cnt = cnt;
     a.cand = (uint64_t *)vcand;
+    a.cap = yk_cand_cap(a.nb);
     int tries = 0;
-    // k <= 16 and a base that fits a list: no list overflows, and the proven
-    // bound leaves no query short (the sketch and the filtered scan evaluate
-    // the same expression), so the queued scan and its sort would find the flag
-    // unset: two launches, 3.3 of the 35 - 55 us of such a search
-    const bool last = small && a.nb <= YK_CAND_CAP;
     for (;;) {
       YK_TRY(yk_launch_scan(3, pb, a));
       YK_TRY(yk_select(a, thr, k, assign + q0 * k, dis + q0 * k, flag, last));
@@ -1866,9 +1874,10 @@ static size_t yk_knn_f32_need(long nq, long nb, int ld, bool weighted, int k, bo
   const YkPlan pa = yk_sketch_plan(qb, nb, ld, weighted, k, 0);
   const YkPlan pc = yk_plan(2, qb, nb, ld, weighted, 1, 1, YK_FALLBACK_SPLITS, 16, 0);
   const size_t bytes_a = sizeof(uint64_t) * qb * pa.nsplit * 2;
-  const size_t bytes_c = k <= YK_REG_R ? sizeof(uint64_t) * qb * pc.nsplit * 2 * YK_REG_R : 0;
+  const size_t bytes_c =
+      k <= YK_REG_R && nb > YK_CAND_CAP ? sizeof(uint64_t) * qb * pc.nsplit * 2 * YK_REG_R : 0;
   return yk_align256(sizeof(uint64_t) * qb) + yk_align256(sizeof(int) * (qb + 64)) +
-         yk_align256(sizeof(uint64_t) * qb * YK_CAND_CAP) +
+         yk_align256(sizeof(uint64_t) * qb * yk_cand_cap(nb)) +
          yk_align256(bytes_a > bytes_c ? bytes_a : bytes_c);
 }
 
@@ -1881,20 +1890,28 @@ extern "C" int yk_knn_f32_noalloc(int type, long nq, long nb, int d, int k, cons
   if (c != YK_OK) return c > 0 ? YK_OK : c;
   char *region = nullptr;
   YK_TRY(yk_noalloc_region(&region));
-  // Queries go in passes small enough for the region: the largest
-  // power-of-two pass (at most 16384 queries) whose scratch fits.  Each
-  // query's result depends only on that query, so the passes give the
-  // single call's results.
-  // (the route is the first pass's for them all)
-  long pass = 16384;
+  // Queries go in passes small enough for the region: of 16384 queries or
+  // fewer, halved until the scratch of a pass and of what the last one leaves
+  // over fits, then a quarter more at a time while that still fits.  Each
+  // query's result depends only on that query, so the passes give the single
+  // call's results.  (The route is the first pass's for them all.)
   const int ld = yk_ld(d);
-  bool lists;
-  size_t need;
-  for (;; pass >>= 1) {
-    const long n = pass < nq ? pass : nq;
+  bool lists = false;
+  auto need_of = [&](long pass) {
+    const long n = pass < nq ? pass : nq, left = nq % n;
     lists = yk_knn_by_lists(k, ld, n, nb);
-    need = yk_knn_f32_need(n, nb, ld, w != nullptr, k, lists);
-    if (need <= YK_NOALLOC_SCRATCH_BYTES || pass <= 32) break;
+    const size_t a = yk_knn_f32_need(n, nb, ld, w != nullptr, k, lists);
+    const size_t b = left ? yk_knn_f32_need(left, nb, ld, w != nullptr, k, lists) : 0;
+    return a > b ? a : b;
+  };
+  long pass = 16384;
+  size_t need = need_of(pass);
+  while (need > YK_NOALLOC_SCRATCH_BYTES && pass > 32) need = need_of(pass >>= 1);
+  if (pass >= 128 && pass < 16384 && pass < nq) {
+    long more = 7;  // quarters of the pass that fits
+    while (more > 4 && need_of(pass / 4 * more) > YK_NOALLOC_SCRATCH_BYTES) more--;
+    pass = pass / 4 * more;
+    need = need_of(pass);
   }
   if (need > YK_NOALLOC_SCRATCH_BYTES)
     return yk_set_error(YK_EINVAL,

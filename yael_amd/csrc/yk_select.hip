@@ -1519,8 +1519,13 @@ static YkPlan yk_sketch_plan(long nq, long nb, int ld, bool weighted, int k, int
 // 0.089 and 0.132)
 static int yk_cand_cap(long nb) { return nb < YK_CAND_CAP ? (int)((nb + 7) & ~7L) : YK_CAND_CAP; }
 
-// queries per pass of the filtered search (bounds the candidate memory)
-#define YK_LARGE_K_QB 16384L
+// queries per batch of the filtered search: candidate memory of 512 MB at
+// most, the batches of one size
+static long yk_filter_batch(long nq, long nb) {
+  const long most = 16384L * YK_CAND_CAP / yk_cand_cap(nb), n = (nq + most - 1) / most;
+  const long even = ((nq + n - 1) / n + 255) & ~255L;
+  return even < nq ? even : nq;
+}
 // splits of the register top-R scan behind it (k <= 16)
 #define YK_FALLBACK_SPLITS 16
 
@@ -1536,8 +1541,7 @@ static int yk_cand_cap(long nb) { return nb < YK_CAND_CAP ? (int)((nb + 7) & ~7L
 // of 1.34 ms for 1,003 queries x 100,003 vectors, d = 100, k = 10, with the
 // sort of its lists 0.36 ms.)
 static int yk_knn_filtered(ScanArgs base, int k, int *assign, float *dis, YkArena *ar, int cfg) {
-  const long QB = YK_LARGE_K_QB;
-  const long nq_all = base.nq;
+  const long nq_all = base.nq, qb = yk_filter_batch(nq_all, base.nb);
   const bool small = k <= YK_REG_R, weighted = base.w != nullptr;
   // k <= 16 and a base that fits a list: no list overflows, and the proven
   // bound leaves no query short (the sketch and the filtered scan evaluate
@@ -1545,7 +1549,6 @@ static int yk_knn_filtered(ScanArgs base, int k, int *assign, float *dis, YkAren
   // unset: two launches, 3.3 of the 35 - 55 us of such a search
   const bool last = small && base.nb <= YK_CAND_CAP;
   void *vthr, *vcnt, *vcand, *vpart;
-  const long qb = nq_all < QB ? nq_all : QB;
   YK_TRY(yk_scratch(ar, 0, sizeof(uint64_t) * qb, &vthr));
   YK_TRY(yk_scratch(ar, 1, sizeof(int) * (qb + 64), &vcnt));
   YK_TRY(yk_scratch(ar, 2, sizeof(uint64_t) * qb * yk_cand_cap(base.nb), &vcand));
@@ -1555,8 +1558,8 @@ static int yk_knn_filtered(ScanArgs base, int k, int *assign, float *dis, YkAren
   int *flag = cnt + qb + 32;
   const long stride = yk_sketch_stride(base.nb, k, cfg);
 
-  for (long q0 = 0; q0 < nq_all; q0 += QB) {
-    const long nq = nq_all - q0 < QB ? nq_all - q0 : QB;
+  for (long q0 = 0; q0 < nq_all; q0 += qb) {
+    const long nq = nq_all - q0 < qb ? nq_all - q0 : qb;
     ScanArgs a = base;
     a.q = base.q + q0 * base.ld;
     a.qn = base.qn ? base.qn + q0 : nullptr;
@@ -1621,27 +1624,31 @@ static int yk_knn_f32_check(int *type, long nq, long nb, int k) {
   return nq <= 0 ? 1 : YK_OK;
 }
 
-// k <= 16 by the register top-16 scan alone: large searches of long vectors,
-// where the sketch's sixteenth of the MFMAs and the filter's fewer waves cost
-// more than the lists' insertions save.  Both routes stream from memory there
-// (d > 256); a tile of 128 queries or fewer, and d <= 256, are the filter's.
-// The line is where the two meet, in 518 shapes of 65 .. 10,000 queries, 2e4 ..
-// 1e6 rows and d = 272 .. 2,048, k = 10 (2 and 16 alike), filter and lists in ms:
-//   d = 400: 4,000 x 1e5 5.32 / 5.63, 10,000 x 4e5 60.1 / 57.8
-//   d = 640: 1,000 x 4e5 8.18 / 8.17, 4,000 x 4e5 41.7 / 38.5
-//   d = 960: 1,000 x 1e5 3.30 / 3.82, 4,000 x 1e5 14.95 / 14.07
-//   d = 1536: 1,000 x 1e5 5.46 / 5.98, 768 x 4e5 16.3 / 15.4
-// Past it the lists take 0.91 - 1.0 of the filter's time, before it 1.0 - 3.6
-// times as long.  Up to 192 queries the second tile's idle waves cost the
-// filter's two scans more than the lists' one, and the line lies lower (124
-// shapes more):
-//   144 queries: 4e5, d = 960 3.67 / 3.36, 1e6, d = 704 6.60 / 6.18
-//   192 queries: 1e5, d = 1536 1.63 / 1.88, 4e5, d = 1536 5.91 / 5.58
-// Over all of them the rule is 0.5% from the faster route on average, 12% at
-// worst (its own line: 129 queries x 2e5, d = 960).
+// k <= 16 by the register top-16 scan alone, without sketch and filter.  The
+// lines lie where the two routes meet, in 2,000 shapes of 1 .. 200,000 queries,
+// 16 .. 1e6 rows, d = 16 .. 2,048, k = 2, 10 and 16; filter and lists in ms:
+// * two blocks of rows at most: the lists' two launches against four (1 query x
+//   33 rows, d = 128 0.032 / 0.029; x 80 0.033 / 0.037);
+// * many queries of few rows, where a query's selections cost more than its
+//   distances (50,000 queries, d = 64: x 200 0.31 / 0.19, x 600 0.37 / 0.36;
+//   200,000 x 1,000 1.63 / 1.45, x 2,000 2.18 / 2.40);
+// * d > 256, where both routes stream from memory: from 12,500 queries on
+//   (16,384 queries, d = 512: x 100 0.145 / 0.151, x 1,000 0.68 / 0.52, x 16,000
+//   4.79 / 4.82), and as the work grows, where the sketch's sixteenth of the MFMAs
+//   and the filter's fewer waves cost more than the lists' insertions save (d =
+//   400: 4,000 x 1e5 5.32 / 5.63, 10,000 x 4e5 60.1 / 57.8; d = 640: 1,000 x 4e5
+//   8.18 / 8.17, 4,000 x 4e5 41.7 / 38.5; d = 960: 1,000 x 1e5 3.30 / 3.82,
+//   4,000 x 1e5 14.95 / 14.07).  Up to 192 queries the second tile's idle waves
+//   cost the filter's two scans more than the lists' one, and the line lies
+//   lower (144 x 4e5, d = 960 3.67 / 3.36; 192 x 1e5, d = 1536 1.63 / 1.88); one
+//   tile is the filter's.
+// Past the lines the lists take 0.5 - 1.0 of the filter's time, before them 1.0
+// - 5 times as long.
 static bool yk_knn_by_lists(int k, int ld, long nq, long nb) {
-  return k > 1 && k <= YK_REG_R && ld > 256 && nq > 128 &&
-         (double)nq * (double)nb * ld * ld >= (nq <= 192 ? 4.6e13 : 1.3e14);
+  if (k < 2 || k > YK_REG_R) return false;
+  if (nb <= 48 || (nq >= 16384 && nb <= 100 + nq / 250)) return true;
+  return ld > 256 && (nq > 12500 || (nq > 128 && (double)nq * (double)nb * ld * ld >=
+                                                     (nq <= 192 ? 4.6e13 : 1.3e14)));
 }
 static YkPlan yk_lists_plan(long nq, long nb, int ld, bool weighted, int cfg) {
   return yk_plan(2, nq, nb, ld, weighted, 1, 1, 256, 16, cfg);
@@ -1771,7 +1778,7 @@ static int yk_f32_plan(const YkF32Call &call, int *cfg, int *ran) {
   const int ld = yk_ld(call.d);
   const bool weighted = call.w != nullptr;
   for (int i = 0; i < ncand; i++) {
-    const long nqb = call.nq < YK_LARGE_K_QB ? call.nq : YK_LARGE_K_QB;
+    const long nqb = yk_filter_batch(call.nq, call.nb);
     if (call.k == 1 || yk_knn_by_lists(call.k, ld, call.nq, call.nb)) {
       const YkPlan p = call.k > 1
                            ? yk_lists_plan(call.nq, call.nb, ld, weighted, i)
@@ -1870,7 +1877,7 @@ static size_t yk_knn_f32_need(long nq, long nb, int ld, bool weighted, int k, bo
     if (p.units) return yk_align256(sizeof(uint64_t) * 2 * (p.kind == YK_LDS2 ? 256 : 128) * p.slots);
     return p.nsplit > 1 ? yk_align256(sizeof(uint64_t) * nq * p.nsplit) : 0;
   }
-  const long qb = nq < YK_LARGE_K_QB ? nq : YK_LARGE_K_QB;
+  const long qb = yk_filter_batch(nq, nb);
   const YkPlan pa = yk_sketch_plan(qb, nb, ld, weighted, k, 0);
   const YkPlan pc = yk_plan(2, qb, nb, ld, weighted, 1, 1, YK_FALLBACK_SPLITS, 16, 0);
   const size_t bytes_a = sizeof(uint64_t) * qb * pa.nsplit * 2;

@@ -125,11 +125,21 @@ __device__ __forceinline__ void yk_reg_insert(uint64_t (&t)[R], uint64_t x) {
 // A lane's 16 row norms, in registers or (the kernels that stage them) read
 // from LDS where they are used: value i's norm is entry 8 (i >> 2) + (i & 3)
 // of the lane half's block norms.  dbl: the norm as a double, held as one in
-// LDS (a conversion per value and block less).
+// LDS (a conversion per value and block less); from a register it is converted
+// where it is used (the compiler moved the 16 conversions in front of the
+// branch, 17 of 117 vector instructions that every block executed).
 struct YkNormRegs {
   float n[16];
   __device__ __forceinline__ float operator[](int i) const { return n[i]; }
-  __device__ __forceinline__ double dbl(int i) const { return n[i]; }
+  __device__ __forceinline__ double dbl(int i) const {
+    float x = n[i];
+    asm volatile("" : "+v"(x));
+    return x;
+  }
+  __device__ __forceinline__ void all(float (&x)[16]) const {
+#pragma unroll
+    for (int i = 0; i < 16; i++) x[i] = n[i];
+  }
 };
 struct YkNormLds {
   const float *p;
@@ -137,6 +147,13 @@ struct YkNormLds {
   __device__ __forceinline__ double dbl(int i) const { return pd[8 * (i >> 2) + (i & 3)]; }
   __device__ __forceinline__ float operator[](int i) const { return p[8 * (i >> 2) + (i & 3)]; }
   __device__ __forceinline__ float pick(int is) const { return p[8 * (is >> 2) + (is & 3)]; }
+  __device__ __forceinline__ void all(float (&x)[16]) const {
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      const float4 v = *(const float4 *)(p + 8 * g);
+      x[4 * g] = v.x, x[4 * g + 1] = v.y, x[4 * g + 2] = v.z, x[4 * g + 3] = v.w;
+    }
+  }
 };
 
 // The approximations of a lane's 16 values, m_i = bn - 2 acc (type 16: acc);
@@ -201,10 +218,11 @@ __device__ __forceinline__ void yk_best1_block(const f32x16 &acc, const Norms &n
   // path, executing them for every block).
   if (test) {
     const float qf = (float)qnd;
-    float mm = INFINITY, nmax = 0.f;
+    float mm = INFINITY, nmax = 0.f, ns[16];
+    nn.all(ns);  // (four 16-byte reads: between the statements below, sixteen)
 #pragma unroll
     for (int i = 0; i < 16; i++) {
-      float ax = acc[i], nx = nn[i];
+      float ax = acc[i], nx = ns[i];
       asm volatile("" : "+v"(ax), "+v"(nx));
       mm = fminf(mm, DOT ? ax : __builtin_fmaf(-2.0f, ax, nx));
       nmax = fmaxf(nmax, nx);

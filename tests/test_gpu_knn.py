@@ -665,3 +665,29 @@ def test_lists_line(ya, nq, nb, d, k, typ, weighted):
     want = np.argsort(dist, axis=1, kind="stable")[:, :k]
     assert np.array_equal(gi, want)
     assert np.array_equal(gd, np.take_along_axis(dist, want, 1))
+
+
+@pytest.mark.parametrize("nq,nb,d,k", [
+    (1300, 32000, 16, 1), (1300, 32768, 12, 1),      # even shares, a hundred to a tile
+    (70, 16000, 16, 1), (100, 3000, 128, 1),         # few tiles: whole splits
+    (32640, 250, 16, 1), (32641, 250, 16, 1),        # 255 and 256 tiles of 8 blocks
+    (65535, 300, 16, 1), (65536, 300, 16, 1), (65537, 1000, 7, 1),  # one, two tiles per wave
+    (50000, 64, 16, 1), (20000, 224, 30, 1), (20000, 225, 30, 1),   # 7 blocks and 8
+    (300, 5000, 32, 10), (300, 5000, 33, 10), (100, 9000, 16, 60), (70, 6001, 33, 17)])
+@pytest.mark.parametrize("typ", [2, 16])
+def test_scan_plans(ya, nq, nb, d, k, typ):
+    """Each side of the lines between the scans' plans.  Integer data, so every
+    value is exact in FP32 and many tie: the k least by (value, index)."""
+    rng = np.random.default_rng(nq + nb + d + k)
+    b = rng.integers(0, 9, (nb, d)).astype(np.float32)
+    q = rng.integers(0, 9, (nq, d)).astype(np.float32)
+    print("scan plans", nq, nb, d, k, typ, flush=True)
+    gi, gd = ya.knn(q, b, k, distance_type=typ)
+    for i in range(0, nq, 8192):
+        dist = q[i:i + 8192] @ b.T
+        if typ == 2:
+            dist = ((q[i:i + 8192] ** 2).sum(1)[:, None] + (b * b).sum(1)[None]) - 2 * dist
+        want = (dist.argmin(1)[:, None] if k == 1
+                else np.argsort(dist, axis=1, kind="stable")[:, :k])
+        assert np.array_equal(gi[i:i + 8192], want)
+        assert np.array_equal(gd[i:i + 8192], np.take_along_axis(dist, want, 1))

@@ -1020,23 +1020,29 @@ yk_scan_f32_lds(ScanArgs a0) {
 
 // k = 1 over even shares (yk_scan_f32_lds with units): the queries of tiles
 // cut by a share's end, from the shares' minima (at most W + 1 of the tiles
-// are cut; the others were written by the scan)
+// are cut; the others were written by the scan).  A thread per query, or where
+// a tile has many shares (few queries) a wave, its lanes striding them: 70
+// queries x 16,000 vectors, d = 16, 500 shares: the search 0.23 -> 0.024 ms.
+template <bool WAVE>
 __global__ __launch_bounds__(256) void yk_merge_share_kernel(const uint64_t *__restrict__ part,
                                                              long nq, int tq, long units, long T,
                                                              long W, int *out_i, float *out_d) {
-  const long q = blockIdx.x * 256L + threadIdx.x;
+  const long q = WAVE ? blockIdx.x * 4L + (threadIdx.x >> 6) : blockIdx.x * 256L + threadIdx.x;
+  const int lane = WAVE ? threadIdx.x & 63 : 0;
   if (q >= nq) return;
   const long tile = q / tq, lo = tile * units, hi = lo + units;
-  long w = yk_share_of(lo, T, W);
-  if ((w + 1) * T / W >= hi) return;  // one share covers the tile
+  const long w0 = yk_share_of(lo, T, W);
+  if ((w0 + 1) * T / W >= hi) return;  // one share covers the tile
   uint64_t best = YK_KEY_NONE;
-  for (; w < W; w++) {
+  for (long w = w0 + lane; w < W; w += WAVE ? 64 : 1) {
     const long s = w * T / W;
     if (s >= hi) break;
     if ((w + 1) * T / W == s) continue;  // an empty share
     const uint64_t v = part[(w * 2 + (s > lo ? 0 : 1)) * tq + q % tq];
     best = v < best ? v : best;
   }
+  if (WAVE) best = yk_wave_min64(best);
+  if (lane > 0) return;
   out_i[q] = best == YK_KEY_NONE ? -1 : (int)(uint32_t)best;
   out_d[q] = best == YK_KEY_NONE ? 1e30f : yk_fkey_inv((uint32_t)(best >> 32));
 }
@@ -1721,8 +1727,10 @@ static int yk_knn_f32_run(int type, long nq, long nb, int d, int k, const float 
   YK_TRY(yk_launch_scan(0, p, a));
   if (p.units) {
     int tok = yk_prof_begin(YK_PROF_MERGE);
-    hipLaunchKernelGGL(yk_merge_share_kernel, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0,
-                       yk_stream(), a.part, nq, (int)tq, (long)p.units,
+    const bool wave = p.slots > 8L * p.tiles;  // shares per tile
+    const auto merge = wave ? yk_merge_share_kernel<true> : yk_merge_share_kernel<false>;
+    hipLaunchKernelGGL(merge, dim3((unsigned)(wave ? (nq + 3) / 4 : (nq + 255) / 256)), dim3(256),
+                       0, yk_stream(), a.part, nq, (int)tq, (long)p.units,
                        (long)p.tiles * p.units, (long)p.slots, assign, dis);
     yk_prof_end(tok);
     YK_HIP(hipGetLastError());

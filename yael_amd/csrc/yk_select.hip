@@ -1344,7 +1344,10 @@ static YkPlan yk_plan(int mode, long nq, long nb, int ld, bool weighted, long sa
   const long nblocks = (nb + p.bstep - 1) / p.bstep;  // processed blocks
   p.kind = YK_STREAM;
   p.waves = 4;
-  if (mode != 2 && ld <= 256 && (nq > YK_STREAM_NQ || ld > 128)) {
+  // (a sketch or filtered scan of one or two chunks has too few MFMAs per block
+  // for the stages' barriers: 5,000 queries x 16,000, d = 16, k = 10 0.166 ms
+  // staged, 0.130 streamed; 300 x 1e6, k = 100 0.32 and 0.245)
+  if (mode != 2 && ld <= 256 && (nq > YK_STREAM_NQ || ld > 128) && (mode == 0 || ld > 32)) {
     // two query tiles per wave where the chip still has work for every wave
     p.kind = ld <= 128 && nq > 128 && (nq + 255) / 256 * nblocks >= 2048 ? YK_LDS2 : YK_LDS1;
   } else if (mode != 2 && nq <= YK_STREAM_NQ) {

@@ -630,14 +630,17 @@ __global__ __launch_bounds__(256) void yk_scan_f32(ScanArgs a0) {
 // n = 1e5 points to 1,024 centroids 0.290 ms, 90 TFLOP/s).  Here the
 // workgroup's four waves share each block: a 32-row block is one contiguous
 // piece of memory, loaded 1 KB per wave instruction straight into the other
-// of two LDS buffers while a stage is multiplied (no registers hold it: 16
-// of them made the two-tile kernel spill).  The four 16-byte units of a
+// of two LDS buffers while a stage is multiplied (no registers hold it).  The four 16-byte units of a
 // row's chunk are stored in the order unit ^ (row & 3), which spreads the
 // rows' reads over four times the banks and leaves the chunk a constant
-// offset of the read's address.  One barrier per stage.  Two query tiles per wave (NB = 2, d <= 128:
-// 128 registers of queries) use each fragment read from LDS twice; short
-// vectors stage G blocks at once so that a stage is at least 64 MFMAs per
-// tile.  Same MFMA operands, same order, same epilogue arithmetic as the
+// offset of the read's address.  One barrier per stage; short vectors stage G
+// blocks at once so that a stage is at least 64 MFMAs.  Two query tiles per
+// wave (NB = 2) would use each fragment read from LDS twice, but at d = 128
+// their 128 registers of queries leave two waves per SIMD and spills, and 256
+// queries a workgroup fewer of them: 1e5 queries x 1,024 0.260 against 0.236 ms,
+// 20,000 x 16,384, k = 100 2.00 and 1.84, 300 x 1e6 1.27 and 1.00 (1.17
+// streamed).  Only k = 1 at d <= 16 keeps them, from 65,536 queries on (3e5 x
+// 1,024 0.144 and 0.150).  Same MFMA operands, same order, same epilogue arithmetic as the
 // streaming kernel: the same bits.  n = 1e5 points to 1,024 centroids: 0.290
 // -> 0.235 ms (112 TFLOP/s; n = 1e6: 123).  What is left of the FP32 rate
 // (153 TFLOP/s for a large library product): timing builds without the
@@ -649,7 +652,7 @@ struct YkLdsShape {
   static constexpr int G = NCH == 1 ? 8 : NCH == 2 ? 4 : NCH <= 4 ? 2 : 1;  // blocks per stage
   static constexpr int KL = G * 32 * U / 64;  // 1 KB wave loads of a stage
   static constexpr int NL = (KL + 3) / 4;     // of them per wave
-  // MODE 3: keys staged per (lane, query tile); fewer where two workgroups
+  // MODE 3: keys staged per lane; fewer where two workgroups
   // would not fit a CU's LDS otherwise
   static constexpr int CST = NCH > 8 ? 4 : 8;
 };
@@ -1239,7 +1242,7 @@ __global__ void yk_zero_cnt_kernel(int *cnt, long n) {
 // by its bytes, and a wave streams rows straight to registers (YK_STREAM; one
 // or two waves per workgroup, so that every wave has queries of its own);
 // beyond that the workgroup shares the base through LDS (YK_LDS1: 32 queries
-// per wave, YK_LDS2: 64).  d > 256 streams both operands.
+// per wave, YK_LDS2: 64, k = 1 of many short queries).  d > 256 streams both operands.
 enum { YK_STREAM = 0, YK_LDS1 = 1, YK_LDS2 = 2 };
 #define YK_STREAM_NQ 64
 
@@ -1284,19 +1287,7 @@ static YkScanKernel yk_stream_pick(int ld, bool weighted) {
 }
 
 template <int MODE, bool WT>
-static YkScanKernel yk_lds_pick(int kind, int ld) {
-  if (kind == YK_LDS2) {
-    switch (ld >> 4) {
-      case 1: return yk_scan_f32_lds<2, 1, MODE, WT>;
-      case 2: return yk_scan_f32_lds<2, 2, MODE, WT>;
-      case 3: return yk_scan_f32_lds<2, 3, MODE, WT>;
-      case 4: return yk_scan_f32_lds<2, 4, MODE, WT>;
-      case 5: return yk_scan_f32_lds<2, 5, MODE, WT>;
-      case 6: return yk_scan_f32_lds<2, 6, MODE, WT>;
-      case 7: return yk_scan_f32_lds<2, 7, MODE, WT>;
-      default: return yk_scan_f32_lds<2, 8, MODE, WT>;
-    }
-  }
+static YkScanKernel yk_lds_pick(int ld) {
   switch (ld >> 4) {
     case 1: return yk_scan_f32_lds<1, 1, MODE, WT>;
     case 2: return yk_scan_f32_lds<1, 2, MODE, WT>;
@@ -1318,14 +1309,15 @@ static YkScanKernel yk_lds_pick(int kind, int ld) {
 }
 
 static YkScanKernel yk_scan_pick(int mode, int kind, int ld, bool weighted) {
-  if (kind != YK_STREAM && weighted)
-    return mode == 0   ? yk_lds_pick<0, true>(kind, ld)
-           : mode == 1 ? yk_lds_pick<1, true>(kind, ld)
-                       : yk_lds_pick<3, true>(kind, ld);
-  if (kind != YK_STREAM)
-    return mode == 0   ? yk_lds_pick<0, false>(kind, ld)
-           : mode == 1 ? yk_lds_pick<1, false>(kind, ld)
-                       : yk_lds_pick<3, false>(kind, ld);
+  if (kind == YK_LDS2) return yk_scan_f32_lds<2, 1, 0, false>;
+  if (kind == YK_LDS1 && weighted)
+    return mode == 0   ? yk_lds_pick<0, true>(ld)
+           : mode == 1 ? yk_lds_pick<1, true>(ld)
+                       : yk_lds_pick<3, true>(ld);
+  if (kind == YK_LDS1)
+    return mode == 0   ? yk_lds_pick<0, false>(ld)
+           : mode == 1 ? yk_lds_pick<1, false>(ld)
+                       : yk_lds_pick<3, false>(ld);
   return mode == 0   ? yk_stream_pick<0, 1>(ld, weighted)
          : mode == 1 ? yk_stream_pick<1, 1>(ld, weighted)
          : mode == 2 ? yk_stream_pick<2, YK_REG_R>(ld, weighted)
@@ -1348,8 +1340,7 @@ static YkPlan yk_plan(int mode, long nq, long nb, int ld, bool weighted, long sa
   // for the stages' barriers: 5,000 queries x 16,000, d = 16, k = 10 0.166 ms
   // staged, 0.130 streamed; 300 x 1e6, k = 100 0.32 and 0.245)
   if (mode != 2 && ld <= 256 && (nq > YK_STREAM_NQ || ld > 128) && (mode == 0 || ld > 32)) {
-    // two query tiles per wave where the chip still has work for every wave
-    p.kind = ld <= 128 && nq > 128 && (nq + 255) / 256 * nblocks >= 2048 ? YK_LDS2 : YK_LDS1;
+    p.kind = mode == 0 && ld <= 16 && !weighted && nq >= 65536 ? YK_LDS2 : YK_LDS1;
   } else if (mode != 2 && nq <= YK_STREAM_NQ) {
     p.waves = nq <= 32 ? 1 : 2;
   }

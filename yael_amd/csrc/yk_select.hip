@@ -1350,19 +1350,21 @@ static YkPlan yk_plan(int mode, long nq, long nb, int ld, bool weighted, long sa
   // too, from beyond the L2: three workgroups per CU (1e4 queries x 1e5, d =
   // 960, k = 100: 37.9 ms; the four that fit 40.6, two 38.8)
   const int most = mode == 3 && ld > 256 && p.waves == 4 ? 3 : 0;
-  p.slots = yk_resident_wgs((const void *)yk_scan_pick(mode, p.kind, ld, weighted), 64 * p.waves,
-                            most);
-  if (mode == 0 && p.kind != YK_STREAM && nb * ld <= (1L << 19) && nblocks >= 8) {
+  const YkScanKernel kern = yk_scan_pick(mode, p.kind, ld, weighted);
+  p.slots = yk_resident_wgs((const void *)kern, 64 * p.waves, most);
+  if (mode == 0 && p.kind != YK_STREAM && nb * ld <= (1L << 19) && nblocks >= 8 &&
+      (p.tiles * nblocks >= 4L * p.slots ||
+       p.tiles >= yk_resident_wgs((const void *)kern, 64 * p.waves, 1))) {
     // k = 1 over a base of at most 2 MB, which every XCD's L2 holds (the
     // k-means assign): even shares of the (tile, block) pairs, so that no CU
-    // waits for a last round of whole tiles (n = 1e5 points are 391 tiles for
-    // 512 workgroups).  Fewer than 8 blocks make a tile too short for the
-    // merge's launch to pay.
+    // waits for a last round of whole tiles (n = 1e5 points are 782 tiles).
+    // Fewer than 8 blocks make a tile too short for the merge's launch to pay;
+    // with fewer tiles than CUs, shares of fewer than 4 blocks are mostly
+    // queries loaded (20,000 x 250, d = 8: 0.87 of the time in whole tiles;
+    // 10,000 x 500 0.80; 100,000 x 250, 391 tiles, 1.28).
     p.units = (int)nblocks;
     p.nsplit = 1;
     p.brange = nblocks * p.bstep;
-    const long T = (long)p.tiles * p.units;
-    if (T < p.slots) p.slots = (int)T;
     return p;
   }
   // ~8 work items per resident workgroup keeps the tail of the persistent

@@ -1372,8 +1372,9 @@ static YkPlan yk_plan(int mode, long nq, long nb, int ld, bool weighted, long sa
   long want = (yk_item_targets[cfg % 3] + p.tiles - 1) / p.tiles;
   long maxs = (nblocks + min_blocks - 1) / min_blocks;
   if (want > maxs) want = maxs;
-  if ((mode == 0 || mode == 3) && p.tiles * nblocks < 96L * p.slots) {
-    // few blocks per workgroup: of the splits that fill r rounds of the
+  if (((mode == 0 && nblocks >= 8) || mode == 3) && p.tiles * nblocks < 96L * p.slots) {
+    // few blocks per workgroup (a k = 1 tile of fewer than 8 is not split: the
+    // merge takes longer; 50,000 queries x 64 rows, d = 16, 0.82 of the rate): of the splits that fill r rounds of the
     // resident workgroups, the one whose rounds take least (a round is a
     // split's blocks, and ~3 more for its queries and its end)
     long best = -1;

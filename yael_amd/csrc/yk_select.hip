@@ -1372,7 +1372,12 @@ static YkPlan yk_plan(int mode, long nq, long nb, int ld, bool weighted, long sa
   long want = (yk_item_targets[cfg % 3] + p.tiles - 1) / p.tiles;
   long maxs = (nblocks + min_blocks - 1) / min_blocks;
   if (want > maxs) want = maxs;
-  if (((mode == 0 && nblocks >= 8) || mode == 3) && p.tiles * nblocks < 96L * p.slots) {
+  // (k = 1 of long vectors, four workgroups per CU streaming both operands:
+  // beyond 20 blocks each the uneven rounds cost more than they save; 100,000 x
+  // 1,000, d = 750 0.70 of the time without, 10,000 x 16,000 0.91, but 50,000 x
+  // 1,600 1.09 and 5,000 x 10,000 1.11)
+  const long few = mode == 0 && ld > 256 ? 20 : 96;
+  if (((mode == 0 && nblocks >= 8) || mode == 3) && p.tiles * nblocks < few * p.slots) {
     // few blocks per workgroup (a k = 1 tile of fewer than 8 is not split: the
     // merge takes longer; 50,000 queries x 64 rows, d = 16, 0.82 of the rate): of the splits that fill r rounds of the
     // resident workgroups, the one whose rounds take least (a round is a

@@ -638,7 +638,8 @@ def test_small_k_list_overflow(ya, nq, k):
 
 
 @pytest.mark.parametrize("nq,nb,d", [(200, 38743, 4096), (200, 38744, 4096), (128, 61000, 4096),
-                                     (129, 60066, 4090), (129, 21254, 4096), (192, 14281, 4096),
+                                     (129, 60066, 4090), (160, 7450, 4096), (160, 7451, 4096),
+                                     (161, 48127, 4096), (161, 48128, 4096),
                                      (513, 5003, 704), (12500, 333, 260), (12501, 333, 260),
                                      (16383, 165, 20), (16384, 165, 20), (16384, 166, 20),
                                      (3, 48, 30), (70, 48, 128), (70, 49, 128), (300, 16, 200)])
@@ -646,8 +647,8 @@ def test_small_k_list_overflow(ya, nq, k):
 @pytest.mark.parametrize("typ,weighted", [(2, False), (16, False), (2, True)])
 def test_lists_line(ya, nq, nb, d, k, typ, weighted):
     """k <= 16 on both sides of the lines past which the register lists answer
-    alone: long vectors (more than 128 queries and nq nb ld^2 of 1.3e14, up to
-    192 queries 4.6e13; more than 12,500 queries), many queries of few rows, 48
+    alone: long vectors (more than a tile and a wave of queries and nq nb ld^2
+    of 1.3e14, with a wave in the second tile 2e13; more than 12,500 queries), many queries of few rows, 48
     rows.  Integer data (weights are powers of two), so every value is exact in
     FP32: the k least by (value, index)."""
     rng = np.random.default_rng(nq + nb + d + k)

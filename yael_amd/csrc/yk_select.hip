@@ -1348,8 +1348,10 @@ static YkPlan yk_plan(int mode, long nq, long nb, int ld, bool weighted, long sa
   p.tiles = (int)((nq + qt - 1) / qt);
   // the filtered scan of vectors too long for registers streams its queries
   // too, from beyond the L2: three workgroups per CU (1e4 queries x 1e5, d =
-  // 960, k = 100: 37.9 ms; the four that fit 40.6, two 38.8)
-  const int most = mode == 3 && ld > 256 && p.waves == 4 ? 3 : 0;
+  // 960, k = 100: 37.9 ms; the four that fit 40.6, two 38.8); the queries of one
+  // tile, or of a tile and a wave, stay in it (65 x 1e6, d = 960, k = 60 0.92 of
+  // the time with four)
+  const int most = mode == 3 && ld > 256 && p.waves == 4 && nq > qt + 32 ? 3 : 0;
   const YkScanKernel kern = yk_scan_pick(mode, p.kind, ld, weighted);
   p.slots = yk_resident_wgs((const void *)kern, 64 * p.waves, most);
   if (mode == 0 && p.kind != YK_STREAM && nb * ld <= (1L << 19) && nblocks >= 8 &&
@@ -1372,16 +1374,22 @@ static YkPlan yk_plan(int mode, long nq, long nb, int ld, bool weighted, long sa
   long want = (yk_item_targets[cfg % 3] + p.tiles - 1) / p.tiles;
   long maxs = (nblocks + min_blocks - 1) / min_blocks;
   if (want > maxs) want = maxs;
-  // (k = 1 of long vectors, four workgroups per CU streaming both operands:
+  // k = 1 of long vectors, four workgroups per CU streaming both operands:
   // beyond 20 blocks each the uneven rounds cost more than they save; 100,000 x
   // 1,000, d = 750 0.70 of the time without, 10,000 x 16,000 0.91, but 50,000 x
-  // 1,600 1.09 and 5,000 x 10,000 1.11)
-  const long few = mode == 0 && ld > 256 ? 20 : 96;
+  // 1,600 1.09 and 5,000 x 10,000 1.11.
+  // A filtered scan of long vectors whose last tile has one wave of queries: the
+  // workgroups of that tile end early, and with much to scan only many items in
+  // turn fill their place (130 x 1e6, d = 512, k = 60 0.72 of the time).
+  const bool uneven =
+      mode == 3 && ld > 256 && nblocks > 8192 && nq > qt && (nq - 1) % qt < 32;
+  const long few = uneven ? 0 : mode == 0 && ld > 256 ? 20 : 96;
   if (((mode == 0 && nblocks >= 8) || mode == 3) && p.tiles * nblocks < few * p.slots) {
     // few blocks per workgroup (a k = 1 tile of fewer than 8 is not split: the
-    // merge takes longer; 50,000 queries x 64 rows, d = 16, 0.82 of the rate): of the splits that fill r rounds of the
-    // resident workgroups, the one whose rounds take least (a round is a
-    // split's blocks, and ~3 more for its queries and its end)
+    // merge takes longer; 50,000 queries x 64 rows, d = 16, 0.82 of the rate):
+    // of the splits that fill r rounds of the resident workgroups, the one whose
+    // rounds take least (a round is a split's blocks, and ~3 more for its
+    // queries and its end)
     long best = -1;
     for (long r = 1; r <= 16; r++) {
       const long s = min(nblocks, r * p.slots / p.tiles);
@@ -1664,17 +1672,20 @@ static int yk_knn_f32_check(int *type, long nq, long nb, int k) {
 //   and the filter's fewer waves cost more than the lists' insertions save (d =
 //   400: 4,000 x 1e5 5.32 / 5.63, 10,000 x 4e5 60.1 / 57.8; d = 640: 1,000 x 4e5
 //   8.18 / 8.17, 4,000 x 4e5 41.7 / 38.5; d = 960: 1,000 x 1e5 3.30 / 3.82,
-//   4,000 x 1e5 14.95 / 14.07).  Up to 192 queries the second tile's idle waves
-//   cost the filter's two scans more than the lists' one, and the line lies
-//   lower (144 x 4e5, d = 960 3.67 / 3.36; 192 x 1e5, d = 1536 1.63 / 1.88); one
-//   tile is the filter's.
+//   4,000 x 1e5 14.95 / 14.07).  One tile is the filter's, and so are a few whose
+//   last one has a single wave of queries (144 x 1e6, d = 960 6.6 / 8.2), but a
+//   second tile of one wave over few blocks (yk_plan's uneven: 144 x 2e5, d = 960
+//   1.98 / 1.81, d = 512 0.96 / 1.05; x 1e5 1.05 / 1.16).
 // Past the lines the lists take 0.5 - 1.0 of the filter's time, before them 1.0
 // - 5 times as long.
 static bool yk_knn_by_lists(int k, int ld, long nq, long nb) {
   if (k < 2 || k > YK_REG_R) return false;
   if (nb <= 48 || (nq >= 16384 && nb <= 100 + nq / 250)) return true;
-  return ld > 256 && (nq > 12500 || (nq > 128 && (double)nq * (double)nb * ld * ld >=
-                                                     (nq <= 192 ? 4.6e13 : 1.3e14)));
+  if (ld <= 256 || nq <= 128) return false;
+  const double work = (double)nq * (double)nb * ld * ld;
+  if (nq <= 160) return nb <= (1L << 18) && work >= 2e13;
+  if (nq <= 512 && (nq - 1) % 128 < 32) return false;
+  return nq > 12500 || work >= 1.3e14;
 }
 static YkPlan yk_lists_plan(long nq, long nb, int ld, bool weighted, int cfg) {
   return yk_plan(2, nq, nb, ld, weighted, 1, 1, 256, 16, cfg);

@@ -243,9 +243,12 @@ extern "C" int yk_sync(void) {
 
 // Copies of YK_STAGE_MIN_* bytes and more from and to pageable host memory: up
 // to YK_STAGE_THREADS host threads, one per YK_STAGE_SLICE bytes, each take a
-// contiguous slice and push it through two pinned buffers on a stream of
-// their own (default priority), the host copy of one buffer overlapping the
-// DMA of the other.  (A plain copy to pageable memory goes in 1 MB pieces, 20
+// contiguous slice and push it through two pinned buffers, the host copy of one
+// buffer overlapping the DMA of the other.  Up, each thread has a stream of its
+// own (default priority; 512 MB 9.9 ms, on one stream 10.7).  Down, the DMAs
+// queue on the library's stream: after copies on several streams the
+// allocations of a later call take longer (two k-means training calls in a row,
+// 16 sub-spaces of 94,555 points, d = 24, k = 93: 3.1 against 2.6 ms a call).  (A plain copy to pageable memory goes in 1 MB pieces, 20
 // us on the bus and ~70 us between them.  256 MB: 17 GB/s plain, 51 with four
 // threads, 42 with eight.)  The pinned buffers (64 MB in all)
 // are allocated at the first such copy and kept until the process ends; a
@@ -255,7 +258,7 @@ extern "C" int yk_sync(void) {
 #define YK_STAGE_BYTES ((size_t)8 << 20)
 static pthread_mutex_t g_stage_mu = PTHREAD_MUTEX_INITIALIZER;
 static void *g_stage_buf[YK_STAGE_THREADS][2];
-static hipStream_t g_stage_st[YK_STAGE_THREADS];
+static hipStream_t g_stage_st[YK_STAGE_THREADS];  // up
 static hipEvent_t g_stage_ev[YK_STAGE_THREADS][2];
 static int g_stage_ready = 0;
 
@@ -264,6 +267,7 @@ struct YkStageJob {
   size_t bytes;
   int t;
   bool up;
+  hipStream_t st;
   hipError_t err;
 };
 
@@ -287,9 +291,9 @@ static void *yk_stage_worker(void *arg) {
     hipError_t e = settle(b);
     if (e == hipSuccess && j->up) memcpy(buf, j->host + off, n);
     if (e == hipSuccess)
-      e = j->up ? hipMemcpyAsync(j->dev + off, buf, n, hipMemcpyHostToDevice, g_stage_st[j->t])
-                : hipMemcpyAsync(buf, j->dev + off, n, hipMemcpyDeviceToHost, g_stage_st[j->t]);
-    if (e == hipSuccess) e = hipEventRecord(g_stage_ev[j->t][b], g_stage_st[j->t]);
+      e = j->up ? hipMemcpyAsync(j->dev + off, buf, n, hipMemcpyHostToDevice, j->st)
+                : hipMemcpyAsync(buf, j->dev + off, n, hipMemcpyDeviceToHost, j->st);
+    if (e == hipSuccess) e = hipEventRecord(g_stage_ev[j->t][b], j->st);
     j->err = e;
     pend[b] = n;
     at[b] = off;
@@ -297,28 +301,28 @@ static void *yk_stage_worker(void *arg) {
   }
   if (j->err == hipSuccess) j->err = settle(0);
   if (j->err == hipSuccess) j->err = settle(1);
-  const hipError_t e = hipStreamSynchronize(g_stage_st[j->t]);
-  if (j->err == hipSuccess) j->err = e;
+  // (after an error: nothing of this slice is left in flight)
+  if (j->err != hipSuccess) (void)hipStreamSynchronize(j->st);
   return nullptr;
 }
 
-static int yk_stage_setup(void) {
+static int yk_stage_setup(bool up) {
+  for (int t = 0; up && t < YK_STAGE_THREADS; t++)
+    if (!g_stage_st[t]) YK_HIP(hipStreamCreateWithFlags(&g_stage_st[t], hipStreamNonBlocking));
   if (g_stage_ready) return YK_OK;
-  for (int t = 0; t < YK_STAGE_THREADS; t++) {
+  for (int t = 0; t < YK_STAGE_THREADS; t++)
     for (int b = 0; b < 2; b++) {
       YK_HIP(hipHostMalloc(&g_stage_buf[t][b], YK_STAGE_BYTES, hipHostMallocDefault));
       YK_HIP(hipEventCreateWithFlags(&g_stage_ev[t][b], hipEventDisableTiming));
     }
-    YK_HIP(hipStreamCreateWithFlags(&g_stage_st[t], hipStreamNonBlocking));
-  }
   g_stage_ready = 1;
   return YK_OK;
 }
 
 static int yk_copy_staged(char *dev, char *host, size_t bytes, bool up) {
-  YK_HIP(hipStreamSynchronize(g_stream));  // earlier work on the device memory has finished
+  if (up) YK_HIP(hipStreamSynchronize(g_stream));  // earlier work on the device memory
   pthread_mutex_lock(&g_stage_mu);
-  int rc = yk_stage_setup();
+  int rc = yk_stage_setup(up);
   if (rc == YK_OK) {
     size_t ways = bytes / YK_STAGE_SLICE;
     if (ways > YK_STAGE_THREADS) ways = YK_STAGE_THREADS;
@@ -328,7 +332,8 @@ static int yk_copy_staged(char *dev, char *host, size_t bytes, bool up) {
     int started[YK_STAGE_THREADS] = {0}, nt = 0;
     for (int t = 0; t < YK_STAGE_THREADS && (size_t)t * per < bytes; t++, nt++) {
       const size_t o = (size_t)t * per;
-      job[t] = {dev + o, host + o, bytes - o < per ? bytes - o : per, t, up, hipSuccess};
+      job[t] = {dev + o, host + o, bytes - o < per ? bytes - o : per, t, up,
+                up ? g_stage_st[t] : g_stream, hipSuccess};
     }
     for (int t = 1; t < nt; t++)
       started[t] = pthread_create(&th[t], nullptr, yk_stage_worker, &job[t]) == 0;

@@ -642,7 +642,8 @@ def test_small_k_list_overflow(ya, nq, k):
                                      (161, 48127, 4096), (161, 48128, 4096),
                                      (513, 5003, 704), (12500, 333, 260), (12501, 333, 260),
                                      (16383, 165, 20), (16384, 165, 20), (16384, 166, 20),
-                                     (3, 48, 30), (70, 48, 128), (70, 49, 128), (300, 16, 200)])
+                                     (3, 48, 30), (70, 48, 128), (70, 49, 128), (4000, 64, 30),
+                                     (4000, 65, 30), (16000, 130, 30), (16000, 131, 30), (300, 16, 200)])
 @pytest.mark.parametrize("k", [2, 16])
 @pytest.mark.parametrize("typ,weighted", [(2, False), (16, False), (2, True)])
 def test_lists_line(ya, nq, nb, d, k, typ, weighted):

@@ -1659,10 +1659,13 @@ static int yk_knn_f32_check(int *type, long nq, long nb, int k) {
 }
 
 // k <= 16 by the register top-16 scan alone, without sketch and filter.  The
-// lines lie where the two routes meet, in 2,000 shapes of 1 .. 200,000 queries,
+// lines lie where the two routes meet, in 2,800 shapes of 1 .. 200,000 queries,
 // 16 .. 1e6 rows, d = 16 .. 2,048, k = 2, 10 and 16; filter and lists in ms:
 // * two blocks of rows at most: the lists' two launches against four (1 query x
-//   33 rows, d = 128 0.032 / 0.029; x 80 0.033 / 0.037);
+//   33 rows, d = 128 0.032 / 0.029; x 80 0.033 / 0.037), and some more rows as
+//   the queries grow in number (d = 128, k = 2: 12,400 x 100 0.088 / 0.078, 16,000
+//   x 130 0.108 / 0.089; k = 10: 4,000 x 49 0.047 / 0.043, 12,400 x 64 0.071 /
+//   0.063, 16,000 x 82 0.088 / 0.076; d = 762, k = 4: 8,000 x 82 0.120 / 0.135);
 // * many queries of few rows, where a query's selections cost more than its
 //   distances (50,000 queries, d = 64: x 200 0.31 / 0.19, x 600 0.37 / 0.36;
 //   200,000 x 1,000 1.63 / 1.45, x 2,000 2.18 / 2.40);
@@ -1680,7 +1683,8 @@ static int yk_knn_f32_check(int *type, long nq, long nb, int k) {
 // - 5 times as long.
 static bool yk_knn_by_lists(int k, int ld, long nq, long nb) {
   if (k < 2 || k > YK_REG_R) return false;
-  if (nb <= 48 || (nq >= 16384 && nb <= 100 + nq / 250)) return true;
+  if (nb <= 48 + nq / 240 || (k < 8 && nb <= 30 + nq / 160)) return true;
+  if (nq >= 16384 && nb <= 100 + nq / 250) return true;
   if (ld <= 256 || nq <= 128) return false;
   const double work = (double)nq * (double)nb * ld * ld;
   if (nq <= 160) return nb <= (1L << 18) && work >= 2e13;

@@ -813,7 +813,7 @@ def main():
             "fp32": {"queries_per_s": qps32, "ms_per_step": r["sec32"] * 1e3,
                      "roofline": {"bound": "mfma", "achieved": ach32, "peak": PEAK_FP32_TFLOPS,
                                   "unit": "TFLOP/s", "frac": ach32 / PEAK_FP32_TFLOPS,
-                                  "kernel": "yk_scan_f32_lds<2,8,3,false> (FP32 filtered pass)",
+                                  "kernel": "yk_scan_f32_lds<1,8,3,false> (FP32 filtered pass)",
                                   "kernel_ms_per_launch": f32_ms_launch,
                                   "launches_per_step": f32_n / args.steps,
                                   "sketch_kernel_ms_per_launch":

@@ -575,8 +575,8 @@ extern "C" int yk_kmeans_readback_checked(const int *counts, int k, int *counts_
 // split probabilities p, the donor's set to 0, and p normalised again in L1
 // norm, every element rounded to float: O(k) per empty cluster (64 us on the
 // host at k = 65,536, 1,865 clusters in one iteration: 120 of a 163 ms call).
-// One workgroup holds p in registers, thread t a run of elements in index
-// order, and takes the empty clusters one after the other: 3.9 us each at
+// One workgroup holds p in registers (the largest kernel in part in scratch
+// memory, below), thread t a run of elements in index order, and takes the empty clusters one after the other: 3.9 us each at
 // k = 65,536, of which the normalisation's five instructions per element on
 // one CU are half.
 //
@@ -591,9 +591,10 @@ extern "C" int yk_kmeans_readback_checked(const int *counts, int k, int *counts_
 // there) *flag is set and the host does the split.
 
 // Each pass converts its p[i] anew: kept from one pass for the next, the
-// doubles of 64 elements alone fill the thread's 128 registers, and p went to
-// scratch memory (with the donor's thread walking its elements one by one:
-// 6.3 us per empty cluster).
+// doubles of 64 elements alone fill the thread's 128 registers, and most of p
+// went to scratch memory (204 registers spilled; with the donor's thread
+// walking its elements one by one 6.3 us per empty cluster).  The kernel for k >
+// 16,384 still spills 75 (276 bytes a lane), the smaller ones none.
 template <int PT>
 __device__ __forceinline__ void yk_split_pass(float (&p)[PT]) {
 #pragma unroll

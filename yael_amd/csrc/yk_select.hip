@@ -39,12 +39,14 @@
 //
 // k > 1 is exact in two passes: (A) MODE 1 over a 1-in-stride sample of
 // base blocks with >= k splits gives, per query, >= 2k minima of disjoint
-// row subsets -- distinct real keys -- whose k-th smallest T_q bounds the
-// true k-th smallest key from above.  (B) MODE 3 over the whole base
-// collects every key <= T_q, then a per-query sort keeps the k smallest.  A
-// query whose candidates overflow the list gets a tighter T_q (the k-th
-// smallest of the keys it did capture, again an upper bound) and is scanned
-// again.
+// row subsets -- distinct real keys -- whose k-th smallest bounds the true
+// k-th smallest key from above: the starting bound T_q for k <= 16.  For k >
+// 16 a smaller one of the minima is the estimated bound (yk_bound_rank).  (B)
+// MODE 3 over the whole base collects every key <= T_q, then a per-query sort
+// keeps the k smallest.  A query with fewer than k keys under an estimate is
+// scanned without a bound; one whose candidates overflow the list gets a
+// tighter T_q (the k-th smallest of the keys it did capture, an upper bound)
+// and is scanned again, or for k <= 16 left to MODE 2.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <pthread.h>
@@ -630,22 +632,22 @@ __global__ __launch_bounds__(256) void yk_scan_f32(ScanArgs a0) {
 // n = 1e5 points to 1,024 centroids 0.290 ms, 90 TFLOP/s).  Here the
 // workgroup's four waves share each block: a 32-row block is one contiguous
 // piece of memory, loaded 1 KB per wave instruction straight into the other
-// of two LDS buffers while a stage is multiplied (no registers hold it).  The four 16-byte units of a
-// row's chunk are stored in the order unit ^ (row & 3), which spreads the
-// rows' reads over four times the banks and leaves the chunk a constant
-// offset of the read's address.  One barrier per stage; short vectors stage G
+// of two LDS buffers while a stage is multiplied (no registers hold it).  The
+// four 16-byte units of a row's chunk are stored in the order unit ^ (row & 3),
+// which spreads the rows' reads over four times the banks and leaves the chunk
+// a constant offset of the read's address.  One barrier per stage; short vectors stage G
 // blocks at once so that a stage is at least 64 MFMAs.  Two query tiles per
 // wave (NB = 2) would use each fragment read from LDS twice, but at d = 128
 // their 128 registers of queries leave two waves per SIMD and spills, and 256
 // queries a workgroup fewer of them: 1e5 queries x 1,024 0.260 against 0.236 ms,
 // 20,000 x 16,384, k = 100 2.00 and 1.84, 300 x 1e6 1.27 and 1.00 (1.17
 // streamed).  Only k = 1 at d <= 16 keeps them, from 65,536 queries on (3e5 x
-// 1,024 0.144 and 0.150).  Same MFMA operands, same order, same epilogue arithmetic as the
-// streaming kernel: the same bits.  n = 1e5 points to 1,024 centroids: 0.290
-// -> 0.235 ms (112 TFLOP/s; n = 1e6: 123).  What is left of the FP32 rate
-// (153 TFLOP/s for a large library product): timing builds without the
-// epilogue 135, without the loads too 141 TFLOP/s at n = 1e6, and at n = 1e5
-// ~0.03 ms of start (every workgroup's 128 KB of queries at once).
+// 1,024 0.144 and 0.150).  Same MFMA operands, same order, same epilogue
+// arithmetic as the streaming kernel: the same bits.  n = 1e5 points to 1,024
+// centroids: 0.290 -> 0.222 ms (118 TFLOP/s of the 153 of a large library
+// product; 1e4 queries x 1e6, k = 100: 124).  What is left is the epilogue's
+// vector instructions, which do not overlap with the MFMAs, and at n = 1e5 the
+// start (every workgroup's queries at once).
 template <int NCH>
 struct YkLdsShape {
   static constexpr int U = 4 * NCH;  // float4 units of a row
@@ -2207,7 +2209,8 @@ int yk_batch_assign_res(int ninst, int d, int kc, int kpad, int chunk, const flo
   const int per_res = yk_resident_wgs((const void *)kern, 256, 2) / 8;
   // The update's chunk is chosen for the update; whole chunks as work items
   // left the last of ~1.4 rounds half empty (2e6 points, 1,094 chunks for 768
-  // workgroups: 0.412 ms, now 0.380).  At least six items a workgroup, of
+  // workgroups: 0.412 ms, now 0.380; two workgroups per CU with whole chunks, as
+  // many registers once made it, were as good: 0.37 - 0.39).  At least six items a workgroup, of
   // 256 points or more (the centroids are staged once per item).
   long nsub = (48L * per_res + nuitems - 1) / nuitems;
   if (nsub > chunk / 256) nsub = chunk / 256;

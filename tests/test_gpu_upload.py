@@ -49,6 +49,29 @@ def test_copies_roundtrip_and_pad_columns(ya, n, d):
     assert np.array_equal(raw[:, :d], x) and not raw[:, d:].any()
 
 
+@pytest.mark.parametrize("nbytes", [(4 << 20) - 4, 4 << 20, (4 << 20) + 4, (8 << 20) + 4092,
+                                    32 << 20, (32 << 20) + 4, (64 << 20) + 4, (97 << 20) - 4])
+@pytest.mark.parametrize("shift", [0, 4])
+def test_copies_down_in_pieces(ya, nbytes, shift):
+    """From 4 MB on in quarters of up to 8 MB, whose buffers are taken again
+    past 64 MB; each piece is shared by two to four threads.  Every byte
+    comes, in its place, at any alignment, and none beside it, twice."""
+    import ctypes
+    from yael_amd import device
+    rng = np.random.default_rng(nbytes + shift)
+    x = rng.integers(0, 256, nbytes, np.uint8)
+    print("down %d bytes, shift %d" % (nbytes, shift), flush=True)
+    mem = device.DeviceBuffer(nbytes)
+    ya.check(ya.lib().yk_memcpy_h2d(mem.ptr, x.ctypes.data, nbytes), "h2d")
+    for fill in (0, 255):
+        back = np.full(nbytes + 64, fill, np.uint8)
+        ya.check(ya.lib().yk_memcpy_d2h(ctypes.c_void_p(back.ctypes.data + 32 + shift), mem.ptr,
+                                        nbytes), "d2h")
+        assert np.array_equal(back[32 + shift:32 + shift + nbytes], x)
+        assert (back[:32 + shift] == fill).all() and (back[32 + shift + nbytes:] == fill).all()
+    mem.free()
+
+
 @pytest.mark.parametrize("n,d", [(1, 65), (500, 128), (600, 100), (2100, 128), (9001, 128),
                                  (11000, 100), (50000, 128), (180001, 100)])
 def test_copies_of_pinned_host_memory(ya, n, d):

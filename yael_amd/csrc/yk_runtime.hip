@@ -2,10 +2,12 @@
 // priority), error reporting, allocation, padded copies, stream timing.
 #include <hip/hip_runtime.h>
 #include <pthread.h>
+#include <sched.h>
 #include <stdarg.h>
 #include <stdio.h>
 #include <string.h>
 #include <sys/stat.h>
+#include <atomic>
 
 #include "yk.h"
 #include "yk_dev.h"
@@ -143,7 +145,8 @@ extern "C" int yk_host_free(void *p) {
 // staged; 32 MB 17 and 38), up 16 MB (37 and 43; plain is ahead below)
 #define YK_STAGE_MIN_DOWN ((size_t)4 << 20)
 #define YK_STAGE_MIN_UP ((size_t)16 << 20)
-static int yk_copy_staged(char *dev, char *host, size_t bytes, bool up);
+static int yk_copy_staged_up(char *dev, const char *host, size_t bytes);
+static int yk_copy_staged_down(char *host, const char *dev, size_t bytes);
 
 // Memory at p that HIP knows (pinned or mapped host memory, or a device's): the
 // DMA reaches it by itself, and a detour through the pinned buffers only costs
@@ -164,7 +167,7 @@ extern "C" int yk_memcpy_d2h(void *dst, const void *src, size_t bytes) {
   if (bytes <= 256 || (bytes <= YK_READ_SMALL && !yk_known_to_hip(dst)))
     return yk_read_small(dst, src, bytes);
   if (bytes >= YK_STAGE_MIN_DOWN && !yk_known_to_hip(dst))
-    return yk_copy_staged((char *)src, (char *)dst, bytes, false);
+    return yk_copy_staged_down((char *)dst, (const char *)src, bytes);
   YK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, g_stream));
   YK_HIP(hipStreamSynchronize(g_stream));
   return YK_OK;
@@ -241,111 +244,196 @@ extern "C" int yk_sync(void) {
   return YK_OK;
 }
 
-// Copies of YK_STAGE_MIN_* bytes and more from and to pageable host memory: up
-// to YK_STAGE_THREADS host threads, one per YK_STAGE_SLICE bytes, each take a
-// contiguous slice and push it through two pinned buffers, the host copy of one
-// buffer overlapping the DMA of the other.  Up, each thread has a stream of its
-// own (default priority; 512 MB 9.9 ms, on one stream 10.7).  Down, the DMAs
-// queue on the library's stream: after copies on several streams the
-// allocations of a later call take longer (two k-means training calls in a row,
-// 16 sub-spaces of 94,555 points, d = 24, k = 93: 3.1 against 2.6 ms a call).  (A plain copy to pageable memory goes in 1 MB pieces, 20
-// us on the bus and ~70 us between them.  256 MB: 17 GB/s plain, 51 with four
-// threads, 42 with eight.)  The pinned buffers (64 MB in all)
-// are allocated at the first such copy and kept until the process ends; a
-// mutex keeps one staged copy at a time.
+// Copies of YK_STAGE_MIN_* bytes and more from and to pageable host memory go
+// through pinned buffers, the host copies of up to YK_STAGE_THREADS threads
+// overlapping the DMAs.  (A plain copy to pageable memory goes in 1 MB pieces,
+// 20 us on the bus and ~70 us between them.  256 MB: 17 GB/s plain, 51 with four
+// threads, 42 with eight.)  The pinned buffers (64 MB in all) are allocated at
+// the first such copy and kept until the process ends; a mutex keeps one staged
+// copy at a time.
 #define YK_STAGE_THREADS 4
-#define YK_STAGE_SLICE ((size_t)2 << 20)
+#define YK_STAGE_SLICE ((size_t)2 << 20)  // one thread per so many bytes
 #define YK_STAGE_BYTES ((size_t)8 << 20)
+#define YK_STAGE_BUFS (2 * YK_STAGE_THREADS)
 static pthread_mutex_t g_stage_mu = PTHREAD_MUTEX_INITIALIZER;
-static void *g_stage_buf[YK_STAGE_THREADS][2];
+static void *g_stage_buf[YK_STAGE_BUFS];
+static hipEvent_t g_stage_ev[YK_STAGE_BUFS];
 static hipStream_t g_stage_st[YK_STAGE_THREADS];  // up
-static hipEvent_t g_stage_ev[YK_STAGE_THREADS][2];
 static int g_stage_ready = 0;
-
-struct YkStageJob {
-  char *dev, *host;
-  size_t bytes;
-  int t;
-  bool up;
-  hipStream_t st;
-  hipError_t err;
-};
-
-static void *yk_stage_worker(void *arg) {
-  YkStageJob *j = (YkStageJob *)arg;
-  size_t pend[2] = {0, 0}, at[2] = {0, 0};  // bytes in flight through each buffer, their place
-  // two pieces of a slice or more, so that the buffers overlap
-  size_t piece = (j->bytes / 2 + 4095) & ~(size_t)4095;
-  if (piece > YK_STAGE_BYTES) piece = YK_STAGE_BYTES;
-  auto settle = [&](int b) {  // the buffer's DMA is done; down: its bytes go to the host
-    if (!pend[b]) return hipSuccess;
-    const hipError_t e = hipEventSynchronize(g_stage_ev[j->t][b]);
-    if (e == hipSuccess && !j->up) memcpy(j->host + at[b], g_stage_buf[j->t][b], pend[b]);
-    pend[b] = 0;
-    return e;
-  };
-  size_t off = 0;
-  for (int b = 0; off < j->bytes && j->err == hipSuccess; b ^= 1) {
-    const size_t n = j->bytes - off < piece ? j->bytes - off : piece;
-    void *buf = g_stage_buf[j->t][b];
-    hipError_t e = settle(b);
-    if (e == hipSuccess && j->up) memcpy(buf, j->host + off, n);
-    if (e == hipSuccess)
-      e = j->up ? hipMemcpyAsync(j->dev + off, buf, n, hipMemcpyHostToDevice, j->st)
-                : hipMemcpyAsync(buf, j->dev + off, n, hipMemcpyDeviceToHost, j->st);
-    if (e == hipSuccess) e = hipEventRecord(g_stage_ev[j->t][b], j->st);
-    j->err = e;
-    pend[b] = n;
-    at[b] = off;
-    off += n;
-  }
-  if (j->err == hipSuccess) j->err = settle(0);
-  if (j->err == hipSuccess) j->err = settle(1);
-  // (after an error: nothing of this slice is left in flight)
-  if (j->err != hipSuccess) (void)hipStreamSynchronize(j->st);
-  return nullptr;
-}
 
 static int yk_stage_setup(bool up) {
   for (int t = 0; up && t < YK_STAGE_THREADS; t++)
     if (!g_stage_st[t]) YK_HIP(hipStreamCreateWithFlags(&g_stage_st[t], hipStreamNonBlocking));
   if (g_stage_ready) return YK_OK;
-  for (int t = 0; t < YK_STAGE_THREADS; t++)
-    for (int b = 0; b < 2; b++) {
-      YK_HIP(hipHostMalloc(&g_stage_buf[t][b], YK_STAGE_BYTES, hipHostMallocDefault));
-      YK_HIP(hipEventCreateWithFlags(&g_stage_ev[t][b], hipEventDisableTiming));
-    }
+  for (int b = 0; b < YK_STAGE_BUFS; b++) {
+    YK_HIP(hipHostMalloc(&g_stage_buf[b], YK_STAGE_BYTES, hipHostMallocDefault));
+    YK_HIP(hipEventCreateWithFlags(&g_stage_ev[b], hipEventDisableTiming));
+  }
   g_stage_ready = 1;
   return YK_OK;
 }
 
-static int yk_copy_staged(char *dev, char *host, size_t bytes, bool up) {
-  if (up) YK_HIP(hipStreamSynchronize(g_stream));  // earlier work on the device memory
+// job(t) on `ways` threads, the caller's among them; where one cannot start,
+// the caller does its job too
+static void yk_stage_threads(void *(*fn)(void *), char *jobs, size_t job_bytes, int ways) {
+  pthread_t th[YK_STAGE_THREADS];
+  bool started[YK_STAGE_THREADS] = {false};
+  for (int t = 1; t < ways; t++)
+    started[t] = pthread_create(&th[t], nullptr, fn, jobs + t * job_bytes) == 0;
+  fn(jobs);
+  for (int t = 1; t < ways; t++) {
+    if (started[t])
+      pthread_join(th[t], nullptr);
+    else
+      fn(jobs + t * job_bytes);
+  }
+}
+
+static int yk_stage_ways(size_t bytes) {
+  const size_t w = bytes / YK_STAGE_SLICE;
+  return w < 1 ? 1 : w > YK_STAGE_THREADS ? YK_STAGE_THREADS : (int)w;
+}
+
+// Up: each thread pushes a contiguous slice through two buffers on a stream of
+// its own (default priority; 512 MB 9.9 ms, on one stream 10.7).
+struct YkStageUp {
+  char *dev;
+  const char *host;
+  size_t bytes;
+  int t;
+  hipError_t err;
+};
+
+static void *yk_stage_up_worker(void *arg) {
+  YkStageUp *j = (YkStageUp *)arg;
+  hipStream_t st = g_stage_st[j->t];
+  // two pieces of a slice or more, so that the buffers overlap
+  size_t piece = (j->bytes / 2 + 4095) & ~(size_t)4095;
+  if (piece > YK_STAGE_BYTES) piece = YK_STAGE_BYTES;
+  bool pend[2] = {false, false};
+  size_t off = 0;
+  for (int b = 0; off < j->bytes && j->err == hipSuccess; b ^= 1) {
+    const size_t n = j->bytes - off < piece ? j->bytes - off : piece;
+    const int slot = 2 * j->t + b;
+    hipError_t e = pend[b] ? hipEventSynchronize(g_stage_ev[slot]) : hipSuccess;
+    if (e == hipSuccess) {
+      memcpy(g_stage_buf[slot], j->host + off, n);
+      e = hipMemcpyAsync(j->dev + off, g_stage_buf[slot], n, hipMemcpyHostToDevice, st);
+    }
+    if (e == hipSuccess) e = hipEventRecord(g_stage_ev[slot], st);
+    j->err = e;
+    pend[b] = true;
+    off += n;
+  }
+  const hipError_t e = hipStreamSynchronize(st);
+  if (j->err == hipSuccess) j->err = e;
+  return nullptr;
+}
+
+static int yk_copy_staged_up(char *dev, const char *host, size_t bytes) {
+  YK_HIP(hipStreamSynchronize(g_stream));  // earlier work on the device memory
   pthread_mutex_lock(&g_stage_mu);
-  int rc = yk_stage_setup(up);
+  int rc = yk_stage_setup(true);
   if (rc == YK_OK) {
-    size_t ways = bytes / YK_STAGE_SLICE;
-    if (ways > YK_STAGE_THREADS) ways = YK_STAGE_THREADS;
-    const size_t per = (bytes / ways + 4095) & ~(size_t)4095;
-    YkStageJob job[YK_STAGE_THREADS];
-    pthread_t th[YK_STAGE_THREADS];
-    int started[YK_STAGE_THREADS] = {0}, nt = 0;
-    for (int t = 0; t < YK_STAGE_THREADS && (size_t)t * per < bytes; t++, nt++) {
-      const size_t o = (size_t)t * per;
-      job[t] = {dev + o, host + o, bytes - o < per ? bytes - o : per, t, up,
-                up ? g_stage_st[t] : g_stream, hipSuccess};
-    }
-    for (int t = 1; t < nt; t++)
-      started[t] = pthread_create(&th[t], nullptr, yk_stage_worker, &job[t]) == 0;
-    yk_stage_worker(&job[0]);
-    for (int t = 1; t < nt; t++) {
-      if (started[t])
-        pthread_join(th[t], nullptr);
-      else
-        yk_stage_worker(&job[t]);  // a thread that could not start: its slice here
-    }
+    const size_t per = (bytes / yk_stage_ways(bytes) + 4095) & ~(size_t)4095;
+    YkStageUp job[YK_STAGE_THREADS];
+    int nt = 0;
+    for (size_t o = 0; nt < YK_STAGE_THREADS && o < bytes; o += per, nt++)
+      job[nt] = {dev + o, host + o, bytes - o < per ? bytes - o : per, nt, hipSuccess};
+    yk_stage_threads(yk_stage_up_worker, (char *)job, sizeof job[0], nt);
     for (int t = 0; t < nt && rc == YK_OK; t++)
       if (job[t].err != hipSuccess) rc = yk_hip_fail(job[t].err, "staged copy");
+  }
+  pthread_mutex_unlock(&g_stage_mu);
+  return rc;
+}
+
+// Down: pieces come one after the other on the library's stream, and the
+// threads share each piece's host copy.  (After copies on several streams the
+// allocations of a later call take longer: two k-means training calls in a row,
+// 16 sub-spaces of 94,555 points, d = 24, k = 93, 3.1 against 2.6 ms a call.  A
+// piece costs ~9 us besides its bytes, hence few and large ones.  8 MB 0.25 ms,
+// 48 MB 1.09, 512 MB 10.5; a slice for each thread on the one stream 0.32, 1.33
+// and 10.7, on four streams 0.25, 1.30 and 10.1.)
+struct YkStageDown {
+  const char *dev;
+  char *host;
+  size_t bytes, piece;
+  long npiece;
+  int ways;
+  std::atomic<long> next;                // (piece, part) to copy, in order
+  std::atomic<long> at[YK_STAGE_BUFS];   // the piece that a buffer holds or waits for
+  std::atomic<int> left[YK_STAGE_BUFS];  // its parts not yet copied
+  std::atomic<int> err;
+};
+
+static void yk_stage_down_queue(YkStageDown *j, long c) {
+  const int slot = (int)(c % YK_STAGE_BUFS);
+  const size_t off = (size_t)c * j->piece;
+  const size_t n = j->bytes - off < j->piece ? j->bytes - off : j->piece;
+  hipError_t e =
+      hipMemcpyAsync(g_stage_buf[slot], j->dev + off, n, hipMemcpyDeviceToHost, g_stream);
+  if (e == hipSuccess) e = hipEventRecord(g_stage_ev[slot], g_stream);
+  if (e != hipSuccess) {
+    j->err.store(e);
+    return;
+  }
+  j->left[slot].store(j->ways, std::memory_order_relaxed);
+  j->at[slot].store(c, std::memory_order_release);
+}
+
+static void *yk_stage_down_worker(void *arg) {
+  YkStageDown *j = *(YkStageDown **)arg;
+  for (;;) {
+    const long u = j->next.fetch_add(1), c = u / j->ways;
+    if (c >= j->npiece) break;
+    const int slot = (int)(c % YK_STAGE_BUFS);
+    // (queued by whoever ends the buffer's last piece, all of whose parts were
+    // taken before this one)
+    while (j->at[slot].load(std::memory_order_acquire) != c) {
+      if (j->err.load()) return nullptr;
+      sched_yield();
+    }
+    const hipError_t e = hipEventSynchronize(g_stage_ev[slot]);
+    if (e != hipSuccess) {
+      j->err.store(e);
+      return nullptr;
+    }
+    const size_t off = (size_t)c * j->piece;
+    const size_t n = j->bytes - off < j->piece ? j->bytes - off : j->piece;
+    const size_t per = (n / j->ways + 64) & ~(size_t)63, o = per * (u % j->ways);
+    if (o < n)
+      memcpy(j->host + off + o, (const char *)g_stage_buf[slot] + o, n - o < per ? n - o : per);
+    if (j->left[slot].fetch_sub(1) == 1 && c + YK_STAGE_BUFS < j->npiece)
+      yk_stage_down_queue(j, c + YK_STAGE_BUFS);
+  }
+  return nullptr;
+}
+
+static int yk_copy_staged_down(char *host, const char *dev, size_t bytes) {
+  pthread_mutex_lock(&g_stage_mu);
+  int rc = yk_stage_setup(false);
+  if (rc == YK_OK) {
+    YkStageDown j;
+    j.dev = dev;
+    j.host = host;
+    j.bytes = bytes;
+    // quarters: an eighth at a time 8 MB take 0.29 ms, from 32 MB on the same
+    j.piece = (bytes / 4 + 4095) & ~(size_t)4095;
+    if (j.piece > YK_STAGE_BYTES) j.piece = YK_STAGE_BYTES;
+    j.npiece = (long)((bytes + j.piece - 1) / j.piece);
+    j.ways = yk_stage_ways(bytes);
+    j.next.store(0);
+    j.err.store(0);
+    for (auto &a : j.at) a.store(-1);
+    for (long c = 0; c < j.npiece && c < YK_STAGE_BUFS && !j.err.load(); c++)
+      yk_stage_down_queue(&j, c);
+    YkStageDown *job[YK_STAGE_THREADS] = {&j, &j, &j, &j};
+    yk_stage_threads(yk_stage_down_worker, (char *)job, sizeof job[0], j.ways);
+    if (j.err.load()) {
+      (void)hipStreamSynchronize(g_stream);  // nothing is left in flight
+      rc = yk_hip_fail((hipError_t)j.err.load(), "staged copy");
+    }
   }
   pthread_mutex_unlock(&g_stage_mu);
   return rc;
@@ -435,7 +523,7 @@ static int yk_dense_copy(float *dev, float *host, long n, int d, bool up) {
       continue;
     }
     if (bytes >= YK_STAGE_MIN_UP && !known)
-      YK_TRY(yk_copy_staged((char *)buf, (char *)(host + i * d), bytes, true));
+      YK_TRY(yk_copy_staged_up((char *)buf, (const char *)(host + i * d), bytes));
     else
       YK_HIP(hipMemcpyAsync(buf, host + i * d, bytes, hipMemcpyHostToDevice, g_stream));
     const long t = m * (ld / 4);
@@ -460,7 +548,7 @@ extern "C" int yk_upload_vectors(float *dst, const float *src, long n, int d) {
     return rc;
   }
   if (bytes >= YK_STAGE_MIN_UP && !yk_known_to_hip(src))
-    return yk_copy_staged((char *)dst, (char *)src, bytes, true);
+    return yk_copy_staged_up((char *)dst, (const char *)src, bytes);
   YK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, g_stream));
   YK_HIP(hipStreamSynchronize(g_stream));
   return YK_OK;
